@@ -750,54 +750,100 @@ __global__ void zero_kernel(T *__restrict__ a, int n) {
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) a[t] = T(0);
 }
 
-// The coarsest level in one workgroup: 50 red-black sweeps with φ and b in LDS,
+// The coarsest level in one workgroup: 50 red-black sweeps with φ in LDS,
 // then the mean projection (_solve_coarsest!, src/Multigrid.jl:685-689).
-template <typename T>
+//
+// It is bound by the latency of 100 dependent half-sweeps, so a half-sweep
+// must be short. A thread owns S slots of each colour (slot s: row s / h,
+// the s % h-th cell of the colour in it, h = ⌈nx/2⌉) and keeps for each, in
+// registers, the six neighbours' LDS indices, the six face weights divided
+// by the diagonal and b over the diagonal: a half-sweep is six LDS reads,
+// six multiply-adds, one LDS write and the barrier. S = 0, for levels with
+// more slots than 2 per thread: the cell's weights are formed from the
+// arrays at every visit (one division per cell), b read from memory.
+// Measured per launch against the form that read the coefficients and
+// divided the linear index by the extents at every visit: 12×12×6 FP64
+// 183 → 24 us, 16×16×6 FP32 211 → 27 us.
+template <typename T, int S>
 __global__ void __launch_bounds__(1024) coarsest_kernel(LevelD<T> L, int nsweeps, int singular,
                                                         const double *__restrict__ bm, int zero_start) {
     extern __shared__ unsigned char smem_raw[];
     T *sphi = reinterpret_cast<T *>(smem_raw);
     const int n = L.nx * L.ny * L.nz;
-    T *sb = sphi + n;
     __shared__ double sh[1024 / 64];
     // bm: b's pending mean; zero_start: φ enters as zero (not read)
     const T bmv = bm ? (T)bm[0] : T(0);
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        sphi[t] = zero_start ? T(0) : L.phi[t];
-        sb[t] = bm ? L.b[t] - bmv : L.b[t];
-    }
-    __syncthreads();
-    LevelD<T> S = L;
-    S.phi = sphi;
-    S.b = sb;
-    for (int sw = 0; sw < nsweeps; sw++) {
-        for (int colour = 0; colour <= 1; colour++) {
-            for (int t = threadIdx.x; t < n; t += blockDim.x) {
-                const int i = t % L.nx, j = (t / L.nx) % L.ny, k = t / (L.nx * L.ny);
-                if (((i + j + k) & 1) != colour) continue;
-                const T d = diagA(S, i, j, k);
-                if (L.cx && fabs(d) < Eps<T>::v) continue;
-                // (b − off)/diag with off the neighbour sum of the reference's form
-                const T xp = sphi[lidx(S, wrapc(i + 1, S.nx, S.bcx), j, k)], xm = sphi[lidx(S, wrapc(i - 1, S.nx, S.bcx), j, k)];
-                const T yp = sphi[lidx(S, i, wrapc(j + 1, S.ny, S.bcy), k)], ym = sphi[lidx(S, i, wrapc(j - 1, S.ny, S.bcy), k)];
-                const T zp = sphi[lidx(S, i, j, wrapc(k + 1, S.nz, S.bcz))], zm = sphi[lidx(S, i, j, wrapc(k - 1, S.nz, S.bcz))];
-                T o;
-                if (!L.cx) {
-                    o = ((xp + xm) * L.ix2 + (yp + ym) * L.iy2) + (zp + zm) * L.iz2;
-                } else {
-                    const uint32_t nx1 = L.nx + 1, ny1 = L.ny + 1;
-                    const T fxp = L.cx[(uint32_t)(i + 1) + nx1 * ((uint32_t)j + (uint32_t)L.ny * k)];
-                    const T fxm = L.cx[(uint32_t)i + nx1 * ((uint32_t)j + (uint32_t)L.ny * k)];
-                    const T fyp = L.cy[(uint32_t)i + (uint32_t)L.nx * ((uint32_t)(j + 1) + ny1 * k)];
-                    const T fym = L.cy[(uint32_t)i + (uint32_t)L.nx * ((uint32_t)j + ny1 * k)];
-                    const T fzp = L.cz[lidx(L, i, j, k + 1)];
-                    const T fzm = L.cz[lidx(L, i, j, k)];
-                    o = ((fxp * xp + fxm * xm) * L.ix2 + (fyp * yp + fym * ym) * L.iy2) + (fzp * zp + fzm * zm) * L.iz2;
-                }
-                sphi[t] = (sb[t] - o) / d;
-            }
-            __syncthreads();
+    for (int t = threadIdx.x; t < n; t += blockDim.x) sphi[t] = zero_start ? T(0) : L.phi[t];
+    const int h = (L.nx + 1) / 2, slots = h * L.ny * L.nz;
+    // the slot's cell (−1: none, or a fully blocked cell, which keeps φ), its
+    // neighbours and weights
+    struct Slot {
+        int c;
+        uint32_t q[3];  // the neighbours of an axis, 16 bits each
+        T w[6], b;
+    };
+    auto make = [&](int s, int colour) {
+        Slot o;
+        o.c = -1;
+        if (s >= slots) return o;
+        const int ih = s % h, jk = s / h, j = jk % L.ny, k = jk / L.ny;
+        const int i = 2 * ih + ((j + k + colour) & 1);
+        if (i >= L.nx) return o;
+        T w[6];
+        if (L.cx) {
+            const uint32_t nx1 = L.nx + 1, ny1 = L.ny + 1;
+            w[0] = L.cx[(uint32_t)(i + 1) + nx1 * ((uint32_t)j + (uint32_t)L.ny * k)] * L.ix2;
+            w[1] = L.cx[(uint32_t)i + nx1 * ((uint32_t)j + (uint32_t)L.ny * k)] * L.ix2;
+            w[2] = L.cy[(uint32_t)i + (uint32_t)L.nx * ((uint32_t)(j + 1) + ny1 * k)] * L.iy2;
+            w[3] = L.cy[(uint32_t)i + (uint32_t)L.nx * ((uint32_t)j + ny1 * k)] * L.iy2;
+            w[4] = L.cz[lidx(L, i, j, k + 1)] * L.iz2;
+            w[5] = L.cz[lidx(L, i, j, k)] * L.iz2;
+        } else {
+            w[0] = w[1] = L.ix2;
+            w[2] = w[3] = L.iy2;
+            w[4] = w[5] = L.iz2;
         }
+        const T d = -(((w[0] + w[1]) + (w[2] + w[3])) + (w[4] + w[5]));
+        if (L.cx && fabs(d) < Eps<T>::v) return o;
+        const T id = T(1) / d;
+        o.c = (int)lidx(L, i, j, k);
+        o.q[0] = lidx(L, wrapc(i + 1, L.nx, L.bcx), j, k) | lidx(L, wrapc(i - 1, L.nx, L.bcx), j, k) << 16;
+        o.q[1] = lidx(L, i, wrapc(j + 1, L.ny, L.bcy), k) | lidx(L, i, wrapc(j - 1, L.ny, L.bcy), k) << 16;
+        o.q[2] = lidx(L, i, j, wrapc(k + 1, L.nz, L.bcz)) | lidx(L, i, j, wrapc(k - 1, L.nz, L.bcz)) << 16;
+#pragma unroll
+        for (int m = 0; m < 6; m++) o.w[m] = w[m] * id;
+        o.b = (L.b[o.c] - bmv) * id;
+        return o;
+    };
+    auto update = [&](const Slot &o) {
+        if (o.c < 0) return;
+        const T u = o.w[0] * sphi[o.q[0] & 0xffffu] + o.w[1] * sphi[o.q[0] >> 16];
+        const T v = o.w[2] * sphi[o.q[1] & 0xffffu] + o.w[3] * sphi[o.q[1] >> 16];
+        const T w = o.w[4] * sphi[o.q[2] & 0xffffu] + o.w[5] * sphi[o.q[2] >> 16];
+        sphi[o.c] = o.b - ((u + v) + w);
+    };
+    if constexpr (S > 0) {
+        Slot own[2][S];
+#pragma unroll
+        for (int colour = 0; colour <= 1; colour++)
+#pragma unroll
+            for (int q = 0; q < S; q++) own[colour][q] = make((int)threadIdx.x + q * (int)blockDim.x, colour);
+        __syncthreads();
+        for (int sw = 0; sw < nsweeps; sw++) {
+#pragma unroll
+            for (int colour = 0; colour <= 1; colour++) {
+#pragma unroll
+                for (int q = 0; q < S; q++) update(own[colour][q]);
+                __syncthreads();
+            }
+        }
+    } else {
+        __syncthreads();
+        for (int sw = 0; sw < nsweeps; sw++)
+            for (int colour = 0; colour <= 1; colour++) {
+                for (int s = threadIdx.x; s < slots; s += blockDim.x) update(make(s, colour));
+                __syncthreads();
+            }
     }
     if (singular) {
         double v = 0.0;
@@ -810,6 +856,19 @@ __global__ void __launch_bounds__(1024) coarsest_kernel(LevelD<T> L, int nsweeps
         __syncthreads();
     }
     for (int t = threadIdx.x; t < n; t += blockDim.x) L.phi[t] = sphi[t];
+}
+
+// Slots per thread of coarsest_kernel (0: from memory), or −1 where the level
+// takes a launch per half-sweep instead. 1024 threads hold 3 slots of each
+// colour in FP64 (4 in FP32) in their 128 registers: 25×17×11 FP64 in
+// 104 us against 100 launches of about 4.5 us. Past that the form from
+// memory loses to the launches (27×25×19 FP64 1055 us), so it serves only
+// levels of up to 4096 cells whose rows are so short that half the slots are
+// empty.
+static int coarsest_slots(int nx, int ny, int nz, int esz) {
+    const int slots = (nx + 1) / 2 * ny * nz, s = (slots + 1023) / 1024;
+    if (s <= (esz == 8 ? 3 : 4)) return s;
+    return nx * ny * nz <= 4096 ? 0 : -1;
 }
 
 // ---- the outer FP64 CG kernels (pcg!, src/Backends.jl:1526-1589) ------------
@@ -1274,10 +1333,19 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
     const int n = h.nx * h.ny * h.nz;
     const bool cf = coarse_fold<T>(P, l);
     if (l == P->nlev - 1) {
-        size_t lds = sizeof(T) * 2 * (size_t)n;
-        if (n <= 4096) {
-            hipLaunchKernelGGL(coarsest_kernel<T>, dim3(1), dim3(1024), lds, st, devlevel<T>(P, l), 50, 1,
-                               cf ? P->bmL[l] : (const double *)nullptr, (int)(cf && zero_start));
+        const int own = coarsest_slots(h.nx, h.ny, h.nz, sizeof(T));
+        if (own >= 0) {
+            // as few waves as hold the slots of one colour (a barrier of fewer waves is shorter)
+            const int slots = (h.nx + 1) / 2 * h.ny * h.nz, bt = slots >= 1024 ? 1024 : (slots + 63) / 64 * 64;
+            auto launch = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(1), dim3(bt), sizeof(T) * (size_t)n, st, devlevel<T>(P, l), 50, 1,
+                                   cf ? P->bmL[l] : (const double *)nullptr, (int)(cf && zero_start));
+            };
+            if (own == 1) launch(coarsest_kernel<T, 1>);
+            else if (own == 2) launch(coarsest_kernel<T, 2>);
+            else if (own == 3) launch(coarsest_kernel<T, 3>);
+            else if (own == 4) launch(coarsest_kernel<T, sizeof(T) == 4 ? 4 : 3>);
+            else launch(coarsest_kernel<T, 0>);
         } else {
             int sm = P->smoother;
             P->smoother = 0;
