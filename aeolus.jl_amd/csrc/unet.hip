@@ -286,110 +286,233 @@ __global__ void __launch_bounds__(256) conv3_slice_kernel(const bf16 *__restrict
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient of a 3³ convolution: part[blk, tap, grp][c][n] =
-// Σ_{v in the block's range, v ≡ grp} in[nb(v, tap)][c] · dy[v][n], FP32.
-// Grid (blocks, 27). VB voxels at a time are staged in LDS as FP32; each
-// thread owns a 4×4 (c, n) tile; the G = 256 / (CIN·COUT/16) thread groups
-// take interleaved voxels and write separate partials.
+// Weight and bias gradients of a 3³ convolution on MFMA:
+//   dW[tap][c][n] = Σ_v in[nb(v, tap)][c] · dy[v][n],   db[n] = Σ_v dy[v][n]
+// as 27 products of M = channels c, N = outputs n, K = voxels. The inputs are
+// BF16 already, so BF16 products with FP32 accumulation lose nothing.
+//
+// K runs along x: lane group g of v_mfma_f32_16x16x32_bf16 takes the 8 voxels
+// 8g .. 8g+7 of a 32-voxel row segment. Both operands are channels-last in
+// memory and need 8 voxels of one channel per lane, so a thread loads 8
+// voxels × 8 channels (eight 16-byte loads), transposes them in registers (a
+// byte permute per dword) and writes [channel][voxel] rows of LDS. A row
+// holds the 32 voxels, then the right and left neighbours at 32 and 39 (a row
+// of 40 elements spreads 16-byte reads over the banks); the three dx taps of
+// a fragment are funnel shifts of one 16-byte read and those two.
+// A block marches y over the three z planes of a segment: four LDS slots per
+// plane, so that row y + 2 is stored while rows y − 1 .. y + 1 are read, one
+// barrier per row. Its waves share out the 9 (dy, dz) taps × channel tiles;
+// dy's fragments are read once per row. The accumulators stay in registers
+// over all of a block's rows; blocks write partials that wgrad_reduce_kernel
+// adds in a fixed order. db is one more product, with ones for the channels.
+//
+// Bound: latency of a row's loads and its barrier (a row is 9 to 36 MFMAs per
+// wave), hidden by the blocks of a CU. Measured at 128×128×64, the sum over
+// the ten layers with their reductions: 19.8 ms on FP32 VALU products from
+// FP32 LDS tiles and column sums of their own → 0.86 ms.
 // ---------------------------------------------------------------------------
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(256) wgrad_kernel(const bf16 *__restrict__ in, const bf16 *__restrict__ dy,
-                                                    float *__restrict__ part, Vol g, int vpb) {
-    constexpr int NT = (CIN / 4) * (COUT / 4);
-    constexpr int G = 256 / NT;
-    constexpr int VB = 32;
-    __shared__ float sx[VB][CIN + 1];
-    __shared__ float sd[VB][COUT + 1];
-    const int t = threadIdx.x, grp = t / NT, tt = t - grp * NT;
-    const int ci = (tt / (COUT / 4)) * 4, co = (tt % (COUT / 4)) * 4;
-    const int tap = blockIdx.y;
-    const int dx = tap % 3 - 1, dy_ = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-    const int nxy = g.nx * g.ny, nvox = nxy * g.nz;
-    const int vs = blockIdx.x * vpb, ve = min(vs + vpb, nvox);
-    float acc[4][4];
+template <int CIN, int COUT, int CS>
+__global__ void __launch_bounds__(256, COUT == 64 ? 1 : 2) wgrad_kernel(const bf16 *__restrict__ in, const bf16 *__restrict__ dy,
+                                                    float *__restrict__ part, float *__restrict__ bpart, Vol g,
+                                                    int ntx, int nyc, int yc) {
+    constexpr int C8 = CS / 8, N8 = COUT / 8, CR = CS < 16 ? 16 : CS, CT = CR / 16, NT = COUT / 16, NG = 9 * CT,
+                  GPW = (NG + 3) / 4, XW = 40;
+    static_assert(CIN % CS == 0 && CS % 8 == 0 && COUT % 16 == 0 && 3 * C8 * 6 + N8 * 4 <= 256, "shapes");
+    __shared__ __attribute__((aligned(16))) unsigned short sx[3][4][CR][XW];
+    __shared__ __attribute__((aligned(16))) unsigned short sd[2][COUT][XW];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int r = lane & 15, grp = lane >> 4;
+    const int slice = blockIdx.y;
+    if constexpr (CS < 16) {  // the rows of absent channels
+        for (int e = t; e < 3 * 4 * (CR - CS) * XW; e += 256) {
+            const int x = e % XW, c = e / XW % (CR - CS), q = e / (XW * (CR - CS));
+            sx[q >> 2][q & 3][CS + c][x] = 0;
+        }
+    }
+    // this thread's part of a row step: 8 voxels × 8 channels of `in` (kind 0)
+    // or dy (kind 2), or one edge voxel of `in` (kind 1)
+    int kind = 3, pz = 0, xb = 0, c8 = 0;
+    if (t < 3 * C8 * 4) {
+        kind = 0;
+        c8 = t % C8;
+        xb = t / C8 % 4;
+        pz = t / (C8 * 4);
+    } else if (t < 3 * C8 * 6) {
+        const int e = t - 3 * C8 * 4;
+        kind = 1;
+        c8 = e % C8;
+        xb = e / C8 % 2;  // 0: left, 1: right
+        pz = e / (C8 * 2);
+    } else if (t < 3 * C8 * 6 + N8 * 4) {
+        const int e = t - 3 * C8 * 6;
+        kind = 2;
+        c8 = e % N8;
+        xb = e / N8;
+    }
+    f32x4 acc[GPW][3][NT], accb[NT];
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+    for (int u = 0; u < NT; u++) {
+        accb[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = 0.f;
-    for (int v0 = vs; v0 < ve; v0 += VB) {
-        for (int e = t; e < VB * CIN; e += 256) {
-            const int vv = e / CIN, c = e - vv * CIN, v = v0 + vv;
-            float val = 0.f;
-            if (v < ve) {
-                const int z = v / nxy, rem = v - z * nxy, y = rem / g.nx, x = rem - y * g.nx;
-                const int zz = z + dz;
-                if (zz >= 0 && zz < g.nz) {
-                    const int xx = wrapi(x + dx, g.nx), yy = wrapi(y + dy_, g.ny);
-                    val = (float)in[(size_t)(xx + g.nx * (yy + g.ny * zz)) * CIN + c];
+        for (int i = 0; i < GPW; i++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) acc[i][d][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const u32x4 ones = u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // eight BF16 ones
+    const int ntask = ntx * nyc * g.nz;
+    for (int task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int x0 = task % ntx * 32, y0 = task / ntx % nyc * yc, z = task / (ntx * nyc);
+        const int y1 = min(y0 + yc, g.ny);
+        u32x4 v[8];
+        // in's row ya (any, wrapped) of plane z + pz − 1, dy's row yd
+        auto load = [&](int ya, int yd) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] = u32x4{0u, 0u, 0u, 0u};
+            const int zz = z + pz - 1;
+            const int yw = ya < 0 ? ya + g.ny : (ya >= g.ny ? ya - g.ny : ya);
+            const bool zin = zz >= 0 && zz < g.nz;
+            if (kind == 0 && zin) {
+                const bf16 *p = in + (size_t)(g.nx * (yw + g.ny * zz)) * CIN + slice * CS + c8 * 8;
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const int xr = x0 + 8 * xb + q;  // one past the axis: the last voxel's right neighbour
+                    if (xr <= g.nx) v[q] = *reinterpret_cast<const u32x4 *>(p + (size_t)wrapi(xr, g.nx) * CIN);
+                }
+            } else if (kind == 1 && zin) {
+                const int xr = xb ? x0 + 32 : x0 - 1;
+                if (xr <= g.nx)
+                    v[0] = *reinterpret_cast<const u32x4 *>(in + (size_t)(wrapi(xr, g.nx) + g.nx * (yw + g.ny * zz)) * CIN +
+                                                            slice * CS + c8 * 8);
+            } else if (kind == 2 && yd < y1) {
+                const bf16 *p = dy + (size_t)(g.nx * (yd + g.ny * z)) * COUT + c8 * 8;
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const int xr = x0 + 8 * xb + q;
+                    if (xr < g.nx) v[q] = *reinterpret_cast<const u32x4 *>(p + (size_t)xr * COUT);
                 }
             }
-            sx[vv][c] = val;
-        }
-        for (int e = t; e < VB * COUT; e += 256) {
-            const int vv = e / COUT, n = e - vv * COUT, v = v0 + vv;
-            sd[vv][n] = v < ve ? (float)dy[(size_t)v * COUT + n] : 0.f;
+        };
+        auto store = [&](int slot, int buf) {
+            if (kind == 0 || kind == 2) {
+                unsigned short *row = kind == 0 ? &sx[pz][slot][c8 * 8][8 * xb] : &sd[buf][c8 * 8][8 * xb];
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    const unsigned sel = (c & 1) ? 0x07060302u : 0x05040100u;
+                    u32x4 o;
+#pragma unroll
+                    for (int d = 0; d < 4; d++) o[d] = __builtin_amdgcn_perm(v[2 * d + 1][c >> 1], v[2 * d][c >> 1], sel);
+                    *reinterpret_cast<u32x4 *>(row + c * XW) = o;
+                }
+            } else if (kind == 1) {
+                unsigned short *row = &sx[pz][slot][c8 * 8][xb ? 32 : 39];
+#pragma unroll
+                for (int c = 0; c < 8; c++)
+                    row[c * XW] = (unsigned short)((c & 1) ? v[0][c >> 1] >> 16 : v[0][c >> 1] & 0xffffu);
+            }
+        };
+        __syncthreads();  // the previous task's last row has been read
+        // rows y0 − 1, y0, y0 + 1 in slots 0, 1, 2; dy's row y0 in buffer 0
+        for (int q = 0; q < 3; q++) {
+            load(y0 - 1 + q, y0);
+            store(q, 0);
         }
         __syncthreads();
-        if (grp < G) {
-            for (int vv = grp; vv < VB; vv += G) {
-                float xa[4], da[4];
+        for (int y = y0; y < y1; y++) {
+            const int s = y - y0;
+            const bool more = y + 1 < y1;
+            if (more) load(y + 2, y + 1);
+            bf16x8 b[NT];
 #pragma unroll
-                for (int a = 0; a < 4; a++) xa[a] = sx[vv][ci + a];
+            for (int u = 0; u < NT; u++)
+                b[u] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(&sd[s & 1][16 * u + r][8 * grp]));
 #pragma unroll
-                for (int b = 0; b < 4; b++) da[b] = sd[vv][co + b];
+            for (int i = 0; i < GPW; i++) {
+                const int gi = wave + 4 * i;
+                if (gi < NG) {
+                    const int yz = gi / CT, ct = gi % CT;
+                    const unsigned short *row = &sx[yz / 3][(s + yz % 3) & 3][16 * ct + r][0];
+                    const u32x4 m = *reinterpret_cast<const u32x4 *>(row + 8 * grp);
+                    const unsigned lf = row[grp ? 8 * grp - 1 : 39], rt = row[8 * grp + 8];
+                    const unsigned e1 = __builtin_amdgcn_alignbit(m[1], m[0], 16),
+                                   e2 = __builtin_amdgcn_alignbit(m[2], m[1], 16),
+                                   e3 = __builtin_amdgcn_alignbit(m[3], m[2], 16);
+                    const bf16x8 a0 = __builtin_bit_cast(bf16x8, u32x4{(m[0] << 16) | lf, e1, e2, e3});
+                    const bf16x8 a1 = __builtin_bit_cast(bf16x8, m);
+                    const bf16x8 a2 = __builtin_bit_cast(bf16x8, u32x4{e1, e2, e3, (m[3] >> 16) | (rt << 16)});
 #pragma unroll
-                for (int a = 0; a < 4; a++)
+                    for (int u = 0; u < NT; u++) {
+                        acc[i][0][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[u], acc[i][0][u], 0, 0, 0);
+                        acc[i][1][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[u], acc[i][1][u], 0, 0, 0);
+                        acc[i][2][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b[u], acc[i][2][u], 0, 0, 0);
+                    }
+                }
+            }
+            if (wave == 3 && slice == 0) {
 #pragma unroll
-                    for (int b = 0; b < 4; b++) acc[a][b] = fmaf(xa[a], da[b], acc[a][b]);
+                for (int u = 0; u < NT; u++)
+                    accb[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ones), b[u], accb[u], 0, 0, 0);
+            }
+            if (more) {
+                store((s + 3) & 3, (s + 1) & 1);
+                __syncthreads();
             }
         }
-        __syncthreads();
     }
-    if (grp < G) {
-        float *p = part + ((size_t)(blockIdx.x * 27 + tap) * G + grp) * (CIN * COUT);
+    // D[4·group + i][r]: channel 16·ct + 4·group + i, output 16·u + r
+    float *p = part + (size_t)(slice * gridDim.x + blockIdx.x) * (27 * CS * COUT);
 #pragma unroll
-        for (int a = 0; a < 4; a++)
+    for (int i = 0; i < GPW; i++) {
+        const int gi = wave + 4 * i;
+        if (gi < NG) {
+            const int yz = gi / CT, ct = gi % CT;
 #pragma unroll
-            for (int b = 0; b < 4; b++) p[(ci + a) * COUT + co + b] = acc[a][b];
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int u = 0; u < NT; u++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int c = 16 * ct + 4 * grp + q;
+                        if (CS >= 16 || c < CS) p[((size_t)(3 * yz + d) * CS + c) * COUT + 16 * u + r] = acc[i][d][u][q];
+                    }
+        }
+    }
+    if (wave == 3 && slice == 0 && grp == 0) {
+#pragma unroll
+        for (int u = 0; u < NT; u++) bpart[(size_t)blockIdx.x * COUT + 16 * u + r] = accb[u][0];
     }
 }
 
-// grad[tap][c][n] (c < cin, the logical input channels) = Σ over blocks and groups
-__global__ void wgrad_reduce_kernel(const float *__restrict__ part, float *__restrict__ grad, int nblk, int G,
-                                    int cinp, int cin, int cout) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    const int per = cin * cout;
-    if (e >= 27 * per) return;
-    const int tap = e / per, rem = e - tap * per, c = rem / cout, n = rem - c * cout;
+// grad[tap][c][n] (c < cin, the logical input channels; cs per slice) and
+// bias[n]: the sums of the nblk partials of each. A block does 16 sums, 16
+// threads each over a contiguous share of the partials (FP64), then the
+// shares in order.
+__global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float *__restrict__ part,
+                                                           const float *__restrict__ bpart, float *__restrict__ grad,
+                                                           float *__restrict__ bias, int nblk, int cs, int cin,
+                                                           int cout) {
+    __shared__ double sh[16][16];
+    const int ei = threadIdx.x & 15, seg = threadIdx.x >> 4;
+    const int e = blockIdx.x * 16 + ei, per = cin * cout, nw = 27 * per;
     double s = 0.0;
-    for (int b = 0; b < nblk; b++)
-        for (int q = 0; q < G; q++) s += part[((size_t)(b * 27 + tap) * G + q) * (cinp * cout) + c * cout + n];
-    grad[e] = (float)s;
-}
-
-// per-block column sums of dy[v][n] (bias gradients)
-template <int COUT>
-__global__ void __launch_bounds__(256) colsum_kernel(const bf16 *__restrict__ dy, float *__restrict__ part, int nvox,
-                                                     int vpb) {
-    __shared__ float sh[256];
-    constexpr int R = 256 / COUT;
-    const int t = threadIdx.x, n = t % COUT, rr = t / COUT;
-    const int vs = blockIdx.x * vpb, ve = min(vs + vpb, nvox);
-    float s = 0.f;
-    for (int v = vs + rr; v < ve; v += R) s += (float)dy[(size_t)v * COUT + n];
-    sh[t] = s;
+    if (e < nw + cout) {
+        const float *p = bpart + (e - nw);
+        size_t stride = cout;
+        if (e < nw) {
+            const int tap = e / per, rem = e - tap * per, c = rem / cout, n = rem - c * cout;
+            stride = (size_t)27 * cs * cout;
+            p = part + (size_t)(c / cs) * nblk * stride + ((size_t)tap * cs + c % cs) * cout + n;
+        }
+        const int b1 = nblk * (seg + 1) / 16;
+#pragma unroll 4
+        for (int b = nblk * seg / 16; b < b1; b++) s += (double)p[(size_t)b * stride];
+    }
+    sh[seg][ei] = s;
     __syncthreads();
-    if (rr == 0) {
-        for (int q = 1; q < R; q++) s += sh[q * COUT + n];
-        part[(size_t)blockIdx.x * COUT + n] = s;
+    if (seg == 0 && e < nw + cout) {
+        for (int q = 1; q < 16; q++) s += sh[q][ei];
+        if (e < nw) grad[e] = (float)s;
+        else bias[e - nw] = (float)s;
     }
-}
-__global__ void colsum_reduce_kernel(const float *__restrict__ part, float *__restrict__ out, int nblk, int cout) {
-    const int n = threadIdx.x;
-    if (n >= cout) return;
-    double s = 0.0;
-    for (int b = 0; b < nblk; b++) s += part[(size_t)b * cout + n];
-    out[n] = (float)s;
 }
 
 // ---------------------------------------------------------------------------
@@ -692,41 +815,36 @@ static int conv_run(hipStream_t st, int cin, int cout, const bf16 *in, const bf1
     return -1;
 }
 
-template <int CIN, int COUT>
-static int wgrad_launch(hipStream_t st, UNet *N, const bf16 *in, const bf16 *dy, Vol g, float *grad, int cin) {
-    constexpr int G = 256 / ((CIN / 4) * (COUT / 4));
-    const int nv = g.nx * g.ny * g.nz;
-    int nb = (nv + 8191) / 8192;
-    if (nb > 64) nb = 64;
-    const int vpb = ((nv + nb - 1) / nb + 31) / 32 * 32;
-    nb = (nv + vpb - 1) / vpb;
-    if ((size_t)nb * 27 * G * CIN * COUT > N->fpart_n) return -1;
-    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT>), dim3(nb, 27), dim3(256), 0, st, in, dy, N->fpart, g, vpb);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblk((size_t)27 * cin * COUT)), dim3(UB), 0, st, N->fpart, grad, nb, G,
-                       CIN, cin, COUT);
+// CS: the input channels of a block (with 16 or 32 the accumulators of a
+// wave's taps stay within 144 registers; 48 needs 84 with 16 outputs)
+template <int CIN, int COUT, int CS>
+static int wgrad_launch(hipStream_t st, UNet *N, const bf16 *in, const bf16 *dy, Vol g, float *grad, float *bias,
+                        int cin) {
+    constexpr int NS = CIN / CS;
+    const int ntx = (g.nx + 31) / 32;
+    // rows per block: few (a row's start costs three rows of loads) until the
+    // blocks fill the chip, 256 CUs × 2
+    int yc = 32;
+    while (yc > 8 && (long long)ntx * g.nz * ((g.ny + yc - 1) / yc) * NS < 512) yc /= 2;
+    const int nyc = (g.ny + yc - 1) / yc;
+    long long nb = (long long)ntx * nyc * g.nz;
+    if (nb > 768 / NS) nb = 768 / NS;
+    const size_t wpart = (size_t)NS * nb * 27 * CS * COUT;
+    if (wpart + nb * COUT > N->fpart_n) return -1;
+    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, CS>), dim3((unsigned)nb, NS), dim3(256), 0, st, in, dy, N->fpart,
+                       N->fpart + wpart, g, ntx, nyc, yc);
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblk((size_t)27 * cin * COUT + COUT, 16)), dim3(256), 0, st, N->fpart,
+                       N->fpart + wpart, grad, bias, (int)nb, CS, cin, COUT);
     return 0;
 }
 static int wgrad_run(hipStream_t st, UNet *N, int cinp, int cin, int cout, const bf16 *in, const bf16 *dy, Vol g,
-                     float *grad) {
-#define CASE(a, b) \
-    if (cinp == a && cout == b) return wgrad_launch<a, b>(st, N, in, dy, g, grad, cin);
-    CASE(8, 16) CASE(16, 16) CASE(16, 32) CASE(32, 32) CASE(32, 64) CASE(64, 64) CASE(96, 32) CASE(48, 16)
+                     float *grad, float *bias) {
+#define CASE(a, b, cs) \
+    if (cinp == a && cout == b) return wgrad_launch<a, b, cs>(st, N, in, dy, g, grad, bias, cin);
+    CASE(8, 16, 8) CASE(16, 16, 16) CASE(16, 32, 16) CASE(32, 32, 32) CASE(32, 64, 16) CASE(64, 64, 16)
+    CASE(96, 32, 32) CASE(48, 16, 48)
 #undef CASE
     return -1;
-}
-template <int COUT>
-static void colsum_launch(hipStream_t st, UNet *N, const bf16 *dy, int nv, float *out) {
-    int nb = (nv + 16383) / 16384;
-    if (nb > 256) nb = 256;
-    const int vpb = (nv + nb - 1) / nb;
-    nb = (nv + vpb - 1) / vpb;
-    hipLaunchKernelGGL(colsum_kernel<COUT>, dim3(nb), dim3(256), 0, st, dy, N->fpart, nv, vpb);
-    hipLaunchKernelGGL(colsum_reduce_kernel, dim3(1), dim3(64), 0, st, N->fpart, out, nb, COUT);
-}
-static void colsum_run(hipStream_t st, UNet *N, int cout, const bf16 *dy, int nv, float *out) {
-    if (cout == 16) colsum_launch<16>(st, N, dy, nv, out);
-    else if (cout == 32) colsum_launch<32>(st, N, dy, nv, out);
-    else colsum_launch<64>(st, N, dy, nv, out);
 }
 
 static int refresh_layouts(UNet *N, hipStream_t st) {
@@ -831,7 +949,7 @@ UNet *unet_create(int nx, int ny, int nz, int inc, uint64_t seed, char *err, siz
     A((void **)&N->scal, 8 * 8);
     const int nbh = nblk(n0);
     A((void **)&N->dpart, (size_t)(nbh > 4096 ? nbh : 4096) * 18 * 8);
-    N->fpart_n = (size_t)64 * 27 * 8 * 1024;  // blocks × taps × groups × (cin·cout) bound
+    N->fpart_n = (size_t)768 * (27 * 1024 + 64);  // blocks × (taps × (channels · outputs) + outputs), wgrad_launch's bounds
     A((void **)&N->fpart, N->fpart_n * 4);
     if (!ok) {
         snprintf(err, errlen, "hipMalloc failed for the U-Net buffers");
@@ -906,60 +1024,59 @@ int unet_backward(UNet *N, hipStream_t st, const double *target) {
                        N->g0b16, N->dpart, n0);
     hipLaunchKernelGGL(head_reduce_kernel, dim3(18), dim3(256), 0, st, N->dpart, nbh, n0, N->scal, G + N->headoff);
     // layer 9 (16 → 16 at full resolution): g9 in g0b16
-    auto layer_grads = [&](int l, const bf16 *in, const bf16 *g, Vol gv, int nv) {
-        rc |= wgrad_run(st, N, L[l].cinp, L[l].cin, L[l].cout, in, g, gv, G + L[l].woff);
-        colsum_run(st, N, L[l].cout, g, nv, G + L[l].boff);
+    auto layer_grads = [&](int l, const bf16 *in, const bf16 *g, Vol gv) {
+        rc |= wgrad_run(st, N, L[l].cinp, L[l].cin, L[l].cout, in, g, gv, G + L[l].woff, G + L[l].boff);
     };
-    layer_grads(9, N->a8, N->g0b16, N->g0, n0);
+    layer_grads(9, N->a8, N->g0b16, N->g0);
     rc |= conv_run(st, 16, 16, N->g0b16, L[9].wt, nullptr, N->g1b16, 16, 0, N->g0, 0);
     hipLaunchKernelGGL(relu_mask_kernel, dim3(nblk((size_t)n0 * 16)), dim3(UB), 0, st, N->g1b16, 16, 0, N->a8, 16, 0,
                        N->g1b16, 16, n0);
     // layer 8 (cat0 48 → 16)
-    layer_grads(8, N->cat0, N->g1b16, N->g0, n0);
+    layer_grads(8, N->cat0, N->g1b16, N->g0);
     rc |= conv_run(st, 16, 48, N->g1b16, L[8].wt, nullptr, N->gcat0, 48, 0, N->g0, 0);
     // up (a7 → cat0[0:32)) backward with a7's mask → g7 (level 1, 32)
     hipLaunchKernelGGL(up_back_kernel, dim3(nblk((size_t)n1 * 32)), dim3(UB), 0, st, N->gcat0, 48, 0, N->a7, N->g1l, 32,
                        N->g0);
     // layer 7 (32 → 32 at 1/2)
-    layer_grads(7, N->a6, N->g1l, N->g1, n1);
+    layer_grads(7, N->a6, N->g1l, N->g1);
     rc |= conv_run(st, 32, 32, N->g1l, L[7].wt, nullptr, N->g2l, 32, 0, N->g1, 0);
     hipLaunchKernelGGL(relu_mask_kernel, dim3(nblk((size_t)n1 * 32)), dim3(UB), 0, st, N->g2l, 32, 0, N->a6, 32, 0,
                        N->g2l, 32, n1);
     // layer 6 (cat1 96 → 32)
-    layer_grads(6, N->cat1, N->g2l, N->g1, n1);
+    layer_grads(6, N->cat1, N->g2l, N->g1);
     rc |= conv_run(st, 32, 96, N->g2l, L[6].wt, nullptr, N->gcat1, 96, 0, N->g1, 0);
     // up (a5 → cat1[0:64)) backward with a5's mask → g5 (level 2, 64)
     hipLaunchKernelGGL(up_back_kernel, dim3(nblk((size_t)n2 * 64)), dim3(UB), 0, st, N->gcat1, 96, 0, N->a5, N->gl2a, 64,
                        N->g1);
     // layer 5 (64 → 64 at 1/4)
-    layer_grads(5, N->a4, N->gl2a, N->g2, n2);
+    layer_grads(5, N->a4, N->gl2a, N->g2);
     rc |= conv_run(st, 64, 64, N->gl2a, L[5].wt, nullptr, N->gl2b, 64, 0, N->g2, 0);
     hipLaunchKernelGGL(relu_mask_kernel, dim3(nblk((size_t)n2 * 64)), dim3(UB), 0, st, N->gl2b, 64, 0, N->a4, 64, 0,
                        N->gl2b, 64, n2);
     // layer 4 (p1 32 → 64)
-    layer_grads(4, N->p1, N->gl2b, N->g2, n2);
+    layer_grads(4, N->p1, N->gl2b, N->g2);
     rc |= conv_run(st, 64, 32, N->gl2b, L[4].wt, nullptr, N->gp1, 32, 0, N->g2, 0);
     // skip1: pool backward + cat1[64:96) slice, masked by skip1 → g3 (level 1, 32)
     hipLaunchKernelGGL(skip_back_kernel, dim3(nblk((size_t)n1 * 32)), dim3(UB), 0, st, N->gp1, N->gcat1, N->cat1, 96, 64,
                        N->g1l, 32, N->g1);
     // layer 3 (a2 32 → 32)
-    layer_grads(3, N->a2, N->g1l, N->g1, n1);
+    layer_grads(3, N->a2, N->g1l, N->g1);
     rc |= conv_run(st, 32, 32, N->g1l, L[3].wt, nullptr, N->g2l, 32, 0, N->g1, 0);
     hipLaunchKernelGGL(relu_mask_kernel, dim3(nblk((size_t)n1 * 32)), dim3(UB), 0, st, N->g2l, 32, 0, N->a2, 32, 0,
                        N->g2l, 32, n1);
     // layer 2 (p0 16 → 32)
-    layer_grads(2, N->p0, N->g2l, N->g1, n1);
+    layer_grads(2, N->p0, N->g2l, N->g1);
     rc |= conv_run(st, 32, 16, N->g2l, L[2].wt, nullptr, N->gp0, 16, 0, N->g1, 0);
     // skip0: pool backward + cat0[32:48) slice, masked by skip0 → g1 (full, 16)
     hipLaunchKernelGGL(skip_back_kernel, dim3(nblk((size_t)n0 * 16)), dim3(UB), 0, st, N->gp0, N->gcat0, N->cat0, 48, 32,
                        N->g0b16, 16, N->g0);
     // layer 1 (a0 16 → 16)
-    layer_grads(1, N->a0, N->g0b16, N->g0, n0);
+    layer_grads(1, N->a0, N->g0b16, N->g0);
     rc |= conv_run(st, 16, 16, N->g0b16, L[1].wt, nullptr, N->g1b16, 16, 0, N->g0, 0);
     hipLaunchKernelGGL(relu_mask_kernel, dim3(nblk((size_t)n0 * 16)), dim3(UB), 0, st, N->g1b16, 16, 0, N->a0, 16, 0,
                        N->g1b16, 16, n0);
     // layer 0 (x0 → 16)
-    layer_grads(0, N->x0, N->g1b16, N->g0, n0);
+    layer_grads(0, N->x0, N->g1b16, N->g0);
     return rc ? -1 : (hipGetLastError() == hipSuccess ? 0 : -2);
 }
 
