@@ -81,6 +81,22 @@ __device__ __forceinline__ void xcd_block3(int &bx, int &by, int &bz) {
     by = (int)(l / (gz * gx));
 }
 
+// Levels per chunk of a kernel whose blocks march `tiles` columns of nz
+// levels: a block costs its kc levels and about `start` more (the first
+// level's windows and faces), and the chip takes `fill` blocks a round. On a
+// large grid that is the longest chunk, kmax; on a small one, chunks short
+// enough to occupy the chip.
+inline int chunk_levels(int tiles, int nz, int kmax, int fill, int start) {
+    int best = 1;
+    long long cost = -1;
+    for (int kc = 1; kc <= kmax && kc <= nz; kc++) {
+        const long long blocks = (long long)tiles * ((nz + kc - 1) / kc);
+        const long long c = (blocks + fill - 1) / fill * (kc + start);
+        if (cost < 0 || c <= cost) { cost = c; best = kc; }
+    }
+    return best;
+}
+
 __device__ __forceinline__ uint32_t lin(int i, int j, int k, int sx, int sy) {
     return (uint32_t)i + (uint32_t)sx * ((uint32_t)j + (uint32_t)sy * (uint32_t)k);
 }

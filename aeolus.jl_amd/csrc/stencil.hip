@@ -482,6 +482,11 @@ __device__ __forceinline__ T win_zface(const T *wf, const T *ww, const T *wt, in
 // within 2 %).
 constexpr int TILE_MINW = 4;
 constexpr int TILE_KC = 16;
+// Blocks a round: one per CU (a second one shares the CU's FP64 units). RK3
+// step, 16 levels on every grid → by chunk_levels: 32³ periodic 507 → 164 us,
+// 90×72×50 with the closure 706 → 404, 128×96×64 679 → 468, 160×160×90
+// 1166 → 1014, 256×256×128 unchanged (16 levels).
+constexpr int TILE_FILL = 256;
 
 template <int MODE, int S, int P, typename T, int BY, int STR>
 __global__ void __launch_bounds__(MW *BY, TILE_MINW) adv_tile_kernel(MarchArgs<T> a) {
@@ -774,7 +779,7 @@ static void launch_march_sp(hipStream_t st, const MarchArgs<T> &a) {
     const Metrics<T> &m = a.m;
     if constexpr (MODE != MODE_SCALAR) {
         MarchArgs<T> t = a;
-        t.kc = m.Nz < TILE_KC ? m.Nz : TILE_KC;
+        t.kc = chunk_levels(((m.Nx + MW - 1) / MW) * ((m.Ny + BY - 1) / BY), m.Nz, TILE_KC, TILE_FILL, 1);
         dim3 grid((m.Nx + MW - 1) / MW, (m.Ny + BY - 1) / BY, (m.Nz + t.kc - 1) / t.kc);
         if (m.stretched)
             hipLaunchKernelGGL((adv_tile_kernel<MODE, S, P, T, BY, 1>), grid, dim3(MW, BY), 0, st, t);
@@ -853,7 +858,11 @@ int launch_advect(hipStream_t st, const Metrics<T> &m, int mode, int scheme, int
     a.m = m;
     a.in = Fields<T>{u, v, w, s};
     a.tu = tu; a.tv = tv; a.tw = tw; a.ts = ts;
-    a.kc = m.Nz < KCM ? m.Nz : KCM;
+    // the brick kernel holds several blocks per CU: shorter chunks pay only
+    // where KCM leaves CUs without a block (33×29×25 FP64 20.6 → 5.5 us,
+    // 130×70×60 WENO-Z7 35.6 → 31.9; 187×141×75 FP32 31.9, 33.3 if shortened)
+    const int tiles = ((m.Nx + MW - 1) / MW) * ((m.Ny + 7) / 8), kmax = m.Nz < KCM ? m.Nz : KCM;
+    a.kc = tiles * ((m.Nz + kmax - 1) / kmax) >= 256 ? kmax : chunk_levels(tiles, m.Nz, kmax, 256, 3);
     if (mode == MODE_SCALAR) return launch_march_mode<MODE_SCALAR, T>(st, a, scheme, p);
     return launch_march_mode<MODE_MOMENTUM, T>(st, a, scheme, p);
 }
@@ -881,7 +890,6 @@ int launch_tendency_step(hipStream_t st, const Metrics<T> &m, int scheme, int p,
     a.has_cor = ph.fcor != 0;
     a.spg = (const T *)ph.sponge;
     stage_coeffs(stage, &ph, &a.ca, &a.cb, &a.combine);
-    a.kc = m.Nz < KCM ? m.Nz : KCM;
     return launch_march_mode<MODE_STEP, T>(st, a, scheme, p);
 }
 template int launch_tendency_step<double>(hipStream_t, const Metrics<double> &, int, int, const double *,
