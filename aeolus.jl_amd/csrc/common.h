@@ -85,11 +85,11 @@ __device__ __forceinline__ void xcd_block3(int &bx, int &by, int &bz) {
 // levels: a block costs its kc levels and about `start` more (the first
 // level's windows and faces), and the chip takes `fill` blocks a round. On a
 // large grid that is the longest chunk, kmax; on a small one, chunks short
-// enough to occupy the chip.
-inline int chunk_levels(int tiles, int nz, int kmax, int fill, int start) {
-    int best = 1;
+// enough to occupy the chip. The length is a multiple of `step`, or nz.
+inline int chunk_levels(int tiles, int nz, int kmax, int fill, int start, int step = 1) {
+    int best = nz;
     long long cost = -1;
-    for (int kc = 1; kc <= kmax && kc <= nz; kc++) {
+    for (int kc = step; kc <= kmax && kc <= nz; kc += step) {
         const long long blocks = (long long)tiles * ((nz + kc - 1) / kc);
         const long long c = (blocks + fill - 1) / fill * (kc + start);
         if (cost < 0 || c <= cost) { cost = c; best = kc; }

@@ -194,10 +194,13 @@ __device__ __forceinline__ T rb_value(const LevelD<T> &L, int i, int j, int k, T
 // one colour of the red-black Gauss-Seidel sweep (_rbgs_body!, src/Multigrid.jl:307-337):
 // colour c updates the cells with (i + j + k + c) even in 0-based interior
 // indices (the reference's i = 2ih + ((j + k + c) & 1) in unit-halo storage).
-// SMODE folds a pending mean removal φ ← φ − m (m = mptr[0]) into a sweep as
-// rbgs_tf_kernel does: 1 reads every φ less m, 2 only the cell's own old
-// value; 3 is the first pass from φ = 0 (reads no φ; the pair's other cell
-// is written zero). bm: b is read less bm[0] (a pending mean of b)
+// SMODE folds a pending mean removal φ ← φ − m (m = mptr[0], shift_kernel's
+// values) into a sweep's two passes: 1, the first, reads every φ less m (its
+// neighbours are the other colour, not written in this pass); 2, the second,
+// whose neighbours the first wrote in the shifted frame, takes only its own
+// old value less m (a blocked cell keeps it, a mirror boundary makes it its
+// own neighbour); 3 is the first pass from φ = 0 (reads no φ; the pair's
+// other cell is written zero). bm: b is read less bm[0] (a pending mean of b)
 template <typename T, int SMODE>
 __global__ void rbgs_kernel(LevelD<T> L, int colour, const double *__restrict__ mptr, const double *__restrict__ bm) {
     constexpr bool Z = SMODE == 3;
@@ -230,25 +233,23 @@ __global__ void rbgs_kernel(LevelD<T> L, int colour, const double *__restrict__ 
 // over a chunk of levels [k0, k1) (FP64; FP32 for the FP32 V-cycle): ρJ_x on the column's west and east
 // faces and ρJ_y on its south and north faces at the cell levels, ρJG^σσ on
 // its σ-faces k0 … k1 (tfw_mgcoef_kernel's expressions at the storage indices
-// (i + H, j + H, k + H)). ρ̄ = ρ0 exp(−z/H_s) is evaluated by exp at the
-// chunk's first level (and at the σ-face k1, the next chunk's first) and
-// carried upwards by its ratio between levels, exp(−Δz J_f/H_s): a product
-// per face and level in place of an exp per face and cell. Every thread that
-// evaluates a face forms the same products from the same first value (the
-// chunks are the same for all columns, both colours and the residual), so
-// the two cells of a face see one coefficient and the operator stays
-// symmetric; the FP64 values are within 32 ulp of the stored arrays'
-// (which still build the coarser levels).
+// (i + H, j + H, k + H)), each times 1/Δ² of its axis. ρ̄ = ρ0 exp(−z/H_s) is
+// evaluated by exp at the chunk's first level (and at the σ-face k1, the next
+// chunk's first), and a face's coefficient is carried upwards by ρ̄'s ratio
+// between levels, exp(−Δz J_f/H_s): a product per face and level in place of
+// an exp, with the level-independent factors folded into the carried value.
+// The chunks are the same for all columns, both colours and the residual, so
+// the two cells of a face form the same products (a red-black pass steps two
+// levels at once: the same to rounding). The FP64 values are within 32 ulp of
+// the stored arrays' (which still build the coarser levels).
 template <typename T>
 struct TFChain {
-    T Jxm, Jxp, Jym, Jyp, Jc, g2, iJJ;
-    T exm, exq, eym, eyp, ez, ez1;  // ρ̄ on the faces at the current level (ez: its lower σ-face); ez1: σ-face k1
-    T qxm, qxp, qym, qyp, qz;       // ρ̄'s ratio between consecutive levels on each face column
-    __device__ __forceinline__ void init(const TFM<T> &gm, int I, int J, int K0, int K1) {
-        const T hxm = gm.hxf(I, J), hxp = gm.hxf(I + 1, J), hym = gm.hyf(I, J), hyp = gm.hyf(I, J + 1);
-        Jxm = gm.Jx(I, J); Jxp = gm.Jx(I + 1, J); Jym = gm.Jy(I, J); Jyp = gm.Jy(I, J + 1);
-        const T hc = gm.hp(I, J);
-        Jc = gm.J(I, J);
+    T g2, iJJ, t, dz;              // σ_x² + σ_y² over (H − σ)², 1/J²; H − σ at the current lower σ-face
+    T xm, xp, ym, yp, z, z1;       // the carried values at the current level (z: its lower σ-face); z1: σ-face k1
+    T qxm, qxp, qym, qyp, qz;      // their ratio between consecutive levels
+    __device__ __forceinline__ void init(const TFM<T> &gm, const LevelD<T> &L, int I, int J, int K0, int K1) {
+        const T Jxm = gm.Jx(I, J), Jxp = gm.Jx(I + 1, J), Jym = gm.Jy(I, J), Jyp = gm.Jy(I, J + 1);
+        const T hc = gm.hp(I, J), Jc = gm.J(I, J);
         const T den = gm.Hl - hc, ax = (T)gm.hx[I + gm.sx * J] / den, ay = (T)gm.hy[I + gm.sx * J] / den;
         g2 = ax * ax + ay * ay;
         iJJ = 1 / (Jc * Jc);
@@ -257,84 +258,94 @@ struct TFChain {
             else return exp(-(gm.dz * Jf) * gm.iHs);
         };
         const T sc = gm.sigc(K0);
-        exm = gm.rho(hxm + sc * Jxm); exq = gm.rho(hxp + sc * Jxp);
-        eym = gm.rho(hym + sc * Jym); eyp = gm.rho(hyp + sc * Jyp);
-        ez = gm.rho(hc + gm.sigf(K0) * Jc);
-        ez1 = gm.rho(hc + gm.sigf(K1) * Jc);
+        xm = gm.rho(gm.hxf(I, J) + sc * Jxm) * Jxm * L.ix2;
+        xp = gm.rho(gm.hxf(I + 1, J) + sc * Jxp) * Jxp * L.ix2;
+        ym = gm.rho(gm.hyf(I, J) + sc * Jym) * Jym * L.iy2;
+        yp = gm.rho(gm.hyf(I, J + 1) + sc * Jyp) * Jyp * L.iy2;
+        z = gm.rho(hc + gm.sigf(K0) * Jc) * Jc * L.iz2;
+        z1 = gm.rho(hc + gm.sigf(K1) * Jc) * Jc * L.iz2;
+        t = gm.Hl - gm.sigf(K0);
+        dz = gm.dz;
         qxm = ratio(Jxm); qxp = ratio(Jxp); qym = ratio(Jym); qyp = ratio(Jyp); qz = ratio(Jc);
     }
-    __device__ __forceinline__ void step() { exm *= qxm; exq *= qxp; eym *= qym; eyp *= qyp; ez *= qz; }
-    // ρ̄ on the upper σ-face of the current level k (the σ-face k1 by exp)
-    __device__ __forceinline__ T ez_up(int k, int k1) const { return k + 1 < k1 ? ez * qz : ez1; }
-    // ρJG^σσ = ρ̄ J ((σ_x² + σ_y²) + 1/J²) at the σ-face K, σ_x = −(H − σ) h_x/(H − h)
-    __device__ __forceinline__ T fz(const TFM<T> &gm, T e, int K) const {
-        const T t = gm.Hl - gm.sigf(K);
-        return e * Jc * ((t * t) * g2 + iJJ);
+    __device__ __forceinline__ void step() { xm *= qxm; xp *= qxp; ym *= qym; yp *= qyp; z *= qz; t -= dz; }
+    // ρJG^σσ = ρ̄ J ((σ_x² + σ_y²) + 1/J²), σ_x = −(H − σ) h_x/(H − h), on the current level k's σ-faces
+    // (the upper one of the chunk's last level by exp)
+    static __device__ __forceinline__ T ma(T a, T b, T c) {
+        if constexpr (sizeof(T) == 4) return __builtin_fmaf(a, b, c);
+        else return __builtin_fma(a, b, c);
+    }
+    __device__ __forceinline__ T lower() const { return z * ma(t * t, g2, iJJ); }
+    __device__ __forceinline__ T upper(int k, int k1, T qup) const {
+        const T tu = t - dz;
+        return (k + 1 < k1 ? z * qup : z1) * ma(tu * tu, g2, iJJ);
     }
 };
 
 // One colour of the red-black sweep on the terrain grid's finest level
 // (FP64), with the face coefficients evaluated from the Gal-Chen metrics
-// (TFChain) instead of read from the stored arrays: three arrays fewer per
-// pass. Thread (i, j) marches its column over a chunk of levels, updating
-// the colour's cells (every other level) and carrying the z-neighbour shared
-// by consecutive cells. Measured with φ and b colour-split, per FP64 step:
-// 2 rows × 32 levels 217.2 ms, 4 × 32 218.0, 4 × 16 220.5, 4 × 64 219.6,
-// 8 × 16 227.5; 1 × 32 and 2 × 24 within 0.5 ms of 2 × 32 (the residual
-// shares the shape, so the chunks of TFChain are the same in both).
+// (TFChain) instead of read from the stored arrays. Thread (i, j) marches its
+// column over a chunk of levels, updating the colour's cells (every other
+// level) and carrying the z-neighbour shared by consecutive cells. φ and b
+// are colour-split (SplitMap), so a pass reads the other colour's half of φ
+// and its own half of b and writes its own half of φ: 3 × 4 bytes per cell.
+// A cell's own old value is read only where the diagonal vanishes.
+// FROM0, a cycle's first pass (colour 0): φ is zero, so no φ is read and
+// b/diag written; the other colour's half is not needed before the next pass
+// has written it, except where a mirror boundary makes a cell its own
+// neighbour, and there that pass takes zero (first).
+// SUM, a cycle's last pass: the block sums of b·φ, φ and b (what the CG needs
+// of z = φ), of the updated cells and of the other colour's, whose φ the pass
+// reads as z-neighbours.
+// Measured at 512×512×256: 257 us and 1.22 GB per pass with every cell's old
+// value read → 221 us and 1.01 GB (4.6 TB/s; 0.81 GB is the least, the rest
+// the neighbouring strips' lines). It is bound by memory: half the VALU work
+// per cell, the next cell's loads issued ahead, 4 rows or 64 levels per block
+// all stay within 2 %; blocks in XCD-contiguous rows are 5 % slower. From
+// zero 170 → 108 us. The pass with the three sums 261 us, where a mean pass
+// (100 us) and a pass over φ and r (183 us) read them before.
 constexpr int RBC_BY = 2;   // rows per block
-constexpr int RBC_KC = 32;  // levels per chunk
-// smode folds a pending mean removal φ ← φ − m (m = mptr[0], shift_kernel's
-// values) into a sweep's two passes: 1, the first pass, reads every φ less m
-// (its neighbours are the other colour, not written in this pass); 2, the
-// second pass, whose neighbours the first pass wrote in the shifted frame,
-// takes only its own old value less m: as itself (a fully blocked cell
-// keeps it) and where a mirror boundary makes it its own neighbour;
-// 3, the first pass from φ = 0: reads no φ, writes the colour's cells from
-// zero neighbours (the same values as from a cleared φ) and zero to the
-// other colour's, so φ needs no clearing pass before it
-// bm: L.b is the CG's r and b = r − bm[0] (load_rhs_kernel's values), read in place
-// SUM: the block sums of φ after the pass (all cells of the block's column
-// chunks: the updated cells and the other colour's, read as z-neighbours),
-// each column's levels in order, then the block's columns, into partials
-template <int SMODE, bool BM, bool SUM>
+constexpr int RBC_KC = 32;  // most levels per chunk
+constexpr int RBC_FILL = 2048;  // blocks a round (chunk_levels); 96×96×48 step 22.1 ms with 32 levels, 18.8 to 19.2 with 1024 or 2048 blocks
+template <bool FROM0, bool SUM>
 __global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, TFM<double> gm, int colour, int kc,
-                                                              const double *__restrict__ mptr,
-                                                              const double *__restrict__ bm,
-                                                              double *__restrict__ partials, uint32_t half,
-                                                              int bsp) {
-    constexpr int smode = SMODE;
-    constexpr bool Z = SMODE == 3;
-    static_assert(!(Z && SUM), "the from-zero pass is a sweep's first");
+                                                              int first, double *__restrict__ partials, int npb,
+                                                              uint32_t half) {
+    static_assert(!(FROM0 && SUM), "the from-zero pass is a sweep's first");
     const int i0 = blockIdx.x * 64 + threadIdx.x, j0 = blockIdx.y * RBC_BY + threadIdx.y;
     const bool ok = i0 < L.nx && j0 < L.ny;
     if (!SUM && !ok) return;
     const int i = ok ? i0 : 0, j = ok ? j0 : 0;
     const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, L.nz);
     const int I = i + gm.H, J = j + gm.H;
-    double sum = 0.0;
+    double srz = 0.0, sz = 0.0, sr = 0.0;
     TFChain<double> q;
-    q.init(gm, I, J, k0 + gm.H, k1 + gm.H);
+    q.init(gm, L, I, J, k0 + gm.H, k1 + gm.H);
     const double *f = L.phi;
-    const double ms = (smode == 1 || smode == 2) ? mptr[0] : 0.0;  // the pending mean
-    const double bmv = BM ? bm[0] : 0.0;            // r's mean
-    // a neighbour cn of cell cs, in the frame the update needs
+    // a neighbour cn of cell cs (cn == cs: a mirror boundary)
     auto nb = [&](uint32_t cn, uint32_t cs) {
-        if constexpr (Z) return 0.0;
-        return (smode == 1 || (smode == 2 && cn == cs)) ? f[cn] - ms : f[cn];
+        if constexpr (FROM0) return 0.0;
+        return first && cn == cs ? 0.0 : f[cn];
     };
     const int ixp = wrapc(i + 1, L.nx, L.bcx), ixm = wrapc(i - 1, L.nx, L.bcx);
     const int jyp = wrapc(j + 1, L.ny, L.bcy), jym = wrapc(j - 1, L.ny, L.bcy);
-    auto pi = [&](int ii, int jj, int kk) { return split_at(half, ii, jj, kk, lidx(L, ii, jj, kk)); };  // φ's index
+    auto pi = [&](int ii, int jj, int kk) { return split_at(half, ii, jj, kk, lidx(L, ii, jj, kk)); };  // the index of φ and b
     int k = k0 + ((i + j + k0 + colour) & 1);
     if (k > k0) q.step();
     double zm = 0.0;
-    if (Z && ok && k > k0) L.phi[pi(i, j, k0)] = 0.0;  // the chunk's first level, of the other colour
     if (ok && k < k1) {
-        zm = nb(pi(i, j, wrapc(k - 1, L.nz, L.bcz)), pi(i, j, k));
-        if (SUM && k - 1 >= k0) sum += zm;  // the chunk's first level, of the other colour
-    } else if (SUM && ok) {
-        for (int kk = k0; kk < k1; kk++) sum += f[pi(i, j, kk)];  // a chunk with none of this colour
+        const uint32_t cb = pi(i, j, wrapc(k - 1, L.nz, L.bcz));
+        zm = nb(cb, pi(i, j, k));
+        if (SUM && k - 1 >= k0) {  // the chunk's first level, of the other colour
+            const double bo = L.b[cb];
+            srz += bo * zm; sz += zm; sr += bo;
+        }
+    } else if (SUM && ok) {  // a chunk with none of this colour (one level)
+        for (int kk = k0; kk < k1; kk++) {
+            const uint32_t co = pi(i, j, kk);
+            const double bo = L.b[co], vo = f[co];
+            srz += bo * vo; sz += vo; sr += bo;
+        }
     }
     // the column's index offsets, in either layout: a neighbour on the cell's
     // level is the cell's index plus a constant of the column, the level
@@ -351,40 +362,212 @@ __global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, 
     };
     const uint32_t oxp = lat(ixp, j), oxm = lat(ixm, j), oyp = lat(i, jyp), oym = lat(i, jym);
     const uint32_t ozp = spl ? dbase + (nxy >> 1) : nxy, sstep = spl ? nxy : 2 * nxy;
-    uint32_t cs = pi(i, j, k), cb = lidx(L, i, j, k);  // φ's and b's indices of the cell
-    for (; ok && k < k1; k += 2, cs += sstep, cb += 2 * nxy) {
+    uint32_t cs = pi(i, j, k);  // the cell's index
+    // from here the chain steps two levels at once
+    const double qz = q.qz;
+    q.qxm *= q.qxm; q.qxp *= q.qxp; q.qym *= q.qym; q.qyp *= q.qyp; q.qz *= q.qz;
+    q.dz += q.dz;
+    for (; ok && k < k1; k += 2, cs += sstep) {
         const double xp = nb(cs + oxp, cs), xm = nb(cs + oxm, cs);
         const double yp = nb(cs + oyp, cs), ym = nb(cs + oym, cs);
         const uint32_t cu = k + 1 < L.nz ? cs + ozp : pi(i, j, wrapc(k + 1, L.nz, L.bcz));
         const double zp = nb(cu, cs);
-        const int K = k + gm.H;
-        const double fxp = q.exq * q.Jxp, fxm = q.exm * q.Jxm;
-        const double fyp = q.eyp * q.Jyp, fym = q.eym * q.Jym;
-        const double ezp = q.ez_up(k, k1);
-        const double fzp = q.fz(gm, ezp, K + 1), fzm = q.fz(gm, q.ez, K);
-        const uint32_t c = bsp ? cs : cb;  // b's index (bsp: b split as φ)
-        const double vnew = rb_value_c(L, BM ? L.b[c] - bmv : L.b[c], fxp, fxm, fyp, fym, fzp, fzm, xp, xm, yp, ym, zp,
-                                       zm, Z ? 0.0 : smode != 0 ? f[cs] - ms : f[cs]);
+        const double fzm = q.lower(), tu = q.t - gm.dz;
+        const double fzp = (k + 1 < k1 ? q.z * qz : q.z1) * __builtin_fma(tu * tu, q.g2, q.iJJ);
+        const double bv = L.b[cs];
+        const double diag = ((q.xp + q.xm) + (q.yp + q.ym)) + (fzp + fzm);  // −diag of A
+        double vnew;
+        if (diag < Eps<double>::v) {
+            vnew = FROM0 || first ? 0.0 : f[cs];
+        } else {
+            const double ox = __builtin_fma(q.xp, xp, q.xm * xm), oy = __builtin_fma(q.yp, yp, q.ym * ym);
+            const double oz = __builtin_fma(fzp, zp, __builtin_fma(fzm, zm, -bv));
+            vnew = qdiv<double>((ox + oy) + oz, diag);
+        }
         L.phi[cs] = vnew;
-        if (Z && k + 1 < k1) L.phi[cu] = 0.0;  // the level above, of the other colour
         if (SUM) {
-            sum += vnew;
-            if (k + 1 < k1) sum += zp;  // the level above, of the other colour, in the chunk
+            srz += bv * vnew; sz += vnew; sr += bv;
+            if (k + 1 < k1) {  // the level above, of the other colour, in the chunk
+                const double bo = L.b[cu];
+                srz += bo * zp; sz += zp; sr += bo;
+            }
         }
         zm = zp;  // the next cell's lower neighbour (k + 1, not updated in this colour)
         q.step();
-        q.step();
     }
     if constexpr (SUM) {
-        __shared__ double sh[RBC_BY];
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
-        if (threadIdx.x == 0) sh[threadIdx.y] = sum;
+        __shared__ double sh[RBC_BY][3];
+        for (int off = 32; off > 0; off >>= 1) {
+            srz += __shfl_down(srz, off, 64);
+            sz += __shfl_down(sz, off, 64);
+            sr += __shfl_down(sr, off, 64);
+        }
+        if (threadIdx.x == 0) { sh[threadIdx.y][0] = srz; sh[threadIdx.y][1] = sz; sh[threadIdx.y][2] = sr; }
         __syncthreads();
-        if (threadIdx.x == 0 && threadIdx.y == 0) {
+        if (threadIdx.x < 3 && threadIdx.y == 0) {
             double t = 0.0;
-            for (int q = 0; q < RBC_BY; q++) t += sh[q];
+            for (int w = 0; w < RBC_BY; w++) t += sh[w][threadIdx.x];
+            partials[threadIdx.x * npb + blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = t;
+        }
+    }
+}
+
+// The residual of the terrain grid's finest level restricted to the coarse
+// right-hand side (the mean of the 8 fine values), after a smoothing whose
+// last pass updated colour 1: those cells' equations then hold, so only the
+// colour-0 cells' residuals (4 of a coarse cell's 8) are formed, and r is
+// never stored. A cell with a mirror boundary is the exception, since its
+// update took its own old value for the missing neighbour: the colour-1 cells
+// of the bottom and top level are formed too (the lateral axes are periodic).
+// A wave is 32 pairs of columns (2I, 2I + 1) × the two rows of a coarse cell;
+// a thread marches its pair of columns over a chunk of levels, in column A on
+// the chunk's even levels and in B on the odd ones (each the colour-0 cell of
+// its level), with a TFChain of each column. Of a pair, the split layout has
+// both colours at one index, so the colour-1 value of the pair on levels
+// k − 1, k, k + 1 is the lower neighbour, the x neighbour inside the pair and
+// the upper neighbour: per level it loads six values. The rows' and levels'
+// sums meet in a lane exchange.
+// With partials, the block sums of the coarse values (for their mean).
+// Bound: memory, φ and half of b read, 13 B per fine cell. At 512×512×256:
+// residual 470 us + restriction 111 us → 202 us.
+constexpr int RRC_BW = 4;  // waves per block
+__global__ void __launch_bounds__(64 * RRC_BW) residual_restrict_tf_kernel(LevelD<double> L, LevelD<double> C,
+                                                                           TFM<double> gm, int kc,
+                                                                           double *__restrict__ partials,
+                                                                           uint32_t half) {
+    __shared__ double sh[RRC_BW];
+    const int lane = threadIdx.x, wv = threadIdx.y;
+    const int ci = blockIdx.x * 32 + (lane & 31), cj = blockIdx.y * RRC_BW + wv;
+    const bool ok = ci < C.nx && cj < C.ny;
+    const int pr = ok ? ci : 0, j = ok ? 2 * cj + (lane >> 5) : 0;
+    const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, L.nz);  // even
+    const uint32_t hx = (uint32_t)L.nx >> 1, pl = hx * (uint32_t)L.ny;  // pairs per row, per level
+    const int sA = j & 1;                                               // column A is 2·pr + sA (k0 even)
+    const int iA = 2 * pr + sA, iB = 2 * pr + 1 - sA;
+    TFChain<double> A, B;
+    A.init(gm, L, iA + gm.H, j + gm.H, k0 + gm.H, k1 + gm.H);
+    B.init(gm, L, iB + gm.H, j + gm.H, k0 + gm.H, k1 + gm.H);
+    // "xp" of a chain: the face towards the pair's other column
+    auto swapx = [](TFChain<double> &q) {
+        const double a = q.xm, c = q.qxm;
+        q.xm = q.xp; q.qxm = q.qxp;
+        q.xp = a; q.qxp = c;
+    };
+    if (sA) swapx(A); else swapx(B);
+    const int left = wrapc(2 * pr - 1, L.nx, L.bcx) >> 1, right = wrapc(2 * pr + 2, L.nx, L.bcx) >> 1;
+    const uint32_t oA = sA ? right : left, oB = sA ? left : right;  // the pair beyond the outer x face
+    const uint32_t jp = wrapc(j + 1, L.ny, L.bcy), jm = wrapc(j - 1, L.ny, L.bcy);
+    const double *f0 = L.phi, *f1 = L.phi + half, *b0 = L.b, *b1 = L.b + half;
+    // b − A φ of a cell of level k: its value c, the pair's other value xi, the
+    // outer x value xo, the y values, the z values
+    auto res = [&](const TFChain<double> &q, int k, double bv, double c, double xi, double xo, double yp, double ym,
+                   double zp, double zm) {
+        const double fzp = q.upper(k, k1, q.qz), fzm = q.lower();
+        const double ax = __builtin_fma(q.xp, xi - c, q.xm * (xo - c)), ay = __builtin_fma(q.yp, yp - c, q.ym * (ym - c));
+        const double az = __builtin_fma(fzp, zp - c, __builtin_fma(fzm, zm - c, -bv));
+        return -((ax + ay) + az);
+    };
+    const uint32_t row = hx * (uint32_t)j, rowp = hx * jp, rowm = hx * jm;
+    uint32_t base = pl * (uint32_t)k0;
+    // the pair's colour-1 value below, on and above the level (mirrored ends: unused)
+    double m0 = k0 > 0 ? f1[base - pl + row + pr] : (L.bcz == BC_PERIODIC ? f1[pl * (uint32_t)(L.nz - 1) + row + pr] : 0.0);
+    double m1 = f1[base + row + pr];
+    double cprev = 0.0, total = 0.0;
+    for (int k = k0; k < k1; k += 2) {
+        double r = 0.0;
+        auto level = [&](const TFChain<double> &q, const TFChain<double> &qo, uint32_t outer, uint32_t outer1, int kk) {
+            const uint32_t s = base + row + pr;
+            const double c = f0[s], bv = b0[s];
+            const bool top = kk + 1 == L.nz, per = L.bcz == BC_PERIODIC;
+            const double m2 = !top ? f1[s + pl] : (per ? f1[row + pr] : c);
+            const double xo = f1[base + row + outer];
+            const double yp = f1[base + rowp + pr], ym = f1[base + rowm + pr];
+            const bool bottom = kk == 0 && !per;
+            r += res(q, kk, bv, c, m1, xo, yp, ym, m2, bottom ? c : m0);
+            if (!per && (kk == 0 || top)) {
+                // the pair's colour-1 cell on a mirror boundary
+                const double xo1 = f0[base + row + outer1], yp1 = f0[base + rowp + pr], ym1 = f0[base + rowm + pr];
+                const double up = top ? m1 : f0[s + pl], dn = kk == 0 ? m1 : cprev;
+                r += res(qo, kk, b1[s], m1, c, xo1, yp1, ym1, up, dn);
+            }
+            m0 = m1;
+            m1 = m2;
+            cprev = c;
+            base += pl;
+        };
+        if (ok) level(A, B, oA, oB, k);
+        A.step();
+        B.step();
+        if (ok) level(B, A, oB, oA, k + 1);
+        A.step();
+        B.step();
+        r += __shfl_xor(r, 32, 64);
+        const double bc = r * 0.125;
+        if (ok && lane < 32) {
+            C.b[lidx(C, ci, cj, k >> 1)] = bc;
+            total += bc;
+        }
+    }
+    if (partials) {
+        for (int off = 16; off > 0; off >>= 1) total += __shfl_down(total, off, 64);
+        if (lane == 0) sh[wv] = total;
+        __syncthreads();
+        if (lane == 0 && wv == 0) {
+            double t = 0.0;
+            for (int w = 0; w < RRC_BW; w++) t += sh[w];
             partials[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = t;
         }
+    }
+}
+
+// φ += the trilinear correction (prolong_kernel's weights) on the terrain
+// grid's finest level, before a smoothing whose first pass updates colour 0:
+// that pass reads no colour-0 value, so only the colour-1 cells are
+// corrected. On a mirror boundary a cell is its own neighbour: both colours
+// of the bottom and top level are corrected.
+// A thread marches a pair of columns; its row's parity is the wave's, so
+// which column holds colour 1 on a level is uniform. The x-y part of the
+// weights is summed once per coarse level, for the pair's left and right
+// column, and kept for three coarse levels.
+// Bound: memory, half of φ read and written, 9 B per fine cell. At
+// 512×512×256: 258 us (both colours, one column per thread) → 142 us.
+constexpr int PRC_BY = 4;   // rows per block
+constexpr int PRC_KC = 16;  // most fine levels per chunk (even)
+constexpr int PRC_FILL = 1024;  // blocks a round (chunk_levels)
+__global__ void __launch_bounds__(64 * PRC_BY) prolong_tf_kernel(LevelD<double> F, LevelD<double> C, int kc,
+                                                                 uint32_t half) {
+    const int pr = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * PRC_BY + __builtin_amdgcn_readfirstlane(threadIdx.y);
+    if (pr >= C.nx || j >= F.ny) return;
+    const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, F.nz);
+    const int xl = wrapc(pr - 1, C.nx, C.bcx), xr = wrapc(pr + 1, C.nx, C.bcx);
+    const int J = j >> 1, jy = wrapc(J + ((j & 1) ? 1 : -1), C.ny, C.bcy);
+    // the x-y sums of coarse level m for the pair's columns 2·pr (l) and 2·pr + 1 (r)
+    auto plane = [&](int m, double &l, double &r) {
+        const int mm = wrapc(m, C.nz, C.bcz);
+        const uint32_t a = lidx(C, 0, J, mm), b = lidx(C, 0, jy, mm);
+        const double near = 0.75 * C.phi[a + pr] + 0.25 * C.phi[b + pr];
+        const double nl = 0.75 * C.phi[a + xl] + 0.25 * C.phi[b + xl], nr = 0.75 * C.phi[a + xr] + 0.25 * C.phi[b + xr];
+        l = 0.75 * near + 0.25 * nl;
+        r = 0.75 * near + 0.25 * nr;
+    };
+    double l0, r0, l1, r1, l2, r2;
+    plane((k0 >> 1) - 1, l0, r0);
+    plane(k0 >> 1, l1, r1);
+    const uint32_t hx = (uint32_t)F.nx >> 1, pl = hx * (uint32_t)F.ny;
+    uint32_t s = hx * (uint32_t)j + pr + pl * (uint32_t)k0;
+    double *f0 = F.phi, *f1 = F.phi + half;
+    const bool mirror = F.bcz != BC_PERIODIC;
+    const int odd = j & 1;  // on an even level colour 1 is the pair's right column in an even row
+    for (int k = k0; k < k1; k += 2) {
+        plane((k >> 1) + 1, l2, r2);
+        const double le = 0.75 * l1 + 0.25 * l0, re = 0.75 * r1 + 0.25 * r0;
+        const double lo = 0.75 * l1 + 0.25 * l2, ro = 0.75 * r1 + 0.25 * r2;
+        f1[s] += odd ? le : re;
+        if (mirror && k == 0) f0[s] += odd ? re : le;
+        f1[s + pl] += odd ? ro : lo;
+        if (mirror && k + 2 == F.nz) f0[s + pl] += odd ? lo : ro;
+        s += 2 * pl;
+        l0 = l1; r0 = r1; l1 = l2; r1 = r2;
     }
 }
 
@@ -403,69 +586,6 @@ __global__ void jacobi_kernel(LevelD<T> L, const T *__restrict__ src, T *__restr
     if (fabs(d) < Eps<T>::v) { dst[c] = x; return; }
     const T r = src ? L.b[c] - applyA(L, src, i, j, k) : L.b[c];
     dst[c] = x + omega * (r / d);
-}
-
-// residual_kernel on the terrain grid's finest level (FP64): r = b − Aφ with
-// the face coefficients of rbgs_tf_kernel (TFChain over the same chunks, so
-// the same operator to the bit), and the block sums of r. A thread marches
-// its column over a chunk of levels; a cell's bottom face is the level
-// below's top face (carried). The block sums add each column's levels in
-// order, then the columns of the block: another order than
-// residual_kernel's rows.
-// with mptr, φ is read less its pending mean (shift_kernel's values)
-__global__ void __launch_bounds__(64 * RBC_BY) residual_tf_kernel(LevelD<double> L, TFM<double> gm, int kc,
-                                                                  double *__restrict__ partials,
-                                                                  const double *__restrict__ mptr,
-                                                                  const double *__restrict__ bm, uint32_t half,
-                                                                  int bsp) {
-    __shared__ double sh[RBC_BY];
-    const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * RBC_BY + threadIdx.y;
-    const bool ok = i < L.nx && j < L.ny;
-    const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, L.nz);
-    const int ic = ok ? i : 0, jc = ok ? j : 0;
-    const int I = ic + gm.H, J = jc + gm.H;
-    TFChain<double> q;
-    q.init(gm, I, J, k0 + gm.H, k1 + gm.H);
-    const uint32_t ixp = wrapc(ic + 1, L.nx, L.bcx), ixm = wrapc(ic - 1, L.nx, L.bcx);
-    const uint32_t jyp = wrapc(jc + 1, L.ny, L.bcy), jym = wrapc(jc - 1, L.ny, L.bcy);
-    const double *f = L.phi;
-    const double m = mptr ? mptr[0] : 0.0;
-    const double bmv = bm ? bm[0] : 0.0;
-    auto rd = [&](uint32_t c) { return mptr ? f[c] - m : f[c]; };
-    double fzm = q.fz(gm, q.ez, k0 + gm.H);
-    auto pi = [&](int ii, int jj, int kk) { return split_at(half, ii, jj, kk, lidx(L, ii, jj, kk)); };  // φ's index
-    double c = ok ? rd(pi(ic, jc, k0)) : 0.0;
-    double zm = ok ? rd(pi(ic, jc, wrapc(k0 - 1, L.nz, L.bcz))) : 0.0;
-    double sum = 0.0;
-    for (int k = k0; k < k1; k++) {
-        const int K = k + gm.H;
-        const double fxm = q.exm * q.Jxm, fxp = q.exq * q.Jxp;
-        const double fym = q.eym * q.Jym, fyp = q.eyp * q.Jyp;
-        const double fzp = q.fz(gm, q.ez_up(k, k1), K + 1);
-        const double zp = ok ? rd(pi(ic, jc, wrapc(k + 1, L.nz, L.bcz))) : 0.0;
-        if (ok) {
-            const double xp = rd(pi(ixp, j, k)), xm = rd(pi(ixm, j, k));
-            const double yp = rd(pi(i, jyp, k)), ym = rd(pi(i, jym, k));
-            const double Ax = ((fxp * (xp - c) - fxm * (c - xm)) * L.ix2 + (fyp * (yp - c) - fym * (c - ym)) * L.iy2) +
-                              (fzp * (zp - c) - fzm * (c - zm)) * L.iz2;
-            const uint32_t cc = lidx(L, i, j, k), cbi = bsp ? pi(i, j, k) : cc;  // r's and b's indices
-            const double r = (bm ? L.b[cbi] - bmv : L.b[cbi]) - Ax;
-            L.r[cc] = r;
-            sum += r;
-        }
-        fzm = fzp;
-        zm = c;
-        c = zp;
-        q.step();
-    }
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
-    if (threadIdx.x == 0) sh[threadIdx.y] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-        double t = 0.0;
-        for (int q = 0; q < RBC_BY; q++) t += sh[q];
-        partials[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = t;
-    }
 }
 
 // The FP32 V-cycle's finest level on the terrain grid: damped Jacobi
@@ -496,20 +616,17 @@ __global__ void __launch_bounds__(64 * JTF_BY) jacobi_tf_kernel(LevelD<float> L,
     const int ic = ok ? i : 0, jc = ok ? j : 0;
     const int I = ic + gm.H, J = jc + gm.H;
     TFChain<float> q;
-    q.init(gm, I, J, k0 + gm.H, k1 + gm.H);
+    q.init(gm, L, I, J, k0 + gm.H, k1 + gm.H);
     const uint32_t ixp = wrapc(ic + 1, L.nx, L.bcx), ixm = wrapc(ic - 1, L.nx, L.bcx);
     const uint32_t jyp = wrapc(jc + 1, L.ny, L.bcy), jym = wrapc(jc - 1, L.ny, L.bcy);
-    float fzm = q.fz(gm, q.ez, k0 + gm.H);
+    float fzm = q.lower();
     float c = 0.f, zm = 0.f;
     if (src && ok) {
         c = src[lidx(L, ic, jc, k0)];
         zm = src[lidx(L, ic, jc, wrapc(k0 - 1, L.nz, L.bcz))];
     }
     for (int k = k0; k < k1; k++) {
-        const int K = k + gm.H;
-        const float fxm = q.exm * q.Jxm, fxp = q.exq * q.Jxp;
-        const float fym = q.eym * q.Jym, fyp = q.eyp * q.Jyp;
-        const float fzp = q.fz(gm, q.ez_up(k, k1), K + 1);
+        const float fzp = q.upper(k, k1, q.qz);
         float zp = 0.f;
         if (src && ok) zp = src[lidx(L, ic, jc, wrapc(k + 1, L.nz, L.bcz))];
         if (ok) {
@@ -518,13 +635,13 @@ __global__ void __launch_bounds__(64 * JTF_BY) jacobi_tf_kernel(LevelD<float> L,
             if (src) {
                 const float xp = src[lidx(L, ixp, j, k)], xm = src[lidx(L, ixm, j, k)];
                 const float yp = src[lidx(L, i, jyp, k)], ym = src[lidx(L, i, jym, k)];
-                Ax = ((fxp * (xp - c) - fxm * (c - xm)) * L.ix2 + (fyp * (yp - c) - fym * (c - ym)) * L.iy2) +
-                     (fzp * (zp - c) - fzm * (c - zm)) * L.iz2;
+                Ax = (__builtin_fmaf(q.xp, xp - c, q.xm * (xm - c)) + __builtin_fmaf(q.yp, yp - c, q.ym * (ym - c))) +
+                     __builtin_fmaf(fzp, zp - c, fzm * (zm - c));
             }
             if constexpr (MODE == 1) {
                 dst[cc] = L.b[cc] - Ax;
             } else {
-                const float d = -(((fxp + fxm) * L.ix2 + (fyp + fym) * L.iy2) + (fzp + fzm) * L.iz2);
+                const float d = -(((q.xp + q.xm) + (q.yp + q.ym)) + (fzp + fzm));
                 if (fabsf(d) < Eps<float>::v) {
                     dst[cc] = c;
                 } else {
@@ -584,6 +701,38 @@ __global__ void restrict_kernel(LevelD<T> C, LevelD<T> F, const double *__restri
     if (threadIdx.x == 0) partials[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = s;
 }
 
+// coarse b = the mean of the 8 fine residuals, where the last smoothing pass
+// updated colour 1 (the colour-1 equations then hold and only colour-0 cells
+// are formed, as in residual_restrict_tf_kernel; a cell on a mirror boundary
+// is formed whichever its colour), with the block sums of b when asked.
+// One coarse cell per work item; r is not stored.
+template <typename T>
+__global__ void residual_restrict_kernel(LevelD<T> C, LevelD<T> F, double *__restrict__ partials) {
+    __shared__ double sh[RB / 64];
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    double v = 0.0;
+    if (t < (uint32_t)C.nx * (uint32_t)C.ny * (uint32_t)C.nz) {
+        const uint32_t JK = t / (uint32_t)C.nx, I = t - JK * (uint32_t)C.nx, K = JK / (uint32_t)C.ny, J = JK - K * (uint32_t)C.ny;
+        const bool mx = F.bcx != BC_PERIODIC, my = F.bcy != BC_PERIODIC, mz = F.bcz != BC_PERIODIC;
+        T s = T(0);
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const int i = 2 * I + (q & 1), j = 2 * J + ((q >> 1) & 1), k = 2 * K + (q >> 2);
+            const bool even = (((q & 1) + ((q >> 1) & 1) + (q >> 2)) & 1) == 0;
+            if (even || (mx && (i == 0 || i == F.nx - 1)) || (my && (j == 0 || j == F.ny - 1)) ||
+                (mz && (k == 0 || k == F.nz - 1)))
+                s += F.b[lidx(F, i, j, k)] - applyA(F, F.phi, i, j, k);
+        }
+        const T bval = s * T(1.0 / 8);
+        C.b[t] = bval;
+        v = (double)bval;
+    }
+    if (partials) {
+        const double sb = block_sum(v, sh);
+        if (threadIdx.x == 0) partials[blockIdx.x] = sb;
+    }
+}
+
 // φ += trilinear correction (_prolong_body!, src/Multigrid.jl:415-432), with block sums of φ
 // with mcptr the coarse φ is read less its pending mean
 template <typename T>
@@ -629,13 +778,11 @@ __global__ void prolong_kernel(LevelD<T> F, LevelD<T> C, double *__restrict__ pa
 // coarse level per two fine levels, so each fine cell's eight coarse terms
 // are summed in prolong_kernel's order from registers. The block sums of φ
 // add each column's levels in order, then the block's columns.
-constexpr int PRC_BY = 4;   // rows per block
-constexpr int PRC_KC = 16;  // fine levels per chunk (even)
 template <typename T>
 __global__ void __launch_bounds__(64 * PRC_BY) prolong_col_kernel(LevelD<T> F, LevelD<T> C, int kc,
                                                                   double *__restrict__ partials,
                                                                   const double *__restrict__ mptr,
-                                                                  const double *__restrict__ mcptr, uint32_t half) {
+                                                                  const double *__restrict__ mcptr) {
     __shared__ double sh[PRC_BY];
     const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * PRC_BY + threadIdx.y;
     const bool ok = i < F.nx && j < F.ny;
@@ -672,7 +819,7 @@ __global__ void __launch_bounds__(64 * PRC_BY) prolong_col_kernel(LevelD<T> F, L
             acc += (f * n * f) * (far ? w[1][2] : w[1][0]);
             acc += (n * f * f) * (far ? w[2][2] : w[2][0]);
             acc += (f * f * f) * (far ? w[3][2] : w[3][0]);
-            const uint32_t c = split_at(half, i, j, k, lidx(F, i, j, k));  // the fine φ's index
+            const uint32_t c = lidx(F, i, j, k);
             const T val = (mptr ? F.phi[c] - m : F.phi[c]) + acc;
             F.phi[c] = val;
             sum += (double)val;
@@ -710,18 +857,11 @@ __global__ void split_copy_kernel(double *__restrict__ dst, const double *__rest
 }
 
 // block sums of an array (for a mean)
-// (sm: a is the colour-split finest φ, read in the natural order)
 template <typename T>
-__global__ void sum_kernel(const T *__restrict__ a, int n, double *__restrict__ partials,
-                           const double *__restrict__ mptr = nullptr, SplitMap sm = SplitMap{0, 0, 0, -1, -1}) {
+__global__ void sum_kernel(const T *__restrict__ a, int n, double *__restrict__ partials) {
     __shared__ double sh[RB / 64];
-    const T m = mptr ? (T)mptr[0] : T(0);
     double v = 0.0;
-    if (mptr)  // the sum of a − m (shift_kernel's values)
-        for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x)
-            v += (double)(a[split_t(sm, t)] - m);
-    else
-        for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) v += (double)a[split_t(sm, t)];
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) v += (double)a[t];
     double s = block_sum(v, sh);
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
@@ -890,19 +1030,18 @@ __global__ void cg_apply_kernel(LevelD<double> L, const double *__restrict__ p, 
     if (threadIdx.x == 0) partials[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = s;
 }
 
-// x += αp; r −= αAp; block sums of (r², r)  (α = num/den from the device)
-// bs: r also written colour-split into bs (the FP64 terrain cycle's finest b)
-__global__ void cg_update_kernel(double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
-                                 const double *__restrict__ Ap, const double *__restrict__ aptr, int n,
-                                 double *__restrict__ partials, int nblk, double *__restrict__ bs, SplitMap sm) {
+// r −= αAp, block sums of (r², r)  (α from the device; null: 0); sm: r is
+// colour-split, Ap natural
+__global__ void cg_update_kernel(double *__restrict__ r, const double *__restrict__ Ap,
+                                 const double *__restrict__ aptr, int n, double *__restrict__ partials, int nblk,
+                                 SplitMap sm) {
     __shared__ double sh[RB / 64];
     const double alpha = aptr ? aptr[0] : 0.0;
     double s2 = 0.0, s1 = 0.0;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
-        if (x) x[t] = x[t] + alpha * p[t];
-        const double rv = r[t] - alpha * Ap[t];
-        r[t] = rv;
-        if (bs) bs[split_t(sm, t)] = rv;
+        const uint32_t q = split_t(sm, t);
+        const double rv = r[q] - alpha * Ap[t];
+        r[q] = rv;
         s2 += rv * rv;
         s1 += rv;
     }
@@ -923,15 +1062,12 @@ __global__ void load_rhs_kernel(T *__restrict__ b, const double *__restrict__ r,
 template <typename T>
 __global__ void store_rz_kernel(double *__restrict__ z, const T *__restrict__ phi, const double *__restrict__ r, int n,
                                 const double *__restrict__ mptr, double *__restrict__ partials, int nblk,
-                                const double *__restrict__ ap, const double *__restrict__ m1ptr = nullptr,
-                                SplitMap sm = SplitMap{0, 0, 0, -1, -1}) {
+                                const double *__restrict__ ap) {
     __shared__ double sh[RB / 64];
     const double m = mptr ? mptr[0] : 0.0;
-    const T m1 = m1ptr ? (T)m1ptr[0] : T(0);  // φ's own mean, not yet removed (shift_kernel's value)
     double srz = 0.0, sz = 0.0, sr = 0.0, szap = 0.0;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
-        const T pv = phi[split_t(sm, t)];
-        const double zv = (double)(m1ptr ? pv - m1 : pv) - m;
+        const double zv = (double)phi[t] - m;
         if (z) z[t] = zv;
         srz += r[t] * zv;
         sz += zv;
@@ -981,23 +1117,21 @@ __global__ void cg_beta_kernel(double *scal, double dn, int flexible) {
 
 // p = (z − m) + βp  (_pcg_dir_body!, src/Backends.jl:1413-1417); first:
 // p = z − m. z is formed from the cycle's φ as store_rz_kernel forms it
-// (z = (φ − m1) − m2, m1 nullable), so that z is never stored; with x (not
-// first), x += αp from the p it replaces (cg_update_kernel's update, deferred
-// to the pass that reads p anyway)
+// (z = φ − m2, m2 nullable), so that z is never stored; not first, x += αp
+// from the p it replaces (the update of x deferred to the pass that reads p
+// anyway)
 template <typename T>
 __global__ void cg_dir_phi_kernel(double *__restrict__ p, const T *__restrict__ phi, int n,
-                                  const double *__restrict__ scal, int first, const double *__restrict__ m1ptr,
-                                  const double *__restrict__ m2ptr, double *__restrict__ x, SplitMap sm) {
-    const double m = scal[S_M], beta = scal[S_BETA], m2 = m2ptr[0], alpha = scal[S_ALPHA];
-    const T m1 = m1ptr ? (T)m1ptr[0] : T(0);
+                                  const double *__restrict__ scal, int first, const double *__restrict__ m2ptr,
+                                  double *__restrict__ x, SplitMap sm) {
+    const double m = scal[S_M], beta = scal[S_BETA], m2 = m2ptr ? m2ptr[0] : 0.0, alpha = scal[S_ALPHA];
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
-        const T pv = phi[split_t(sm, t)];
-        const double z = (double)(m1ptr ? pv - m1 : pv) - m2;
+        const double z = (double)phi[split_t(sm, t)] - m2;
         if (first) {
             p[t] = z - m;
         } else {
             const double pv = p[t];
-            if (x) x[t] = x[t] + alpha * pv;
+            x[t] = x[t] + alpha * pv;
             p[t] = (z - m) + beta * pv;
         }
     }
@@ -1102,21 +1236,19 @@ struct MGLevelH {
 struct MGPlan {
     int nlev = 0;
     bool gen0 = false;  // the finest level's coefficients from the terrain metrics (FP64 red-black)
+    int kc0 = RBC_KC;   // levels per chunk of its kernels
     TFM<double> gm{};
     bool gen0f = false;  // likewise in FP32 (FP32 Jacobi V-cycle)
     TFM<float> gmf{};
-    // the FP64 terrain finest level's b read in place from the CG's r, less
-    // its mean (slot 7): set by the preconditioner for its cycle
-    const double *b0 = nullptr;
     MGLevelH L[24];
-    // the FP64 red-black cycle's pending mean of a coarse level's b (set by
-    // the level above for the cycle's visit, null otherwise)
+    // the pending mean of a coarse level's b in a red-black cycle (set by the
+    // level above for the cycle's visit, null otherwise)
     const double *bmL[24] = {};
-    // the finest φ's colour split (SplitMap::half; 0: natural), on during an
-    // FP64 terrain PCG solve
+    // the colour split of the finest φ and b (SplitMap::half; 0: natural), on
+    // during an FP64 terrain PCG solve
     uint32_t half0 = 0;
-    // P->b0 is colour-split too (the CG update's copy of r in the finest b)
-    int b0split = 0;
+    // every cell of every level has a non-vanishing diagonal
+    bool open = false;
     int bcx, bcy, bcz, nu1, nu2, smoother, prec;  // prec 0 double, 1 float
     int wcycle = 0, fmg = 0;  // cycle = :W (two coarse recursions); the nested-iteration start
     double omega;
@@ -1142,13 +1274,6 @@ static LevelD<T> devlevel(const MGPlan *P, int l) {
     L.phi = (T *)h.phi; L.b = (T *)h.b; L.r = (T *)h.r; L.tmp = (T *)h.tmp;
     L.cx = (const T *)h.cx; L.cy = (const T *)h.cy; L.cz = (const T *)h.cz;
     L.bcx = P->bcx; L.bcy = P->bcy; L.bcz = P->bcz;
-    return L;
-}
-
-// the FP64 finest level with b read from the preconditioner's r when set
-static LevelD<double> level0_b(const MGPlan *P) {
-    LevelD<double> L = devlevel<double>(P, 0);
-    if (P->b0) L.b = (double *)P->b0;
     return L;
 }
 
@@ -1226,16 +1351,27 @@ static SplitMap split0(const MGPlan *P) {
     const bool pow2 = sx >= 0 && sy >= 0;
     return SplitMap{sizeof(T) == 8 ? P->half0 : 0u, nx, ny, pow2 ? sx : -1, pow2 ? sy : -1};
 }
-// the FP64 terrain finest level's red-black smoothing starts from zero in its first pass
-static bool rb_tf_from_zero(const MGPlan *P) { return P->smoother == 0 && P->nu1 >= 1 && P->gen0 && P->nlev > 1; }
+// A red-black cycle on an open operator (no fully blocked cell) with
+// smoothing on both sides of the coarse correction leaves out what changes no
+// iterate of the CG beyond rounding:
+//  - the mean removals inside the cycle: a constant is in the kernel of every
+//    level's operator, changes no residual and prolongs to a constant, and the
+//    residual and its restriction have the mean of b, which the CG keeps zero.
+//    Only the coarsest right-hand side's rounding is removed, which 50 sweeps
+//    would let drift. (With blocked cells the constant is not the whole
+//    kernel: a removal moves the fluid against the blocked cells' values.)
+//  - the residual of the colour the last pass updated, and the correction of
+//    the colour the next pass overwrites (residual_restrict_kernel,
+//    prolong_tf_kernel);
+//  - the clearing of φ: a cycle's first sweep starts from zero.
+static bool rb_cycle(const MGPlan *P) { return P->smoother == 0 && P->open && P->nu1 >= 1 && P->nu2 >= 1; }
 
+// m_first: a mean removal of φ still pending, folded into the first sweep
+// sums (FP64 terrain finest level): the last pass also writes the block sums
+// of b·φ, φ and b to P->part; their count goes to *sum_nb
 template <typename T>
-// m_first (FP64 terrain finest level only): a mean removal of φ still
-// pending, folded into the first sweep (rbgs_tf_kernel's smode)
-// sum_part (FP64 terrain finest level): the last pass also writes the block
-// sums of φ there; their count goes to *sum_nb
 static void smooth(MGPlan *P, hipStream_t st, int l, int nsweeps, bool from_zero = false,
-                   const double *m_first = nullptr, double *sum_part = nullptr, int *sum_nb = nullptr) {
+                   const double *m_first = nullptr, int *sum_nb = nullptr) {
     MGLevelH &h = P->L[l];
     LevelD<T> L = devlevel<T>(P, l);
     // the finest level's launches are booked one by one when profiling
@@ -1249,30 +1385,21 @@ static void smooth(MGPlan *P, hipStream_t st, int l, int nsweeps, bool from_zero
             for (int colour = 0; colour <= 1; colour++) {
                 ProfScope ps(tag);
                 if (gen) {
-                    const int kc = h.nz < RBC_KC ? h.nz : RBC_KC;
-                    const int smode = (from_zero && s == 0 && colour == 0) ? 3 : (m_first && s == 0) ? 1 + colour : 0;
-                    const bool last = s == nsweeps - 1 && colour == 1;
-                    const dim3 gr((h.nx + 63) / 64, (h.ny + RBC_BY - 1) / RBC_BY, (h.nz + kc - 1) / kc);
-                    const double *bm = P->b0 ? (const double *)(P->scal + 7) : (const double *)nullptr;
-                    double *part = (last && sum_part) ? sum_part : nullptr;
-                    if (part) *sum_nb = (int)(gr.x * gr.y * gr.z);
+                    const dim3 gr((h.nx + 63) / 64, (h.ny + RBC_BY - 1) / RBC_BY, (h.nz + P->kc0 - 1) / P->kc0);
+                    const int nb = (int)(gr.x * gr.y * gr.z);
+                    const bool zero = from_zero && s == 0;
+                    const bool sums = sum_nb && s == nsweeps - 1 && colour == 1;
                     auto launch = [&](auto kern) {
-                        hipLaunchKernelGGL(kern, gr, dim3(64, RBC_BY), 0, st, level0_b(P), P->gm, colour, kc, m_first, bm,
-                                           part, P->half0, P->b0split);
+                        hipLaunchKernelGGL(kern, gr, dim3(64, RBC_BY), 0, st, devlevel<double>(P, 0), P->gm, colour, P->kc0,
+                                           (int)(zero && colour == 1), P->part, nb, P->half0);
                     };
-                    if (part) {  // the last pass of a sweep (colour 1) with the sums
-                        if (bm) { if (smode == 2) launch(rbgs_tf_kernel<2, true, true>); else launch(rbgs_tf_kernel<0, true, true>); }
-                        else { if (smode == 2) launch(rbgs_tf_kernel<2, false, true>); else launch(rbgs_tf_kernel<0, false, true>); }
-                    } else if (bm) {
-                        if (smode == 3) launch(rbgs_tf_kernel<3, true, false>);
-                        else if (smode == 1) launch(rbgs_tf_kernel<1, true, false>);
-                        else if (smode == 2) launch(rbgs_tf_kernel<2, true, false>);
-                        else launch(rbgs_tf_kernel<0, true, false>);
+                    if (sums) {
+                        *sum_nb = nb;
+                        launch(rbgs_tf_kernel<false, true>);
+                    } else if (zero && colour == 0) {
+                        launch(rbgs_tf_kernel<true, false>);
                     } else {
-                        if (smode == 3) launch(rbgs_tf_kernel<3, false, false>);
-                        else if (smode == 1) launch(rbgs_tf_kernel<1, false, false>);
-                        else if (smode == 2) launch(rbgs_tf_kernel<2, false, false>);
-                        else launch(rbgs_tf_kernel<0, false, false>);
+                        launch(rbgs_tf_kernel<false, false>);
                     }
                 } else {
                     // the generic sweep: a pending b mean (bmL), the first pass
@@ -1318,20 +1445,42 @@ static void smooth(MGPlan *P, hipStream_t st, int l, int nsweeps, bool from_zero
 // W-cycle, whose second visit starts from the first one's φ.
 template <typename T>
 static bool coarse_fold(const MGPlan *P, int l) {
-    return sizeof(T) == 8 && P->prec == 0 && !P->wcycle && P->smoother == 0 && l >= 1 && 33 + 2 * l < MG_NSCAL;
+    return sizeof(T) == 8 && P->prec == 0 && !rb_cycle(P) && !P->wcycle && P->smoother == 0 && l >= 1 && 33 + 2 * l < MG_NSCAL;
 }
 
+static int prolong_chunk(const MGPlan *P) {
+    const MGLevelH &h = P->L[0];
+    return chunk_levels(((h.nx + 63) / 64) * ((h.ny + PRC_BY - 1) / PRC_BY), h.nz, PRC_KC, PRC_FILL, 2, 2);
+}
+
+// φ of level l += the prolongation of the coarse φ, with the block sums of
+// the result in P->part; returns their count. pre_m, mc: pending means of the
+// fine and the coarse φ
+template <typename T>
+static int prolong(MGPlan *P, hipStream_t st, int l, const double *pre_m, const double *mc) {
+    const MGLevelH &h = P->L[l];
+    const LevelD<T> L = devlevel<T>(P, l), C = devlevel<T>(P, l + 1);
+    if (l == 0 && h.nx % 2 == 0 && h.ny % 2 == 0 && h.nz % 2 == 0) {
+        const int kc = prolong_chunk(P);
+        const dim3 gp((h.nx + 63) / 64, (h.ny + PRC_BY - 1) / PRC_BY, (h.nz + kc - 1) / kc);
+        hipLaunchKernelGGL(prolong_col_kernel<T>, gp, dim3(64, PRC_BY), 0, st, L, C, kc, P->part, pre_m, mc);
+        return (int)(gp.x * gp.y * gp.z);
+    }
+    hipLaunchKernelGGL(prolong_kernel<T>, grid3(h.nx, h.ny, h.nz), dim3(RB), 0, st, L, C, P->part, pre_m, mc);
+    return nblocks3(h.nx, h.ny, h.nz);
+}
 // zero_start: φ of level l enters as zero (a preconditioner's cycle or the
 // first visit of a coarse level), so a Jacobi smoother's first sweep can
 // read it as zero without a clearing pass. defer_final: leave the
-// post-smoothing's mean removal pending, its mean in slot 4 (for the FP64
-// terrain finest level and the folded coarse levels); returns whether it
-// was left pending
+// post-smoothing's mean removal pending, its mean in slot 4 (for the folded
+// coarse levels); returns whether it was left pending. sum_nb: smooth's, for
+// the finest level's last pass
 template <typename T>
-static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer_final = false) {
+static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer_final = false, int *sum_nb = nullptr) {
     MGLevelH &h = P->L[l];
     const int n = h.nx * h.ny * h.nz;
     const bool cf = coarse_fold<T>(P, l);
+    const bool rb = rb_cycle(P) && P->nlev > 1;
     if (l == P->nlev - 1) {
         const int own = coarsest_slots(h.nx, h.ny, h.nz, sizeof(T));
         if (own >= 0) {
@@ -1339,7 +1488,7 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
             const int slots = (h.nx + 1) / 2 * h.ny * h.nz, bt = slots >= 1024 ? 1024 : (slots + 63) / 64 * 64;
             auto launch = [&](auto kern) {
                 hipLaunchKernelGGL(kern, dim3(1), dim3(bt), sizeof(T) * (size_t)n, st, devlevel<T>(P, l), 50, 1,
-                                   cf ? P->bmL[l] : (const double *)nullptr, (int)(cf && zero_start));
+                                   cf || rb ? P->bmL[l] : (const double *)nullptr, (int)((cf || rb) && zero_start));
             };
             if (own == 1) launch(coarsest_kernel<T, 1>);
             else if (own == 2) launch(coarsest_kernel<T, 2>);
@@ -1349,8 +1498,9 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
         } else {
             int sm = P->smoother;
             P->smoother = 0;
-            smooth<T>(P, st, l, 50, cf && zero_start);
+            smooth<T>(P, st, l, 50, (cf || rb) && zero_start);
             P->smoother = sm;
+            if (rb) return false;
             if (cf && defer_final) {
                 mean_to<T>(P, st, (const T *)h.phi, n, 4);
                 return true;
@@ -1361,28 +1511,47 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
     }
     MGLevelH &c = P->L[l + 1];
     const int nc = c.nx * c.ny * c.nz;
+    if (rb) {
+        smooth<T>(P, st, l, P->nu1, zero_start);
+        const bool last = l + 1 == P->nlev - 1;  // the coarsest right-hand side: its mean is left out
+        const LevelD<T> L = devlevel<T>(P, l), C = devlevel<T>(P, l + 1);
+        double *part = last ? P->part : nullptr;
+        const bool gen = sizeof(T) == 8 && l == 0 && P->gen0;
+        int nb;
+        if (gen) {
+            const dim3 gr((c.nx + 31) / 32, (c.ny + RRC_BW - 1) / RRC_BW, (h.nz + P->kc0 - 1) / P->kc0);
+            nb = (int)(gr.x * gr.y * gr.z);
+            hipLaunchKernelGGL(residual_restrict_tf_kernel, gr, dim3(64, RRC_BW), 0, st, devlevel<double>(P, 0),
+                               devlevel<double>(P, 1), P->gm, P->kc0, part, P->half0);
+        } else {
+            nb = stream_blocks(nc);
+            hipLaunchKernelGGL(residual_restrict_kernel<T>, dim3(nb), dim3(RB), 0, st, C, L, part);
+        }
+        if (last) {
+            P->bmL[l + 1] = P->scal + 32 + 2 * (l + 1);
+            finalize_to(P, st, P->scal + 32 + 2 * (l + 1), P->part, nb, 1.0 / nc);
+        }
+        for (int rec = 0; rec < (P->wcycle ? 2 : 1); rec++) vcycle<T>(P, st, l + 1, rec == 0);
+        P->bmL[l + 1] = nullptr;
+        if (gen) {
+            const int kc = prolong_chunk(P);
+            hipLaunchKernelGGL(prolong_tf_kernel, dim3((c.nx + 63) / 64, (h.ny + PRC_BY - 1) / PRC_BY, (h.nz + kc - 1) / kc),
+                               dim3(64, PRC_BY), 0, st, devlevel<double>(P, 0), devlevel<double>(P, 1), kc, P->half0);
+        } else {
+            prolong<T>(P, st, l, nullptr, nullptr);
+        }
+        smooth<T>(P, st, l, P->nu2, false, nullptr, sum_nb);
+        return false;
+    }
     // the FP32 V-cycle keeps only the projection that makes the coarsest
     // problem consistent (the restricted residual's mean): a constant in φ
     // is in the operator's kernel, changes no residual, and the CG removes
     // z's mean when it forms the direction
     const bool lean = P->prec != 0;
-    // the FP64 terrain finest level folds its mean removals into the kernels
-    // that read φ next (the same values): after the pre-smoothing into the
-    // residual (reads φ − m) and the prolongation (writes (φ − m) + e);
-    // after the prolongation into the first post-smoothing sweep; after the
-    // post-smoothing, with defer_final, into the caller's use of φ (the mean
-    // left in slot 4)
-    const bool fuse = !lean && l == 0 && sizeof(T) == 8 && P->gen0;
     const double *bm = cf ? P->bmL[l] : nullptr;  // b's pending mean
-    int nbs = 0;
-    smooth<T>(P, st, l, P->nu1,
-              zero_start && (jacobi_from_zero(P) || (fuse && rb_tf_from_zero(P)) || (cf && P->nu1 >= 1)), nullptr,
-              fuse ? P->part : nullptr, &nbs);
+    smooth<T>(P, st, l, P->nu1, zero_start && (jacobi_from_zero(P) || (cf && P->nu1 >= 1)));
     const double *pre_m = nullptr;  // φ's pending mean after the pre-smoothing
-    if (fuse) {
-        finalize_to(P, st, P->scal + 21, P->part, nbs, 1.0 / n);
-        pre_m = P->scal + 21;
-    } else if (cf) {
+    if (cf) {
         mean_to<T>(P, st, (const T *)h.phi, n, 33 + 2 * l);
         pre_m = P->scal + 33 + 2 * l;
     } else if (!lean) {
@@ -1395,15 +1564,7 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
     // an intermediate level's right-hand side drifts that level's φ by a
     // constant, which the next consistent level and the CG ignore)
     const bool consistent = !lean || l + 1 == P->nlev - 1;
-    int nb_r = nb;  // the residual's block sums
-    if (sizeof(T) == 8 && l == 0 && P->gen0) {
-        const int kc = h.nz < RBC_KC ? h.nz : RBC_KC;
-        const dim3 gr((h.nx + 63) / 64, (h.ny + RBC_BY - 1) / RBC_BY, (h.nz + kc - 1) / kc);
-        nb_r = (int)(gr.x * gr.y * gr.z);
-        hipLaunchKernelGGL(residual_tf_kernel, gr, dim3(64, RBC_BY), 0, st, level0_b(P), P->gm, kc, P->part,
-                           pre_m, P->b0 ? (const double *)(P->scal + 7) : (const double *)nullptr, P->half0,
-                           P->b0split);
-    } else if (sizeof(T) == 4 && l == 0 && P->gen0f && !consistent) {
+    if (sizeof(T) == 4 && l == 0 && P->gen0f && !consistent) {
         const int kc = h.nz < JTF_KC ? h.nz : JTF_KC;
         hipLaunchKernelGGL(jacobi_tf_kernel<1>, dim3((h.nx + 63) / 64, (h.ny + JTF_BY - 1) / JTF_BY, (h.nz + kc - 1) / kc),
                            dim3(64, JTF_BY), 0, st, devlevel<float>(P, 0), P->gmf, (const float *)h.phi,
@@ -1411,7 +1572,7 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
     } else {
         hipLaunchKernelGGL(residual_kernel<T>, grid3(h.nx, h.ny, h.nz), dim3(RB), 0, st, L, P->part, pre_m, bm);
     }
-    if (consistent) finalize_to(P, st, P->scal + 5, P->part, nb_r, 1.0 / n);
+    if (consistent) finalize_to(P, st, P->scal + 5, P->part, nb, 1.0 / n);
     int nbc = nblocks3(c.nx, c.ny, c.nz);
     hipLaunchKernelGGL(restrict_kernel<T>, grid3(c.nx, c.ny, c.nz), dim3(RB), 0, st, C, L,
                        consistent ? (const double *)(P->scal + 5) : (const double *)nullptr, P->part);
@@ -1434,32 +1595,15 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
     for (int rec = 0; rec < (P->wcycle ? 2 : 1); rec++) child_def = vcycle<T>(P, st, l + 1, rec == 0, ccf);
     P->bmL[l + 1] = nullptr;
     // prolong and correct (with the sum of the corrected φ), project
-    L = devlevel<T>(P, l);
-    C = devlevel<T>(P, l + 1);
-    int nb_p = nb;  // the prolongation's block sums
-    const double *mc = child_def ? (const double *)(P->scal + 4) : (const double *)nullptr;
-    if (l == 0 && h.nx % 2 == 0 && h.ny % 2 == 0 && h.nz % 2 == 0) {
-        const int kc = h.nz < PRC_KC ? h.nz : PRC_KC;
-        const dim3 gp((h.nx + 63) / 64, (h.ny + PRC_BY - 1) / PRC_BY, (h.nz + kc - 1) / kc);
-        nb_p = (int)(gp.x * gp.y * gp.z);
-        hipLaunchKernelGGL(prolong_col_kernel<T>, gp, dim3(64, PRC_BY), 0, st, L, C, kc, P->part, pre_m, mc,
-                           sizeof(T) == 8 ? P->half0 : 0u);
-    } else {
-        hipLaunchKernelGGL(prolong_kernel<T>, grid3(h.nx, h.ny, h.nz), dim3(RB), 0, st, L, C, P->part, pre_m, mc);
-    }
+    const int nb_p = prolong<T>(P, st, l, pre_m, child_def ? (const double *)(P->scal + 4) : (const double *)nullptr);
     // the corrected φ's mean: folded into the first post-smoothing sweep
-    const bool post_fold = fuse || (cf && P->nu2 >= 1);
+    const bool post_fold = cf && P->nu2 >= 1;
     if (!lean) {
         finalize_to(P, st, P->scal + 4, P->part, nb_p, 1.0 / n);
         if (!post_fold)
             hipLaunchKernelGGL(shift_kernel<T>, dim3(stream_blocks(n)), dim3(RB), 0, st, (T *)h.phi, n, P->scal + 4);
     }
-    smooth<T>(P, st, l, P->nu2, false, post_fold ? (const double *)(P->scal + 4) : (const double *)nullptr,
-              (fuse && defer_final) ? P->part : nullptr, &nbs);
-    if (fuse && defer_final) {
-        finalize_to(P, st, P->scal + 4, P->part, nbs, 1.0 / n);
-        return true;
-    }
+    smooth<T>(P, st, l, P->nu2, false, post_fold ? (const double *)(P->scal + 4) : (const double *)nullptr);
     if (cf && defer_final) {
         mean_to<T>(P, st, (const T *)h.phi, n, 4);
         return true;
@@ -1525,6 +1669,7 @@ MGPlan *mg_create(int nx, int ny, int nz, double dx, double dy, double dz, int b
     P->bcx = bcx; P->bcy = bcy; P->bcz = bcz; P->nu1 = nu1; P->nu2 = nu2; P->smoother = smoother;
     P->omega = omega; P->prec = prec;
     P->coeff = cx != nullptr;
+    P->open = !P->coeff;
     const size_t esz = prec == 0 ? 8 : 4;
     std::vector<double> hx, hy, hz;
     if (P->coeff) {
@@ -1576,6 +1721,9 @@ MGPlan *mg_create(int nx, int ny, int nz, double dx, double dy, double dz, int b
     P->npart = nblocks3(nx, ny, nz);
     if (P->npart < 4 * flat_blocks((int)n0)) P->npart = 4 * flat_blocks((int)n0);
     if (P->npart < 4 * 2048) P->npart = 4 * 2048;
+    // three sums per block of the terrain finest level's last pass (two levels a chunk at least)
+    const int npt = 3 * ((nx + 63) / 64) * ((ny + RBC_BY - 1) / RBC_BY) * ((nz + 1) / 2);
+    if (P->coeff && prec == 0 && P->npart < npt) P->npart = npt;
     if (hipMalloc(&P->part, sizeof(double) * P->npart) != hipSuccess) return fail("mg: allocation failed");
     if (hipMalloc(&P->part2, sizeof(double) * 2048) != hipSuccess) return fail("mg: allocation failed");
     if (hipMalloc(&P->scal, sizeof(double) * MG_NSCAL) != hipSuccess) return fail("mg: allocation failed");
@@ -1607,12 +1755,13 @@ int mg_levels(const MGPlan *P) { return P->nlev; }
 // with ap, z·Ap into scal[3]. r is P->r and z P->z unless given (not
 // aliased). The FP32 V-cycle neither removes r's mean (r is mean-free in a
 // consistent CG to its rounding) nor z's: the CG subtracts Σz/n when it
-// forms the direction (the sums above carry what it needs).
-template <typename T>
+// forms the direction (the sums above carry what it needs). A red-black
+// cycle on an open operator leaves z's mean in likewise.
 // store_z false: z is not written (the caller forms it again from φ with
 // cg_dir_phi_kernel)
 // rsum_in_part: P->part[fb .. 2fb) holds the block sums of r in sum_kernel's
 // layout (cg_update_kernel's second component), so r's mean needs no pass
+template <typename T>
 static void precond(MGPlan *P, hipStream_t st, const double *ap = nullptr, const double *rin = nullptr,
                     double *zout = nullptr, bool store_z = true, bool rsum_in_part = false) {
     MGLevelH &h = P->L[0];
@@ -1621,34 +1770,31 @@ static void precond(MGPlan *P, hipStream_t st, const double *ap = nullptr, const
     const double *r = rin ? rin : P->r;
     double *z = zout ? zout : P->z;
     const bool lean = P->prec != 0;
-    // the mean of r, then b = r − m (the FP64 terrain finest level reads r
-    // and m in place: its kernels are the only readers of b on that level)
-    const bool defer = !lean && sizeof(T) == 8 && P->gen0;
+    const bool rb = rb_cycle(P) && P->nlev > 1;
+    // the mean of r, then b = r − m
     if (!lean && rsum_in_part) finalize_to(P, st, P->scal + 7, P->part + fb, fb, 1.0 / n);
     else if (!lean) mean_to<double>(P, st, r, n, 7);
-    if (defer)
-        P->b0 = P->b0split ? (const double *)h.b : r;  // (b0split: the colour-split copy of r in h.b)
-    else
-        hipLaunchKernelGGL(load_rhs_kernel<T>, dim3(stream_blocks(n)), dim3(RB), 0, st, (T *)h.b, r, n,
-                           lean ? (const double *)nullptr : (const double *)(P->scal + 7));
-    if (!(jacobi_from_zero(P) && P->nlev > 1) && !(defer && rb_tf_from_zero(P)))
+    hipLaunchKernelGGL(load_rhs_kernel<T>, dim3(stream_blocks(n)), dim3(RB), 0, st, (T *)h.b, r, n,
+                       lean ? (const double *)nullptr : (const double *)(P->scal + 7));
+    if (!(jacobi_from_zero(P) && P->nlev > 1) && !rb)
         hipLaunchKernelGGL(zero_kernel<T>, dim3(stream_blocks(n)), dim3(RB), 0, st, (T *)h.phi, n);
-    // the FP64 terrain cycle leaves φ's last mean (slot 4) for z to remove
-    // (one level: the coarsest solve removes φ's mean itself)
-    const bool zdefer = defer && P->nlev > 1;
-    vcycle<T>(P, st, 0, true, zdefer);
-    P->b0 = nullptr;
-    if (zdefer) {
-        hipLaunchKernelGGL(sum_kernel<T>, dim3(fb), dim3(RB), 0, st, (const T *)h.phi, n, P->part,
-                           (const double *)(P->scal + 4), split0<T>(P));
-        finalize_to(P, st, P->scal + 8, P->part, fb, 1.0 / n);
-    } else if (!lean) {
+    vcycle<T>(P, st, 0, true);
+    const double *m2 = nullptr;
+    if (!lean && !rb) {
         mean_to<T>(P, st, (const T *)h.phi, n, 8);
+        m2 = P->scal + 8;
     }
     hipLaunchKernelGGL(store_rz_kernel<T>, dim3(fb), dim3(RB), 0, st, store_z ? z : (double *)nullptr, (const T *)h.phi, r, n,
-                       lean ? (const double *)nullptr : (const double *)(P->scal + 8), P->part, fb, ap,
-                       zdefer ? (const double *)(P->scal + 4) : (const double *)nullptr, split0<T>(P));
+                       m2, P->part, fb, ap);
     finalize_multi_to(P, st, P->scal, P->part, fb, ap ? 4 : 3);
+}
+
+// the FP64 terrain cycle inside the CG: r in place as the finest right-hand
+// side (colour-split), the sums of (r·z, z, r), z = φ, from the last pass
+static void precond_split(MGPlan *P, hipStream_t st) {
+    int nb = 0;
+    vcycle<double>(P, st, 0, true, false, &nb);
+    finalize_multi_to(P, st, P->scal, P->part, nb, 3);
 }
 
 // the FP32 V-cycle's preconditioning inside the fused CG: the level-0
@@ -1659,7 +1805,7 @@ static void precond_fused(MGPlan *P, hipStream_t st, const double *ap) {
     MGLevelH &h = P->L[0];
     const int n = h.nx * h.ny * h.nz;
     const int fb = flat_blocks(n);
-    if (!(jacobi_from_zero(P) && P->nlev > 1))
+    if (!(jacobi_from_zero(P) && P->nlev > 1) && !(rb_cycle(P) && P->nlev > 1))
         hipLaunchKernelGGL(zero_kernel<T>, dim3(stream_blocks(n)), dim3(RB), 0, st, (T *)h.phi, n);
     vcycle<T>(P, st, 0, true);
     hipLaunchKernelGGL(rz_sums_kernel<T>, dim3(fb), dim3(RB), 0, st, (const T *)h.phi, (const double *)P->r, ap, n,
@@ -1692,23 +1838,21 @@ static int pcg_run(MGPlan *P, hipStream_t st, const FCGOp *op, double tol, doubl
     const int fb = flat_blocks(n), sb = stream_blocks(n);
     const double dn = (double)n;
     const bool fused = P->prec != 0;
-    // the FP64 cycle's z = (φ − m1) − m2: m1 the mean the terrain cycle leaves in slot 4
-    const double *zm1 = (!fused && P->gen0 && P->nlev > 1) ? (const double *)(P->scal + 4) : (const double *)nullptr;
+    const bool split = !fused && P->half0 != 0;  // the FP64 terrain cycle: r lives in the finest b, colour-split
+    // the FP64 cycle's z = φ − m2
+    const double *m2 = !split && !(rb_cycle(P) && P->nlev > 1) ? (const double *)(P->scal + 8) : (const double *)nullptr;
     double rnorm = *rnorm_io;
     int iters = 0, status = rnorm <= tol * bnorm ? 0 : 1;
-    // the FP64 terrain cycle reads r colour-split from h.b: a copy for the
-    // first cycle, then the update kernel's
-    const bool bsplit = !fused && P->half0 != 0;
-    if (status != 0 && bsplit) {
+    if (status != 0 && split)
         hipLaunchKernelGGL(split_copy_kernel, dim3(sb), dim3(RB), 0, st, (double *)h.b, (const double *)P->r, n,
                            split0<double>(P));
-        P->b0split = 1;
-    }
     if (status != 0) {
         if (fused) {
             hipLaunchKernelGGL(load_rhs_kernel<float>, dim3(sb), dim3(RB), 0, st, (float *)h.b, (const double *)P->r,
                                n, (const double *)nullptr);
             precond_fused<float>(P, st, nullptr);
+        } else if (split) {
+            precond_split(P, st);
         } else {
             precond<double>(P, st, nullptr, nullptr, nullptr, false);
         }
@@ -1718,8 +1862,7 @@ static int pcg_run(MGPlan *P, hipStream_t st, const FCGOp *op, double tol, doubl
                                (const double *)P->scal, 1);
         else
             hipLaunchKernelGGL(cg_dir_phi_kernel<double>, dim3(sb), dim3(RB), 0, st, P->p, (const double *)h.phi, n,
-                               (const double *)P->scal, 1, zm1, (const double *)(P->scal + 8), (double *)nullptr,
-                               split0<double>(P));
+                               (const double *)P->scal, 1, m2, (double *)nullptr, split0<double>(P));
     }
     const int nb3 = nblocks3(h.nx, h.ny, h.nz);
     while (status != 0 && iters < maxit) {
@@ -1745,9 +1888,9 @@ static int pcg_run(MGPlan *P, hipStream_t st, const FCGOp *op, double tol, doubl
             hipLaunchKernelGGL(cg_update_rhs_kernel<float>, dim3(fb), dim3(RB), 0, st, P->r, (const double *)P->Ap,
                                (float *)h.b, (const double *)P->scal, n, P->part, fb);
         else
-            hipLaunchKernelGGL(cg_update_kernel, dim3(fb), dim3(RB), 0, st, (double *)nullptr, P->r, (const double *)P->p,
+            hipLaunchKernelGGL(cg_update_kernel, dim3(fb), dim3(RB), 0, st, split ? (double *)h.b : P->r,
                                (const double *)P->Ap, (const double *)(P->scal + S_ALPHA), n, P->part, fb,
-                               bsplit ? (double *)h.b : (double *)nullptr, split0<double>(P));
+                               split0<double>(P));
         finalize_multi_to(P, st, P->scal + S_R2, P->part, fb, 2);
         double sc[S_BREAK - S_R2 + 1];
         read_scals(st, P->scal + S_R2, sc, S_BREAK - S_R2 + 1);
@@ -1761,6 +1904,7 @@ static int pcg_run(MGPlan *P, hipStream_t st, const FCGOp *op, double tol, doubl
             break;
         }
         if (fused) precond_fused<float>(P, st, P->Ap);
+        else if (split) precond_split(P, st);
         else precond<double>(P, st, nullptr, nullptr, nullptr, false, true);
         hipLaunchKernelGGL(cg_beta_kernel, dim3(1), dim3(1), 0, st, P->scal, dn, (int)fused);
         if (fused)
@@ -1768,9 +1912,8 @@ static int pcg_run(MGPlan *P, hipStream_t st, const FCGOp *op, double tol, doubl
                                (const double *)P->scal, 0);
         else
             hipLaunchKernelGGL(cg_dir_phi_kernel<double>, dim3(sb), dim3(RB), 0, st, P->p, (const double *)h.phi, n,
-                               (const double *)P->scal, 0, zm1, (const double *)(P->scal + 8), P->x, split0<double>(P));
+                               (const double *)P->scal, 0, m2, P->x, split0<double>(P));
     }
-    P->b0split = 0;
     *iters_out = iters;
     *rnorm_io = rnorm;
     return status;
@@ -1794,11 +1937,9 @@ int mg_pcg_solve(MGPlan *P, hipStream_t st, double *xout, const double *bin, dou
     double mb = read_scal(st, P->scal + 9);
     hipLaunchKernelGGL(shift_copy_kernel, dim3(stream_blocks(n)), dim3(RB), 0, st, P->r, (const double *)b, n, mb);
     hipLaunchKernelGGL(fill_kernel, dim3(stream_blocks(n)), dim3(RB), 0, st, P->x, n, 0.0);
-    hipLaunchKernelGGL(fill_kernel, dim3(stream_blocks(n)), dim3(RB), 0, st, P->z, n, 0.0);
-    // b2 = Σ r² (z = 0): the update kernel with α = 0
-    hipLaunchKernelGGL(cg_update_kernel, dim3(fb), dim3(RB), 0, st, P->x, P->r, (const double *)P->z,
-                       (const double *)P->z, (const double *)nullptr, n, P->part, fb, (double *)nullptr,
-                       SplitMap{0, 0, 0, -1, -1});
+    // b2 = Σ r²: the update kernel with α = 0
+    hipLaunchKernelGGL(cg_update_kernel, dim3(fb), dim3(RB), 0, st, P->r, (const double *)P->r, (const double *)nullptr, n,
+                       P->part, fb, SplitMap{0, 0, 0, -1, -1});
     finalize_multi_to(P, st, P->scal + 12, P->part, fb, 2);
     double b2 = read_scal(st, P->scal + 12);
     double bnorm = sqrt(b2);
@@ -1862,9 +2003,9 @@ int mg_pcg_solve_op(MGPlan *P, hipStream_t st, const FCGOp &op, double *xout, co
     double rnorm = sqrt(read_scal(st, P->scal + 12));
     if (r0_out) *r0_out = rnorm;
     int iters = 0;
-    // the FP64 terrain preconditioner keeps its finest φ colour-split for the solve
-    // (even extents: the finest prolongation is then prolong_col_kernel)
-    P->half0 = (P->gen0 && P->prec == 0 && h.nx % 2 == 0 && h.ny % 2 == 0 && h.nz % 2 == 0) ? (uint32_t)(n / 2) : 0u;
+    // the FP64 terrain preconditioner keeps its finest φ and b colour-split for
+    // the solve (a level with a coarser one has even extents)
+    P->half0 = P->gen0 && P->nlev > 1 ? (uint32_t)(n / 2) : 0u;
     const int status = pcg_run(P, st, &op, tol, bnorm, maxit, &iters, &rnorm);
     P->half0 = 0;
     mean_to<double>(P, st, P->x, n, 13);
@@ -1896,7 +2037,10 @@ void mg_set_terrain_coef(MGPlan *P, const TFWView &v) {
     const bool dims = P->coeff && P->L[0].nx == v.Nx && P->L[0].ny == v.Ny && P->L[0].nz == v.Nz;
     P->gm = make_tfm<double>(v);
     P->gmf = make_tfm<float>(v);
-    P->gen0 = dims && P->prec == 0 && P->smoother == 0;
+    // ρ̄ > 0 and J > 0 on every face, so every diagonal is negative
+    P->open = P->open || dims;
+    P->gen0 = dims && P->prec == 0 && P->smoother == 0 && (P->nlev == 1 || (P->nu1 >= 1 && P->nu2 >= 1));
+    P->kc0 = chunk_levels(((v.Nx + 63) / 64) * ((v.Ny + RBC_BY - 1) / RBC_BY), v.Nz, RBC_KC, RBC_FILL, 3, 2);
     P->gen0f = dims && P->prec == 1 && P->smoother == 1;
 }
 
@@ -1992,7 +2136,7 @@ void mg_precond_apply(MGPlan *P, hipStream_t st, double *z, const double *r) {
         r = P->r;
     }
     if (P->prec == 0) precond<double>(P, st, nullptr, r, z); else precond<float>(P, st, nullptr, r, z);
-    if (P->prec != 0) {  // the FP32 cycle leaves z's mean in: remove it here
+    if (P->prec != 0 || (rb_cycle(P) && P->nlev > 1)) {  // the cycle leaves z's mean in: remove it here
         mean_to<double>(P, st, z, n, 8);
         hipLaunchKernelGGL(shift_kernel<double>, dim3(stream_blocks(n)), dim3(RB), 0, st, z, n, P->scal + 8);
     }
