@@ -1122,13 +1122,13 @@ struct aeo_tf_stepper {
 static void tfw_apply_cb(void *ctx, hipStream_t st, double *out, const double *x) {
     aeo_tf_stepper *h = (aeo_tf_stepper *)ctx;
     Timed tm("tf_apply");
-    launch_tfw_apply_march(st, h->v, h->bx, h->by, h->rs, out, x, nullptr, 0);
+    launch_tfw_apply_march(st, h->v, out, x, nullptr, 0);
 }
 // L x with the block sums of x·Lx (−1: too many blocks for the slots, no sums)
 static int tfw_apply_dot_cb(void *ctx, hipStream_t st, double *out, const double *x, double *part, int cap) {
     aeo_tf_stepper *h = (aeo_tf_stepper *)ctx;
     Timed tm("tf_apply");
-    return launch_tfw_apply_march(st, h->v, h->bx, h->by, h->rs, out, x, part, cap);
+    return launch_tfw_apply_march(st, h->v, out, x, part, cap);
 }
 
 extern "C" int aeo_tf_stepper_create(aeo_terrain *t, const aeo_tf_params *p, aeo_tf_stepper **out) {

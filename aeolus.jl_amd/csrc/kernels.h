@@ -215,13 +215,10 @@ int launch_tfw_tendency(hipStream_t st, const TFWView &v, int scheme, int f32, d
 void launch_tfw_halos(hipStream_t st, const TFWView &v, double *u, double *vv, double *w, double *th);
 void launch_tfw_div(hipStream_t st, const TFWView &v, const double *bx, const double *by, const double *rs,
                     double *out, const double *u, const double *vv, const double *w);
-void launch_tfw_apply(hipStream_t st, const TFWView &v, const double *bx, const double *by, const double *rs,
-                      double *gx, double *gy, double *gw, double *out, const double *x);
 void launch_tfw_grad(hipStream_t st, const TFWView &v, const double *bx, const double *by, const double *rs,
                      double *gx, double *gy, double *gw, const double *x);
 // L x in one column-marching pass; with part, the block sums of x·(Lx); returns the block count
-int launch_tfw_apply_march(hipStream_t st, const TFWView &v, const double *bx, const double *by, const double *rs,
-                           double *out, const double *x, double *part, int cap);
+int launch_tfw_apply_march(hipStream_t st, const TFWView &v, double *out, const double *x, double *part, int cap);
 void launch_tfw_correct(hipStream_t st, const TFWView &v, const double *bx, const double *by, const double *rs,
                         double *u, double *vv, double *w, double *th, double *p, const double *us, const double *vs,
                         const double *ws, const double *tn, const double *u0, const double *v0, const double *w0,
