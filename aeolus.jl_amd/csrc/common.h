@@ -102,7 +102,8 @@ __device__ __forceinline__ uint32_t lin(int i, int j, int k, int sx, int sy) {
 }
 
 // ---------------------------------------------------------------------------
-// Reconstructions, in the reference's evaluation order. The library is built
+// Reconstructions, in the reference's evaluation order (WENO-Z5 excepted: its
+// own form below). The library is built
 // with -ffp-contract=off; the reconstructions (and the tendency kernel, which
 // turns the same pragma on for its file) let the compiler fuse a multiply and
 // an add into one FMA: each fused pair rounds once instead of twice (at most
@@ -158,18 +159,17 @@ template <typename T> __device__ __forceinline__ T b4_m1(T v1, T v2, T v3, T v4)
 }
 // General divisions of the nonlinear weights. The divisors are β + ε ≥ ε > 0
 // or sums of positive weights: positive, normal and finite.
-//  FP64: a · (1/b) with 1/b from v_rcp_f64 refined by two Newton steps
-//        (e = 1 − b·r, r ← r + r·e): within 1 ulp of the correctly rounded
-//        quotient (checked on 2e7 random pairs with the initial reciprocal
-//        perturbed by up to 2^-22); the tests hold the kernels to 1e-12.
+//  FP64: a · (1/b) with 1/b from v_rcp_f64 refined by one third-order step
+//        (e = 1 − b·r, r ← r + r·(e + e²)): within 1.49 ulp of the correctly
+//        rounded quotient, as with two Newton steps of one instruction more
+//        (checked on 2e7 random pairs with the initial reciprocal perturbed
+//        by up to 2^-22: e³ = 2^-66); the tests hold the kernels to 1e-12.
 //  FP32: a · v_rcp_f32(b) (≤ 1 ulp of 1/b), stated against the FP64 oracle.
 template <typename T> __device__ __forceinline__ T qdiv(T a, T b);
 template <> __device__ __forceinline__ double qdiv<double>(double a, double b) {
     double r = __builtin_amdgcn_rcp(b);
-    double e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(e, r, r);
-    e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(e, r, r);
+    const double e = __builtin_fma(-b, r, 1.0);
+    r = __builtin_fma(__builtin_fma(e, e, e), r, r);
     return a * r;
 }
 template <> __device__ __forceinline__ float qdiv<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
@@ -195,22 +195,49 @@ template <typename T> __device__ __forceinline__ T b5_m4(T v1, T v2, T v3, T v4,
                     div24<T>((((v1 - T(4) * v2) + T(6) * v3) - T(4) * v4) + v5));
 }
 
-// _weno_z5_left, src/AdvectionSchemes.jl:240-255
+// The three ratios t_k = τ/b_k of the Z weights. FP64: one reciprocal, of the
+// product (b ≥ 4ε² = 2e-31, so the product is at least 8e-93, and finite for
+// fields below 1e50), and five products in place of two more refined
+// reciprocals; each ratio is within 5 roundings. FP32 has no such range:
+// three hardware reciprocals.
+template <typename T>
+__device__ __forceinline__ void z_ratios(T tau, T b0, T b1, T b2, T &t0, T &t1, T &t2) {
+    if constexpr (sizeof(T) == 8) {
+        const T b01 = b0 * b1, r = qdiv<T>(tau, b01 * b2);
+        t0 = (b1 * b2) * r;
+        t1 = (b0 * b2) * r;
+        t2 = b01 * r;
+    } else {
+        t0 = qdiv<T>(tau, b0);
+        t1 = qdiv<T>(tau, b1);
+        t2 = qdiv<T>(tau, b2);
+    }
+}
+
+// _weno_z5_left, src/AdvectionSchemes.jl:240-255, from the differences
+// e_m = v_{m+1} − v_m: the smoothness indicators (times 4, with ε² times 4)
+// and the candidates less v3 (times 6) depend on nothing else, and the face is
+// v3 + Σ a_k (6 (q_k − v3)) / (6 Σ a_k). The reconstruction bounds the
+// advection kernels: of the tiled FP64 kernel's VALU instructions per
+// wave and level this form leaves 1143 where the indicators and candidates
+// from the values, each ratio by its own reciprocal, took 1439; it rounds
+// relative to the variation, not the value. 256×256×128 RK3 stage 606 → 506 us
+// (FP32 289 → 265), the limited tracer's two passes 316 → 278.
 template <int P, typename T>
 __device__ __forceinline__ T weno_z5(T v1, T v2, T v3, T v4, T v5) {
-    // the candidate polynomials times 6: the common 1/6 is taken once, in the
-    // normalisation (Σ ω_k q_k = Σ a_k (6 q_k) / (6 Σ a_k)), instead of three
-    // exact divisions by 6 (12 FP64 instructions per face fewer)
-    T q0 = (T(2) * v1 - T(7) * v2) + T(11) * v3;
-    T q1 = (-v2 + T(5) * v3) + T(2) * v4;
-    T q2 = (T(2) * v3 + T(5) * v4) - v5;
-    T b0 = b3_m2<T>(v1, v2, v3), b1 = b3_m1<T>(v2, v3, v4), b2 = b3_p0<T>(v3, v4, v5);
-    const T eps = Eps<T>::v * Eps<T>::v;
-    T tau = fabs(b0 - b2);
-    T a0 = T(1.0 / 10.0) * (T(1) + ipow<P>(qdiv<T>(tau, b0 + eps)));
-    T a1 = T(6.0 / 10.0) * (T(1) + ipow<P>(qdiv<T>(tau, b1 + eps)));
-    T a2 = T(3.0 / 10.0) * (T(1) + ipow<P>(qdiv<T>(tau, b2 + eps)));
-    return qdiv<T>((a0 * q0 + a1 * q1) + a2 * q2, T(6) * ((a0 + a1) + a2));
+    const T e1 = v2 - v1, e2 = v3 - v2, e3 = v4 - v3, e4 = v5 - v4;
+    const T s0 = e2 - e1, s1 = e3 - e2, s2 = e4 - e3;                      // second differences
+    const T f0 = T(3) * e2 - e1, f1 = e2 + e3, f2 = T(3) * e3 - e4;        // twice the slopes at v3
+    const T c = T(13.0 / 3.0), eps = T(4) * Eps<T>::v * Eps<T>::v;
+    const T b0 = f0 * f0 + ((c * s0) * s0 + eps), b1 = f1 * f1 + ((c * s1) * s1 + eps),
+            b2 = f2 * f2 + ((c * s2) * s2 + eps);
+    T t0, t1, t2;
+    z_ratios<T>(fabs(b0 - b2), b0, b1, b2, t0, t1, t2);
+    const T a0 = T(1.0 / 10.0) + T(1.0 / 10.0) * ipow<P>(t0);
+    const T a1 = T(6.0 / 10.0) + T(6.0 / 10.0) * ipow<P>(t1);
+    const T a2 = T(3.0 / 10.0) + T(3.0 / 10.0) * ipow<P>(t2);
+    const T p0 = T(5) * e2 - T(2) * e1, p1 = T(2) * e3 + e2, p2 = T(4) * e3 - e4;
+    return v3 + qdiv<T>((a0 * p0 + a1 * p1) + a2 * p2, T(6) * ((a0 + a1) + a2));
 }
 // _weno_z7_left, src/AdvectionSchemes.jl:284-303
 template <int P, typename T>
