@@ -36,40 +36,6 @@ namespace aeo {
 // ---------------------------------------------------------------------------
 // the tendencies + predictor (+ the θ stage combination)
 // ---------------------------------------------------------------------------
-// the face value between cells c and c+1 from d at element offsets o + m·st,
-// o the offset of cell c − 2: centred, or WENO-Z5 (p = 2) upwinded on `vel`
-template <int S, typename TC>
-__device__ __forceinline__ TC tf_face(const double *__restrict__ d, uint32_t o, uint32_t st, TC vel) {
-    if constexpr (S == SCH_CENTERED) {
-        return ((TC)d[o + 2 * st] + (TC)d[o + 3 * st]) / TC(2);
-    } else {
-        const TC a0 = (TC)d[o], a1 = (TC)d[o + st], a2 = (TC)d[o + 2 * st], a3 = (TC)d[o + 3 * st],
-                 a4 = (TC)d[o + 4 * st], a5 = (TC)d[o + 5 * st];
-        const bool up = vel >= TC(0);
-        return weno_z5<2, TC>(up ? a0 : a5, up ? a1 : a4, up ? a2 : a3, up ? a3 : a2, up ? a4 : a1);
-    }
-}
-
-// the face value minus a base value q0, reconstructed from the stencil's
-// differences to q0 (formed in FP64) in TC: centred and WENO-Z5 are
-// translation invariant, so this is tf_face − q0 with TC's relative
-// precision on the local variation instead of on the value
-template <int S, typename TC>
-__device__ __forceinline__ TC tf_face_dev(const double *__restrict__ d, uint32_t o, uint32_t st, TC vel, double q0) {
-    if constexpr (S == SCH_CENTERED) {
-        return ((TC)(d[o + 2 * st] - q0) + (TC)(d[o + 3 * st] - q0)) / TC(2);
-    } else {
-        const TC a0 = (TC)(d[o] - q0), a1 = (TC)(d[o + st] - q0), a2 = (TC)(d[o + 2 * st] - q0),
-                 a3 = (TC)(d[o + 3 * st] - q0), a4 = (TC)(d[o + 4 * st] - q0), a5 = (TC)(d[o + 5 * st] - q0);
-        const bool up = vel >= TC(0);
-        return weno_z5<2, TC>(up ? a0 : a5, up ? a1 : a4, up ? a2 : a3, up ? a3 : a2, up ? a4 : a1);
-    }
-}
-
-#ifndef TFW_TEND_CH
-#define TFW_TEND_CH 32  // levels per thread of the marching tendency kernel
-#endif
-
 // the face value of six values a0..a5 along the line (the face between a2
 // and a3): centred, or WENO-Z5 upwinded on `vel`
 template <int S, typename TC>
@@ -82,227 +48,420 @@ __device__ __forceinline__ TC tf_face6(TC a0, TC a1, TC a2, TC a3, TC a4, TC a5,
     }
 }
 
-// The tendencies + predictor marching up the column: a thread owns the
-// column (i, j) and CH levels. Per level it computes what is new there and
-// carries the rest from the level below:
-//   - the vertical fluxes of u, v, w, θ through the face below a level are
-//     the ones through the face above the level before (same mass flux, same
-//     stencil), so one vertical reconstruction per field and level;
-//   - Ω on the faces of the own column and of the columns i − 1 and j − 1;
-//   - each field's six values along σ stay in registers (one load per level);
-//   - the reference densities of the fifteen (column, level kind) families
-//     the fluxes use follow ρ̄(k+1) = ρ̄(k)·e^{−Δσ J/Hs} (J of the column),
-//     from one exp per family at the chunk's start, in FP64.
-// The buoyancy about θ̄(z) = θ0 + Γz at the w-face follows _anelastic_buoyancy
-// (src/Anelastic.jl:1352-1360), formed in FP64 whatever TC (θ_face − θ̄ is a
-// small difference of values near 300 K).
-template <int S, typename TC, int CH>
-__global__ void __launch_bounds__(256, sizeof(TC) == 4 ? 2 : 1) tfw_tendency_march_kernel(double *__restrict__ us, double *__restrict__ vs,
-                                                                  double *__restrict__ ws, double *__restrict__ tn,
-                                                                  const double *__restrict__ u,
-                                                                  const double *__restrict__ v,
-                                                                  const double *__restrict__ w,
-                                                                  const double *__restrict__ th,
-                                                                  const double *__restrict__ th0, TFM<TC> m,
-                                                                  double dt, double ca, double cb, int combine,
-                                                                  int raw) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + m.H;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + m.H;
-    if (i >= m.H + m.Nx || j >= m.H + m.Ny) return;
-    const int H = m.H;
-    const int kb = H + (int)blockIdx.z * CH;
-    const int ke = kb + CH < H + m.Nz ? kb + CH : H + m.Nz;
+// The tendencies + predictor: a block owns 64 × BY columns and marches a chunk
+// of levels, each face flux of the x-y plane computed once.
+//   - Every thread keeps its column's values of the four fields over the
+//     reach of the σ-stencil (k − 2 .. k + 3) in registers, one load a level;
+//     the σ-faces read these, and a level's top fluxes are the next one's
+//     bottom fluxes.
+//   - The block's tile with a 3-cell halo is in LDS (u, v, w at levels k and
+//     k + 1, θ at k), the halo loaded a level ahead; the x- and y-faces read
+//     it. A cell computes its west and south fluxes into LDS; its east and
+//     north ones are its neighbours'. The last row's north faces take one
+//     wave per field, the rows' last east faces 4·BY lanes.
+//   - Ω on the faces k + 1 is computed once per column into LDS (and for the
+//     row and the column of columns before the block), for the averages that
+//     carry u and v up.
+//   - ρ̄ J of the points the fluxes live at follows its ratio per (half) level
+//     of its column, from one exp per column at the chunk's start, in FP64.
+// Two barriers a level: after the tile is written, and after the x-y fluxes and
+// Ω are. The buoyancy about θ̄(z) = θ0 + Γz at the w-face follows
+// _anelastic_buoyancy (src/Anelastic.jl:1352-1360), formed in FP64 whatever TC
+// (θ_face − θ̄ is a small difference of values near 300 K).
+//
+// What bounds it is the FP64 VALU: about 13 WENO faces a cell, where a thread
+// per column that evaluates both faces of each direction has 20 and 15
+// density families, and at one wave per SIMD (over 256 registers) issued
+// half the time. At 512×512×256 7.95 → 3.70 ms, 320×256×160 with FP32
+// fluxes 1.37 → 0.70, 96×96×48 250 → 49 us (chunks of 32 levels on every grid
+// before). Two waves per SIMD (225 registers): three for the FP32 form spill
+// (0.80 ms); blocks of 8 rows, one per CU: 3.79, 0.67 ms, 46 us.
+#pragma clang fp contract(fast)
+constexpr int TFT_BY = 4;
+constexpr int TFT_KC = 32;     // most levels per chunk
+constexpr int TFT_FILL = 512;  // blocks a round: two per CU
+template <int S, typename TC, int BY>
+__global__ void __launch_bounds__(64 * BY, 2)
+    tfw_tendency_tile_kernel(double *__restrict__ us, double *__restrict__ vs, double *__restrict__ ws,
+                             double *__restrict__ tn, const double *__restrict__ u, const double *__restrict__ v,
+                             const double *__restrict__ w, const double *__restrict__ th,
+                             const double *__restrict__ th0, TFM<TC> m, double dt, double ca, double cb, int combine,
+                             int raw, int kc) {
+    constexpr int R = 3, RL = 2, NW = 6;
+    constexpr int TW = 64 + 2 * R, TH = BY + 2 * R, TN = TW * TH, NT = 64 * BY;
+    constexpr int NHALO = TN - NT, NHP = (NHALO + NT - 1) / NT;
+    constexpr bool DEV = sizeof(TC) == 4;  // θ's fluxes about the cell's own θ
+    constexpr int XN = BY * 65, YN = (BY + 1) * 64;
+    __shared__ TC tl[6 * TN];                // u, v, w: the levels of even and odd k − k0
+    __shared__ double ts[TN];                // θ
+    __shared__ TC xs[4 * XN], ys[4 * YN];    // west fluxes [F][row][c], south fluxes [F][r][lane]
+    __shared__ TC xm[DEV ? XN : 1], ym[DEV ? YN : 1];  // θ's mass fluxes
+    __shared__ TC om[(BY + 1) * 65];         // Ω(k + 1) of column (i0 − 1 + c, jb − 1 + r)
+    int bx, by, bz;
+    xcd_block3(bx, by, bz);
+    const int H = m.H, lane = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + lane;
+    const int wv = __builtin_amdgcn_readfirstlane(ty);
+    const int i0 = H + bx * 64, jb = H + by * BY, i = i0 + lane, j = jb + ty;
+    const int k0 = H + bz * kc, k1 = min(k0 + kc, H + m.Nz);
+    const int ilast = min(i0 + 63, H + m.Nx - 1), jlast = min(jb + BY - 1, H + m.Ny - 1);
+    const bool ok = i <= ilast && j <= jlast;          // computes its cell
+    const bool inb = i <= ilast + R && j <= jlast + R;  // its column feeds the tile
+    const int at = (ty + R) * TW + lane + R;
     const int sxi = m.sx;
-    const int sxyi = m.sx * m.sy;
-    const uint32_t sx = (uint32_t)sxi, sxy = (uint32_t)sxyi;
-    // FP64 plane values and the density families
-    const double *hp = m.h;
-    auto hd = [&](int a, int b) -> double { return hp[a + sxi * b]; };
+    const uint32_t sx = (uint32_t)m.sx, sxy = (uint32_t)m.sx * (uint32_t)m.sy;
     const double Hl = (double)m.Hl, iHl = 1.0 / Hl, dz = (double)m.dz, iHs = (double)m.iHs, rho0 = (double)m.rho0;
-    auto hxfd = [&](int a, int b) -> double { return (hd(a, b) + hd(a - 1, b)) / 2; };
-    auto hyfd = [&](int a, int b) -> double { return (hd(a, b) + hd(a, b - 1)) / 2; };
-    auto hxyd = [&](int a, int b) -> double { return (hxfd(a, b) + hxfd(a, b - 1)) / 2; };
-    struct Fam {
-        double r, q;
-    };
-    // ρ̄ at σ-level index kk (σ = (kk − H + off)·dz) of a column with surface hs
-    auto fam = [&](double hs, int kk, double off) -> Fam {
-        const double J = (Hl - hs) * iHl;
-        return Fam{rho0 * exp(-(hs + ((double)(kk - H) + off) * dz * J) * iHs), exp(-dz * J * iHs)};
-    };
-    // centre-level families at the chunk's first level kb
-    Fam fc00 = fam(hd(i, j), kb, 0.5), fcm0 = fam(hd(i - 1, j), kb, 0.5), fc0m = fam(hd(i, j - 1), kb, 0.5);
-    Fam fx00 = fam(hxfd(i, j), kb, 0.5), fx10 = fam(hxfd(i + 1, j), kb, 0.5);
-    Fam fy00 = fam(hyfd(i, j), kb, 0.5), fy01 = fam(hyfd(i, j + 1), kb, 0.5);
-    Fam fxy00 = fam(hxyd(i, j), kb, 0.5), fxy01 = fam(hxyd(i, j + 1), kb, 0.5), fxy10 = fam(hxyd(i + 1, j), kb, 0.5);
-    // face-level families at the face kb (the level's bottom face)
-    Fam fs00 = fam(hd(i, j), kb, 0.0), fxs00 = fam(hxfd(i, j), kb, 0.0), fxs10 = fam(hxfd(i + 1, j), kb, 0.0);
-    Fam fys00 = fam(hyfd(i, j), kb, 0.0), fys01 = fam(hyfd(i, j + 1), kb, 0.0);
-    // ρ̄ at the centre below the chunk (w's lower flux)
-    double rc_below = fc00.r / fc00.q;
 
-    auto U = [&](uint32_t c, int di, int dj, int dk) { return (TC)u[c + di + sxi * dj + sxyi * dk]; };
-    auto V = [&](uint32_t c, int di, int dj, int dk) { return (TC)v[c + di + sxi * dj + sxyi * dk]; };
-    // Ω at the σ-face kk of column (i + di, j + dj)
-    auto Om = [&](int di, int dj, int kk) -> TC {
-        if (kk == H || kk == H + m.Nz) return TC(0);
-        const uint32_t c = lin(i + di, j + dj, kk, m.sx, m.sy);
-        const TC ucm = (U(c, 0, 0, -1) + U(c, 1, 0, -1)) / TC(2), uck = (U(c, 0, 0, 0) + U(c, 1, 0, 0)) / TC(2);
-        const TC vcm = (V(c, 0, 0, -1) + V(c, 0, 1, -1)) / TC(2), vck = (V(c, 0, 0, 0) + V(c, 0, 1, 0)) / TC(2);
-        const TC ub = TC(0.5) * ucm + TC(0.5) * uck, vb = TC(0.5) * vcm + TC(0.5) * vck;
-        return (TC)w[c] + (m.jsx(i + di, j + dj, kk) * ub + m.jsy(i + di, j + dj, kk) * vb);
+    // surfaces of the columns the fluxes live on
+    auto hd = [&](int a, int b) -> double { return m.h[a + sxi * b]; };
+    auto hxd = [&](int a, int b) -> double { return (hd(a, b) + hd(a - 1, b)) / 2; };
+    auto hyd = [&](int a, int b) -> double { return (hd(a, b) + hd(a, b - 1)) / 2; };
+    auto hxyd = [&](int a, int b) -> double { return (hxd(a, b) + hxd(a, b - 1)) / 2; };
+    auto Jd = [&](double hs) -> double { return (Hl - hs) * iHl; };
+    // ρ̄ at σ = (k0 − H + off)·dz over surface hs, and its ratio over f levels
+    auto rho = [&](double hs, double off) -> double {
+        return rho0 * exp(-(hs + ((double)(k0 - H) + off) * dz * Jd(hs)) * iHs);
     };
-    const TC J00 = m.J(i, j), Jm0 = m.J(i - 1, j), J0m = m.J(i, j - 1);
-    const TC Jx00 = m.Jx(i, j), Jx10 = m.Jx(i + 1, j), Jy00 = m.Jy(i, j), Jy01 = m.Jy(i, j + 1);
-    const TC Jxy00 = m.Jxy(i, j), Jxy01 = m.Jxy(i, j + 1), Jxy10 = m.Jxy(i + 1, j);
-    // the rolling σ-windows: F(k − 2 .. k + 3) of the own column at level k
-    const uint32_t c0 = lin(i, j, kb, m.sx, m.sy);
-    TC wu[6], wv[6], ww[6];
-    double wt[6];
-    for (int q = 0; q < 6; q++) {
-        const uint32_t cq = c0 + (uint32_t)((q - 2) * sxyi);
-        wu[q] = (TC)u[cq];
-        wv[q] = (TC)v[cq];
-        ww[q] = (TC)w[cq];
-        wt[q] = th[cq];
+    auto ratio = [&](double hs, double f) -> double { return exp(-f * dz * Jd(hs) * iHs); };
+
+    // the halo cells this thread loads: bottom and top R rows, then the left
+    // and right R columns; cells past the last cell + R feed nothing
+    uint32_t hof[NHP];
+    int hat[NHP];
+    bool hv[NHP];
+#pragma unroll
+    for (int p = 0; p < NHP; p++) {
+        const int e = tid + p * NT;
+        int r, c;
+        if (e < 2 * R * TW) {
+            r = e / TW;
+            c = e % TW;
+            if (r >= R) r += BY;
+        } else {
+            const int e2 = e - 2 * R * TW, q = e2 % (2 * R);
+            r = R + e2 / (2 * R);
+            c = q < R ? q : 64 + q;
+        }
+        const int hi = i0 - R + c, hj = jb - R + r;
+        hv[p] = e < NHALO && hi <= ilast + R && hj <= jlast + R;
+        hat[p] = r * TW + c;
+        hof[p] = hv[p] ? lin(hi, hj, 0, m.sx, m.sy) : 0u;
     }
-    // Ω carries: own column at faces kb − 1, kb; columns i − 1 and j − 1 at face kb
-    TC OmB = Om(0, 0, kb - 1), Om0 = Om(0, 0, kb), Omm0 = Om(-1, 0, kb), Om0m = Om(0, -1, kb);
-    // the vertical fluxes through the face kb (the level kb − 1's upper fluxes), from the same stencils
-    // (θ's as its mass flux FBm_t and face value FBf_t; in FP32 the face value
-    // less θ of the level, re-based when the level moves up)
-    TC FBm_t, FBf_t, FB_u, FB_v, FB_w;
-    {
-        const TC Ft = (TC)fs00.r * Om0;
-        const uint32_t oz = c0 - 3 * sxy;
-        FBm_t = Ft;
-        if constexpr (sizeof(TC) == 8)
-            FBf_t = tf_face<S, TC>(th, oz, sxy, Ft);
-        else
-            FBf_t = tf_face_dev<S, TC>(th, oz, sxy, Ft, wt[2]);
-        const TC Wu = (TC)fxs00.r * ((Omm0 + Om0) / TC(2));
-        FB_u = Wu * tf_face<S, TC>(u, oz, sxy, Wu);
-        const TC Wv = (TC)fys00.r * ((Om0m + Om0) / TC(2));
-        FB_v = Wv * tf_face<S, TC>(v, oz, sxy, Wv);
-        // w's: through the centre kb − 1 (between faces kb − 1 and kb)
-        const TC Ww = (TC)rc_below * ((OmB + Om0) / TC(2));
-        FB_w = Ww * tf_face<S, TC>(w, oz, sxy, Ww);
+    const uint32_t cof = inb ? lin(i, j, 0, m.sx, m.sy) : 0u;
+
+    TC win[3][NW];
+    double wt[NW], nxt[4], hal[4][NHP];
+#pragma unroll
+    for (int n = 0; n < NW; n++) {
+        const uint32_t c = cof + (uint32_t)(k0 - 1 - RL + n) * sxy;
+        win[0][n] = inb ? (TC)u[c] : TC(0);
+        win[1][n] = inb ? (TC)v[c] : TC(0);
+        win[2][n] = inb ? (TC)w[c] : TC(0);
+        wt[n] = inb ? th[c] : 0.0;
     }
-    for (int k = kb; k < ke; k++) {
-        const uint32_t c = lin(i, j, k, m.sx, m.sy);
-        // Ω on the faces k + 1
-        const TC Om1 = Om(0, 0, k + 1), Omm1 = Om(-1, 0, k + 1), Om0m1 = Om(0, -1, k + 1);
-        const uint32_t ox = c - 3, oy = c - 3 * sx;
-        const TC rc00 = (TC)fc00.r;
-        // θ
-        TC tt, FTf_t;
-        {
-            const TC FE = (TC)fx10.r * Jx10 * U(c, 1, 0, 0);
-            const TC FW = (TC)fx00.r * Jx00 * U(c, 0, 0, 0);
-            const TC FN = (TC)fy01.r * Jy01 * V(c, 0, 1, 0);
-            const TC FS = (TC)fy00.r * Jy00 * V(c, 0, 0, 0);
-            const TC FT = (TC)(fs00.r * fs00.q) * Om1;
-            if constexpr (sizeof(TC) == 8) {
-                FTf_t = tf_face6<S, TC>(wt[0], wt[1], wt[2], wt[3], wt[4], wt[5], FT);
-                const TC d = ((FE * tf_face<S, TC>(th, ox + 1, 1, FE) - FW * tf_face<S, TC>(th, ox, 1, FW)) * m.idx +
-                              (FN * tf_face<S, TC>(th, oy + sx, sx, FN) - FS * tf_face<S, TC>(th, oy, sx, FS)) * m.idy) +
-                             (FT * FTf_t - FBm_t * FBf_t) * m.idz;
-                tt = TC(0) - d / (rc00 * J00);
-            } else {
-                // the flux form less θ_c·(B u)/(ρJ): B u vanishes to the projection's tolerance, and its
-                // FP32 rounding times θ ≈ 300 K would swamp the tendency of the perturbation
-                const double q0 = wt[2];
-                FTf_t = tf_face6<S, TC>((TC)(wt[0] - q0), (TC)(wt[1] - q0), TC(0), (TC)(wt[3] - q0),
-                                        (TC)(wt[4] - q0), (TC)(wt[5] - q0), FT);
-                const TC d = ((FE * tf_face_dev<S, TC>(th, ox + 1, 1, FE, q0) - FW * tf_face_dev<S, TC>(th, ox, 1, FW, q0)) * m.idx +
-                              (FN * tf_face_dev<S, TC>(th, oy + sx, sx, FN, q0) - FS * tf_face_dev<S, TC>(th, oy, sx, FS, q0)) * m.idy) +
-                             (FT * FTf_t - FBm_t * FBf_t) * m.idz;
-                tt = TC(0) - d / (rc00 * J00);
+    // the own column's top values and the tile's halo of level kk (u, v, w one further)
+    auto load_level = [&](int kk) {
+        const uint32_t c = cof + (uint32_t)(kk + R) * sxy;
+        nxt[0] = inb ? u[c] : 0.0;
+        nxt[1] = inb ? v[c] : 0.0;
+        nxt[2] = inb ? w[c] : 0.0;
+        nxt[3] = inb ? th[c] : 0.0;
+#pragma unroll
+        for (int p = 0; p < NHP; p++) {
+            if (hv[p]) {
+                const uint32_t h0 = hof[p] + (uint32_t)kk * sxy, h1 = h0 + sxy;
+                hal[0][p] = u[h1];
+                hal[1][p] = v[h1];
+                hal[2][p] = w[h1];
+                hal[3][p] = th[h0];
             }
-            FBm_t = FT;
         }
-        // u at the x-face i
-        TC tu, FT_u;
-        {
-            const TC UE = rc00 * J00 * ((U(c, 0, 0, 0) + U(c, 1, 0, 0)) / TC(2));
-            const TC UW = (TC)fcm0.r * Jm0 * ((U(c, -1, 0, 0) + U(c, 0, 0, 0)) / TC(2));
-            const TC VN = (TC)fxy01.r * Jxy01 * ((V(c, -1, 1, 0) + V(c, 0, 1, 0)) / TC(2));
-            const TC VS = (TC)fxy00.r * Jxy00 * ((V(c, -1, 0, 0) + V(c, 0, 0, 0)) / TC(2));
-            const TC WT = (TC)(fxs00.r * fxs00.q) * ((Omm1 + Om1) / TC(2));
-            FT_u = WT * tf_face6<S, TC>(wu[0], wu[1], wu[2], wu[3], wu[4], wu[5], WT);
-            const TC d = ((UE * tf_face<S, TC>(u, ox + 1, 1, UE) - UW * tf_face<S, TC>(u, ox, 1, UW)) * m.idx +
-                          (VN * tf_face<S, TC>(u, oy + sx, sx, VN) - VS * tf_face<S, TC>(u, oy, sx, VS)) * m.idy) +
-                         (FT_u - FB_u) * m.idz;
-            tu = TC(0) - d / ((TC)fx00.r * Jx00);
+    };
+    // the tile of u, v, w at k0
+#pragma unroll
+    for (int p = 0; p < NHP; p++) {
+        if (hv[p]) {
+            const uint32_t h0 = hof[p] + (uint32_t)k0 * sxy;
+            tl[hat[p]] = (TC)u[h0];
+            tl[2 * TN + hat[p]] = (TC)v[h0];
+            tl[4 * TN + hat[p]] = (TC)w[h0];
         }
-        // v at the y-face j
-        TC tv, FT_v;
-        {
-            const TC VN = rc00 * J00 * ((V(c, 0, 0, 0) + V(c, 0, 1, 0)) / TC(2));
-            const TC VS = (TC)fc0m.r * J0m * ((V(c, 0, -1, 0) + V(c, 0, 0, 0)) / TC(2));
-            const TC UE = (TC)fxy10.r * Jxy10 * ((U(c, 1, -1, 0) + U(c, 1, 0, 0)) / TC(2));
-            const TC UW = (TC)fxy00.r * Jxy00 * ((U(c, 0, -1, 0) + U(c, 0, 0, 0)) / TC(2));
-            const TC WT = (TC)(fys00.r * fys00.q) * ((Om0m1 + Om1) / TC(2));
-            FT_v = WT * tf_face6<S, TC>(wv[0], wv[1], wv[2], wv[3], wv[4], wv[5], WT);
-            const TC d = ((UE * tf_face<S, TC>(v, ox + 1, 1, UE) - UW * tf_face<S, TC>(v, ox, 1, UW)) * m.idx +
-                          (VN * tf_face<S, TC>(v, oy + sx, sx, VN) - VS * tf_face<S, TC>(v, oy, sx, VS)) * m.idy) +
-                         (FT_v - FB_v) * m.idz;
-            tv = TC(0) - d / ((TC)fy00.r * Jy00);
+    }
+    if (inb) {
+        tl[at] = win[0][RL + 1];
+        tl[2 * TN + at] = win[1][RL + 1];
+        tl[4 * TN + at] = win[2][RL + 1];
+    }
+    load_level(k0);
+
+    // the thread's metric terms: ρ̄ at the σ-face k of its column, x-face and
+    // y-face (r), the ratio per half level (q), J; ρ̄J at the centres i − 1,
+    // j − 1 and at the corner (i, j), and the ratios per level
+    double r0 = 0, q0 = 0, rx = 0, qx = 0, ry = 0, qy = 0, ga = 0, qa = 0, gb = 0, qb = 0, gc = 0, qc = 0;
+    TC J0 = 0, Jx = 0, Jy = 0, hx0 = 0, hy0 = 0, uc = 0, vc = 0;
+    TC Om0 = 0, FBm = 0, FBf = 0, FBu = 0, FBv = 0, FBw = 0;
+    if (ok) {
+        const double h00 = hd(i, j), hw = hd(i - 1, j), hs = hd(i, j - 1), hx = hxd(i, j), hy = hyd(i, j), hc = hxyd(i, j);
+        r0 = rho(h00, 0.0); q0 = ratio(h00, 0.5);
+        rx = rho(hx, 0.0); qx = ratio(hx, 0.5);
+        ry = rho(hy, 0.0); qy = ratio(hy, 0.5);
+        ga = rho(hw, 0.5) * Jd(hw); qa = ratio(hw, 1.0);
+        gb = rho(hs, 0.5) * Jd(hs); qb = ratio(hs, 1.0);
+        gc = rho(hc, 0.5) * Jd(hc); qc = ratio(hc, 1.0);
+        J0 = (TC)Jd(h00); Jx = (TC)Jd(hx); Jy = (TC)Jd(hy);
+        hx0 = (TC)m.hx[i + sxi * j]; hy0 = (TC)m.hy[i + sxi * j];
+        // Ω at the σ-face kk of column (i + di, j + dj)
+        auto Om = [&](int di, int dj, int kk) -> TC {
+            if (kk == H || kk == H + m.Nz) return TC(0);
+            const uint32_t c = lin(i + di, j + dj, kk, m.sx, m.sy);
+            const TC ub = TC(0.25) * (((TC)u[c - sxy] + (TC)u[c - sxy + 1]) + ((TC)u[c] + (TC)u[c + 1]));
+            const TC vb = TC(0.25) * (((TC)v[c - sxy] + (TC)v[c - sxy + sx]) + ((TC)v[c] + (TC)v[c + sx]));
+            return (TC)w[c] + (m.jsx(i + di, j + dj, kk) * ub + m.jsy(i + di, j + dj, kk) * vb);
+        };
+        const uint32_t c = cof + (uint32_t)k0 * sxy;
+        uc = (TC)u[c] + (TC)u[c + 1];
+        vc = (TC)v[c] + (TC)v[c + sx];
+        Om0 = Om(0, 0, k0);
+        // the fluxes through the faces k0 (w's: through the centre k0 − 1)
+        const TC Ft = (TC)r0 * Om0;
+        const TC Wu = (TC)rx * ((Om(-1, 0, k0) + Om0) * TC(0.5)), Wv = (TC)ry * ((Om(0, -1, k0) + Om0) * TC(0.5));
+        const TC Ww = (TC)(r0 / q0) * ((Om(0, 0, k0 - 1) + Om0) * TC(0.5));
+        FBm = Ft;
+        if constexpr (DEV) {
+            const double b = wt[RL + 1];  // about θ of level k0
+            FBf = tf_face6<S, TC>((TC)(wt[0] - b), (TC)(wt[1] - b), (TC)(wt[2] - b), TC(0), (TC)(wt[4] - b), (TC)(wt[5] - b), Ft);
+        } else {
+            FBf = tf_face6<S, TC>(wt[0], wt[1], wt[2], wt[3], wt[4], wt[5], Ft);
         }
-        // w at the σ-face k (the ground face is diagnostic); its upper flux
-        // through the centre k is carried whatever k
-        TC tw = TC(0), FT_w;
-        {
-            const TC WT = rc00 * ((Om0 + Om1) / TC(2));
-            // w(k − 2 .. k + 3): the face between the centre k's faces k and k + 1 is w(k), w(k+1)
-            FT_w = WT * tf_face6<S, TC>(ww[0], ww[1], ww[2], ww[3], ww[4], ww[5], WT);
+        FBu = Wu * tf_face6<S, TC>(win[0][0], win[0][1], win[0][2], win[0][3], win[0][4], win[0][5], Wu);
+        FBv = Wv * tf_face6<S, TC>(win[1][0], win[1][1], win[1][2], win[1][3], win[1][4], win[1][5], Wv);
+        FBw = Ww * tf_face6<S, TC>(win[2][0], win[2][1], win[2][2], win[2][3], win[2][4], win[2][5], Ww);
+    }
+    // a face of the block's far edges: the field's tile cell f whose west or
+    // south face it is (stride st), the velocities at tile cells A and B (w:
+    // one cell, at levels k − 1 and k), ρ̄J there and its ratio per level
+    struct Item {
+        double r, q;
+        TC prev;
+        int F, f, st, A, B, dst;
+    };
+    Item it[2];
+    it[0].F = it[1].F = -1;
+    auto set_item = [&](Item &t, int F, int a, int b, int dir) {  // the minus face of cell (a, b) in direction dir
+        const int cell = (b - jb + R) * TW + (a - i0 + R), vel = dir == 0 ? 0 : 2 * TN;
+        const int st = dir == 0 ? 1 : TW;
+        t.F = F;
+        t.f = cell;
+        t.st = st;
+        t.B = vel + cell;
+        t.A = t.B;
+        t.prev = TC(0);
+        double hs, off = 0.5;
+        if (F == 3) hs = dir == 0 ? hxd(a, b) : hyd(a, b);
+        else if (F == dir) {
+            hs = dir == 0 ? hd(a - 1, b) : hd(a, b - 1);
+            t.A = t.B - st;
+        } else if (F == 2) {
+            hs = dir == 0 ? hxd(a, b) : hyd(a, b);
+            off = 0.0;
+            const uint32_t c = lin(a, b, k0 - 1, m.sx, m.sy);
+            t.prev = (TC)(dir == 0 ? u[c] : v[c]);
+        } else {
+            hs = hxyd(a, b);
+            t.A = t.B - (F == 0 ? 1 : TW);
+        }
+        t.r = rho(hs, off) * Jd(hs);
+        t.q = ratio(hs, 1.0);
+        t.dst = dir == 0 ? F * XN + (b - jb) * 65 + (a - i0) : F * YN + (b - jb) * 64 + (a - i0);
+    };
+    if (wv < 4 && i <= ilast) set_item(it[0], wv, i, jlast + 1, 1);
+    constexpr int WE = BY == 4 ? 1 : 4;  // the waves of the east faces: u, v, w; θ
+    if (wv == WE && lane < 3 * BY && jb + lane % BY <= jlast) set_item(it[1], lane / BY, ilast + 1, jb + lane % BY, 0);
+    if (wv == WE + 1 && lane < BY && jb + lane <= jlast) set_item(it[1], 3, ilast + 1, jb + lane, 0);
+    // Ω of the row (wave 0) and the column (wave 3) before the block
+    int oat = -1, odst = 0;
+    TC ohx = 0, ohy = 0;
+    if ((wv == 0 && i <= ilast) || (wv == 3 && lane < BY && jb + lane <= jlast)) {
+        const int a = wv == 0 ? i : i0 - 1, b = wv == 0 ? jb - 1 : jb + lane;
+        oat = (b - jb + R) * TW + (a - i0 + R);
+        odst = (b - jb + 1) * 65 + (a - i0 + 1);
+        ohx = (TC)m.hx[a + sxi * b];
+        ohy = (TC)m.hy[a + sxi * b];
+    }
+
+    // the minus face of tile cell f: a velocity vel, stride st
+    auto face = [&](const TC *f, int st, TC vel) -> TC {
+        return vel * tf_face6<S, TC>(f[-3 * st], f[-2 * st], f[-st], f[0], f[st], f[2 * st], vel);
+    };
+    // θ's: FP64 the flux; FP32 the flux of θ less the θ of the cell f
+    auto face_t = [&](const double *f, int st, TC vel) -> TC {
+        const double b = DEV ? f[0] : 0.0;
+        return vel * tf_face6<S, TC>((TC)(f[-3 * st] - b), (TC)(f[-2 * st] - b), (TC)(f[-st] - b), (TC)(f[0] - b),
+                                     (TC)(f[st] - b), (TC)(f[2 * st] - b), vel);
+    };
+    auto run_item = [&](Item &t, TC *out, TC *mout, int po) {
+        if (t.F >= 0) {
+            const TC B = tl[t.B + po];
+            const TC A = t.F == 2 ? t.prev : tl[t.A + po];
+            const TC vel = (TC)t.r * ((A + B) * TC(0.5));
+            t.prev = B;
+            t.r *= t.q;
+            if (t.F == 3) {
+                out[t.dst] = face_t(ts + t.f, t.st, vel);
+                if constexpr (DEV) mout[t.dst - 3 * (out == xs ? XN : YN)] = vel;
+            } else {
+                out[t.dst] = face(tl + 2 * t.F * TN + t.f + po, t.st, vel);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    for (int k = k0; k < k1; k++) {
+        const int po = ((k - k0) & 1) * TN, pn = TN - po;  // the slots of levels k and k + 1
+#pragma unroll
+        for (int n = 0; n < NW - 1; n++) {
+            win[0][n] = win[0][n + 1]; win[1][n] = win[1][n + 1]; win[2][n] = win[2][n + 1];
+            wt[n] = wt[n + 1];
+        }
+        win[0][NW - 1] = (TC)nxt[0]; win[1][NW - 1] = (TC)nxt[1]; win[2][NW - 1] = (TC)nxt[2];
+        wt[NW - 1] = nxt[3];
+#pragma unroll
+        for (int p = 0; p < NHP; p++) {
+            if (hv[p]) {
+                tl[pn + hat[p]] = (TC)hal[0][p];
+                tl[2 * TN + pn + hat[p]] = (TC)hal[1][p];
+                tl[4 * TN + pn + hat[p]] = (TC)hal[2][p];
+                ts[hat[p]] = hal[3][p];
+            }
+        }
+        if (k + 1 < k1) load_level(k + 1);  // in flight over this level's faces
+        if (inb) {
+            tl[pn + at] = win[0][RL + 1];
+            tl[2 * TN + pn + at] = win[1][RL + 1];
+            tl[4 * TN + pn + at] = win[2][RL + 1];
+            ts[at] = wt[RL];
+        }
+        __syncthreads();
+
+        const TC *tu = tl + po + at, *tv = tu + 2 * TN, *tw = tu + 4 * TN;
+        const double *tt_ = ts + at;
+        const double rc = r0 * q0;                                   // ρ̄ at the centre k
+        const TC mx = (TC)(rx * qx) * Jx, my = (TC)(ry * qy) * Jy;  // ρ̄J at the x- and the y-face
+        const TC tauf = ((TC)(k + 1 - H) * m.dz - m.Hl) * m.iHl;    // −τ/H of the face k + 1
+        TC Om1 = TC(0), de = TC(0), dn = TC(0);
+        if (ok) {
+            const TC U = win[0][RL], V = win[1][RL];
+            // Ω(k + 1)
+            const TC u1 = win[0][RL + 1] + tl[pn + at + 1], v1 = win[1][RL + 1] + tl[2 * TN + pn + at + TW];
+            if (k + 1 < H + m.Nz)
+                Om1 = win[2][RL + 1] + tauf * TC(0.25) * (hx0 * (uc + u1) + hy0 * (vc + v1));
+            om[(ty + 1) * 65 + lane + 1] = Om1;
+            uc = u1;
+            vc = v1;
+            TC *xo = xs + ty * 65 + lane, *yo = ys + ty * 64 + lane;
+            const TC ul = tu[-1], vl = tv[-1], ud = tu[-TW], vd = tv[-TW];
+            xo[0] = face(tu, 1, (TC)ga * ((ul + U) * TC(0.5)));
+            __builtin_amdgcn_sched_barrier(0);
+            yo[0] = face(tu, TW, (TC)gc * ((vl + V) * TC(0.5)));
+            __builtin_amdgcn_sched_barrier(0);
+            xo[XN] = face(tv, 1, (TC)gc * ((ud + U) * TC(0.5)));
+            __builtin_amdgcn_sched_barrier(0);
+            yo[YN] = face(tv, TW, (TC)gb * ((vd + V) * TC(0.5)));
+            __builtin_amdgcn_sched_barrier(0);
+            xo[2 * XN] = face(tw, 1, (TC)rx * Jx * ((win[0][RL - 1] + U) * TC(0.5)));
+            __builtin_amdgcn_sched_barrier(0);
+            yo[2 * YN] = face(tw, TW, (TC)ry * Jy * ((win[1][RL - 1] + V) * TC(0.5)));
+            __builtin_amdgcn_sched_barrier(0);
+            xo[3 * XN] = face_t(tt_, 1, mx * U);
+            __builtin_amdgcn_sched_barrier(0);
+            yo[3 * YN] = face_t(tt_, TW, my * V);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (DEV) {
+                xm[ty * 65 + lane] = mx * U;
+                ym[ty * 64 + lane] = my * V;
+                de = (TC)(tt_[1] - wt[RL]);
+                dn = (TC)(tt_[TW] - wt[RL]);
+            }
+        }
+        run_item(it[0], ys, ym, po);
+        run_item(it[1], xs, xm, po);
+        if (oat >= 0) {
+            TC o = TC(0);
+            if (k + 1 < H + m.Nz) {
+                const TC *a = tl + po + oat, *b = tl + pn + oat;
+                const TC *av = a + 2 * TN, *bv = b + 2 * TN;
+                o = b[4 * TN] + tauf * TC(0.25) * (ohx * ((a[0] + a[1]) + (b[0] + b[1])) + ohy * ((av[0] + av[TW]) + (bv[0] + bv[TW])));
+            }
+            om[odst] = o;
+        }
+        __syncthreads();
+
+        if (ok) {
+            const uint32_t c = cof + (uint32_t)k * sxy;
+            const double r1 = rc * q0, rx1 = rx * qx * qx, ry1 = ry * qy * qy;  // at the faces k + 1
+            const TC *xo = xs + ty * 65 + lane, *yo = ys + ty * 64 + lane;
+            // u
+            const TC Wu = (TC)rx1 * ((om[(ty + 1) * 65 + lane] + Om1) * TC(0.5));
+            const TC FTu = Wu * tf_face6<S, TC>(win[0][0], win[0][1], win[0][2], win[0][3], win[0][4], win[0][5], Wu);
+            const TC tu_ = -qdiv<TC>(((xo[1] - xo[0]) * m.idx + (yo[64] - yo[0]) * m.idy) + (FTu - FBu) * m.idz, mx);
+            FBu = FTu;
+            us[c] = raw ? (double)tu_ : (DEV ? u[c] : (double)win[0][RL]) + dt * (double)tu_;
+            __builtin_amdgcn_sched_barrier(0);
+            // v
+            const TC Wv = (TC)ry1 * ((om[ty * 65 + lane + 1] + Om1) * TC(0.5));
+            const TC FTv = Wv * tf_face6<S, TC>(win[1][0], win[1][1], win[1][2], win[1][3], win[1][4], win[1][5], Wv);
+            const TC tv_ = -qdiv<TC>(((xo[XN + 1] - xo[XN]) * m.idx + (yo[YN + 64] - yo[YN]) * m.idy) + (FTv - FBv) * m.idz, my);
+            FBv = FTv;
+            vs[c] = raw ? (double)tv_ : (DEV ? v[c] : (double)win[1][RL]) + dt * (double)tv_;
+            __builtin_amdgcn_sched_barrier(0);
+            // w at the σ-face k (the ground face is diagnostic); its upper flux is carried whatever k
+            const TC Ww = (TC)rc * ((Om0 + Om1) * TC(0.5));
+            const TC FTw = Ww * tf_face6<S, TC>(win[2][0], win[2][1], win[2][2], win[2][3], win[2][4], win[2][5], Ww);
+            TC tw_ = TC(0);
             if (k > H) {
-                const TC UE = (TC)fxs10.r * Jx10 * ((U(c, 1, 0, -1) + U(c, 1, 0, 0)) / TC(2));
-                const TC UW = (TC)fxs00.r * Jx00 * ((U(c, 0, 0, -1) + U(c, 0, 0, 0)) / TC(2));
-                const TC VN = (TC)fys01.r * Jy01 * ((V(c, 0, 1, -1) + V(c, 0, 1, 0)) / TC(2));
-                const TC VS = (TC)fys00.r * Jy00 * ((V(c, 0, 0, -1) + V(c, 0, 0, 0)) / TC(2));
-                const TC d = ((UE * tf_face<S, TC>(w, ox + 1, 1, UE) - UW * tf_face<S, TC>(w, ox, 1, UW)) * m.idx +
-                              (VN * tf_face<S, TC>(w, oy + sx, sx, VN) - VS * tf_face<S, TC>(w, oy, sx, VS)) * m.idy) +
-                             (FT_w - FB_w) * m.idz;
-                tw = TC(0) - d / ((TC)fs00.r * J00);
+                tw_ = -qdiv<TC>(((xo[2 * XN + 1] - xo[2 * XN]) * m.idx + (yo[2 * YN + 64] - yo[2 * YN]) * m.idy) +
+                                    (FTw - FBw) * m.idz, (TC)r0 * J0);
                 if (m.buoyancy) {
-                    const TC zf = m.hp(i, j) + m.sigf(k) * J00;
+                    const TC zf = m.hp(i, j) + m.sigf(k) * J0;
                     const double tb = (double)m.theta0 + (double)m.gamma * (double)zf;
-                    const double coef = (double)m.g / tb;
-                    const double tface = 0.5 * (wt[1] + wt[2]);
-                    tw += (TC)(coef * (tface - tb));
+                    tw_ += (TC)((double)m.g / tb * (0.5 * (wt[RL - 1] + wt[RL]) - tb));
                 }
             }
-        }
-        if (raw) {
-            us[c] = (double)tu;
-            vs[c] = (double)tv;
-            ws[c] = (double)tw;
-            tn[c] = (double)tt;
-        } else {
-            us[c] = u[c] + dt * (double)tu;
-            vs[c] = v[c] + dt * (double)tv;
-            ws[c] = k > H ? w[c] + dt * (double)tw : w[c];
-            const double tnew = wt[2] + dt * (double)tt;
-            tn[c] = combine ? ca * th0[c] + cb * tnew : tnew;
-        }
-        // up one level: the carries and the windows
-        FBf_t = FTf_t; FB_u = FT_u; FB_v = FT_v; FB_w = FT_w;
-        OmB = Om0; Om0 = Om1; Omm0 = Omm1; Om0m = Om0m1;
-        if (k + 1 < ke) {
-            const uint32_t cn = c + 4 * sxy;  // level k + 4 = the new window top (k + 1) + 3
-            for (int q = 0; q < 5; q++) {
-                wu[q] = wu[q + 1]; wv[q] = wv[q + 1]; ww[q] = ww[q + 1]; wt[q] = wt[q + 1];
+            FBw = FTw;
+            const double w0 = DEV ? w[c] : (double)win[2][RL];
+            ws[c] = raw ? (double)tw_ : k > H ? w0 + dt * (double)tw_ : w0;
+            __builtin_amdgcn_sched_barrier(0);
+            // θ
+            const TC FT = (TC)r1 * Om1;
+            TC d, FTf;
+            if constexpr (DEV) {
+                // the flux form less θ_c·(B u)/(ρJ): B u vanishes to the projection's tolerance, and its
+                // FP32 rounding times θ ≈ 300 K would swamp the tendency of the perturbation
+                const double b = wt[RL];
+                FTf = tf_face6<S, TC>((TC)(wt[0] - b), (TC)(wt[1] - b), TC(0), (TC)(wt[3] - b), (TC)(wt[4] - b), (TC)(wt[5] - b), FT);
+                const TC FE = xo[3 * XN + 1] + xm[ty * 65 + lane + 1] * de, FN = yo[3 * YN + 64] + ym[(ty + 1) * 64 + lane] * dn;
+                d = ((FE - xo[3 * XN]) * m.idx + (FN - yo[3 * YN]) * m.idy) + (FT * FTf - FBm * FBf) * m.idz;
+                FBf = FTf - (TC)(wt[RL + 1] - wt[RL]);  // re-based on θ of level k + 1
+            } else {
+                FTf = tf_face6<S, TC>(wt[0], wt[1], wt[2], wt[3], wt[4], wt[5], FT);
+                d = ((xo[3 * XN + 1] - xo[3 * XN]) * m.idx + (yo[3 * YN + 64] - yo[3 * YN]) * m.idy) + (FT * FTf - FBm * FBf) * m.idz;
+                FBf = FTf;
             }
-            wu[5] = (TC)u[cn]; wv[5] = (TC)v[cn]; ww[5] = (TC)w[cn]; wt[5] = th[cn];
-            if constexpr (sizeof(TC) == 4) FBf_t -= (TC)(wt[2] - wt[1]);  // re-based on θ of level k + 1
-            fc00.r *= fc00.q; fcm0.r *= fcm0.q; fc0m.r *= fc0m.q;
-            fx00.r *= fx00.q; fx10.r *= fx10.q; fy00.r *= fy00.q; fy01.r *= fy01.q;
-            fxy00.r *= fxy00.q; fxy01.r *= fxy01.q; fxy10.r *= fxy10.q;
-            fs00.r *= fs00.q; fxs00.r *= fxs00.q; fxs10.r *= fxs10.q; fys00.r *= fys00.q; fys01.r *= fys01.q;
+            FBm = FT;
+            const double tt = (double)-qdiv<TC>(d, (TC)rc * J0);
+            const double tnew = wt[RL] + dt * tt;
+            tn[c] = raw ? tt : combine ? ca * th0[c] + cb * tnew : tnew;
+            Om0 = Om1;
+            r0 = r1;
+            rx = rx1;
+            ry = ry1;
+            ga *= qa;
+            gb *= qb;
+            gc *= qc;
         }
+        // no barrier here: the next level's tile writes touch nothing this phase reads
     }
 }
+#pragma clang fp contract(off)
 
 // ---------------------------------------------------------------------------
 // halos: u, v, θ periodic in x, y and mirrored in σ (the generic halo
@@ -709,17 +868,26 @@ static TFOp make_op(const TFWView &v, const double *bx, const double *by, const 
     return op;
 }
 
+template <int S, typename TC>
+static void launch_tendency_tile(hipStream_t st, const TFWView &v, double *us, double *vs, double *ws, double *tn,
+                                 const double *u, const double *vv, const double *w, const double *th,
+                                 const double *th0, double dt, double ca, double cb, int combine, int raw) {
+    constexpr int BY = TFT_BY;
+    const int tx = (v.Nx + 63) / 64, ty = (v.Ny + BY - 1) / BY;
+    const int kc = chunk_levels(tx * ty, v.Nz, TFT_KC, TFT_FILL, 2);
+    hipLaunchKernelGGL((tfw_tendency_tile_kernel<S, TC, BY>), dim3(tx, ty, (v.Nz + kc - 1) / kc), dim3(64, BY), 0, st,
+                       us, vs, ws, tn, u, vv, w, th, th0, make_tfm<TC>(v), dt, ca, cb, combine, raw, kc);
+}
+
 int launch_tfw_tendency(hipStream_t st, const TFWView &v, int scheme, int f32, double *us, double *vs, double *ws,
                         double *tn, const double *u, const double *vv, const double *w, const double *th,
                         const double *th0, double dt, double ca, double cb, int combine, int raw) {
-    constexpr int CH = TFW_TEND_CH;
-    dim3 blk(64, 4), grid((v.Nx + 63) / 64, (v.Ny + 3) / 4, (v.Nz + CH - 1) / CH);
     if (scheme == SCH_CENTERED) {
-        if (f32) hipLaunchKernelGGL((tfw_tendency_march_kernel<SCH_CENTERED, float, CH>), grid, blk, 0, st, us, vs, ws, tn, u, vv, w, th, th0, make_tfm<float>(v), dt, ca, cb, combine, raw);
-        else hipLaunchKernelGGL((tfw_tendency_march_kernel<SCH_CENTERED, double, CH>), grid, blk, 0, st, us, vs, ws, tn, u, vv, w, th, th0, make_tfm<double>(v), dt, ca, cb, combine, raw);
+        if (f32) launch_tendency_tile<SCH_CENTERED, float>(st, v, us, vs, ws, tn, u, vv, w, th, th0, dt, ca, cb, combine, raw);
+        else launch_tendency_tile<SCH_CENTERED, double>(st, v, us, vs, ws, tn, u, vv, w, th, th0, dt, ca, cb, combine, raw);
     } else if (scheme == SCH_WENO_Z5) {
-        if (f32) hipLaunchKernelGGL((tfw_tendency_march_kernel<SCH_WENO_Z5, float, CH>), grid, blk, 0, st, us, vs, ws, tn, u, vv, w, th, th0, make_tfm<float>(v), dt, ca, cb, combine, raw);
-        else hipLaunchKernelGGL((tfw_tendency_march_kernel<SCH_WENO_Z5, double, CH>), grid, blk, 0, st, us, vs, ws, tn, u, vv, w, th, th0, make_tfm<double>(v), dt, ca, cb, combine, raw);
+        if (f32) launch_tendency_tile<SCH_WENO_Z5, float>(st, v, us, vs, ws, tn, u, vv, w, th, th0, dt, ca, cb, combine, raw);
+        else launch_tendency_tile<SCH_WENO_Z5, double>(st, v, us, vs, ws, tn, u, vv, w, th, th0, dt, ca, cb, combine, raw);
     } else {
         return -1;
     }
