@@ -280,7 +280,122 @@ struct TFChain {
         const T tu = t - dz;
         return (k + 1 < k1 ? z * qup : z1) * ma(tu * tu, g2, iJJ);
     }
+    // a colour's march, every other level: from here step() takes two levels
+    __device__ __forceinline__ void col(const TFM<T> &gm, const LevelD<T> &L, const double *, int i, int j, int k0, int k1) {
+        init(gm, L, i + gm.H, j + gm.H, k0 + gm.H, k1 + gm.H);
+    }
+    __device__ __forceinline__ void skip() { step(); }  // up one level, before two()
+    T q1, d1;                                           // z's ratio and t's step of one level
+    __device__ __forceinline__ void two() {
+        q1 = qz; d1 = dz;
+        qxm *= qxm; qxp *= qxp; qym *= qym; qyp *= qyp; qz *= qz;
+        dz += dz;
+    }
+    __device__ __forceinline__ T cxm() const { return xm; }
+    __device__ __forceinline__ T cxp() const { return xp; }
+    __device__ __forceinline__ T cym() const { return ym; }
+    __device__ __forceinline__ T cyp() const { return yp; }
+    // the lower and upper σ-face's coefficients of level k
+    __device__ __forceinline__ void zfaces(int k, int k1, T &lo, T &up) {
+        lo = lower();
+        const T tu = t - d1;
+        up = (k + 1 < k1 ? z * q1 : z1) * ma(tu * tu, g2, iJJ);
+    }
 };
+
+// The same for the level below the finest (FP64): a coarse face's coefficient
+// is the mean of its four fine faces' (restrict_coeff). On a lateral face
+// these are two levels of two fine columns, so the sum over the levels is each
+// column's lower value times 1 + ratio, carried by the ratio's square; a
+// σ-face takes four fine columns at one fine level, each with its share
+// of (H − σ)² and of 1. The values at each chunk's first level and the ratios
+// are kept in a table (tf_table_kernel), read once per chunk, since the 24 exps
+// of a thread cost as much as half its cells (128×68×44: 12.6 us a pass with
+// the exps, 7.8 from the table).
+constexpr int TFC_Q = 8, TFC_V = 12;  // planes of ratios, of values per chunk
+constexpr size_t TFC_MIN = 3 << 19;   // least cells of the level (mg_set_terrain_coef)
+struct TFChain2 {
+    double x[4], y[4], qx[4], qy[4];  // west, west, east, east; south, south, north, north
+    double zg[4], zi[4], qz[4], t, dz;                // t: H − σ at the current lower σ-face
+    __device__ __forceinline__ void col(const TFM<double> &gm, const LevelD<double> &L, const double *tab, int i, int j, int k0, int) {
+        // the planes, each (nx + 1) × (ny + 1)
+        const uint32_t w = (uint32_t)L.nx + 1, n = w * ((uint32_t)L.ny + 1), c = (uint32_t)i + w * (uint32_t)j;
+        const double *v = tab + (size_t)n * (TFC_Q + TFC_V * blockIdx.z);
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            x[o] = v[o * n + c]; x[2 + o] = v[o * n + c + 1];
+            y[o] = v[(2 + o) * n + c]; y[2 + o] = v[(2 + o) * n + c + w];
+            qx[o] = tab[o * n + c]; qx[2 + o] = tab[o * n + c + 1];
+            qy[o] = tab[(2 + o) * n + c]; qy[2 + o] = tab[(2 + o) * n + c + w];
+        }
+#pragma unroll
+        for (int o = 0; o < 4; o++) {
+            qz[o] = tab[(4 + o) * n + c];
+            zg[o] = v[(4 + o) * n + c];
+            zi[o] = v[(8 + o) * n + c];
+        }
+        dz = 2.0 * gm.dz;
+        t = gm.Hl - k0 * dz;
+    }
+    __device__ __forceinline__ double zf() const {
+        return __builtin_fma(t * t, (zg[0] + zg[1]) + (zg[2] + zg[3]), (zi[0] + zi[1]) + (zi[2] + zi[3]));
+    }
+    // σ's part goes up with each face taken, two a cell
+    __device__ __forceinline__ void zfaces(int, int, double &lo, double &up) {
+        lo = zf();
+        zstep();
+        up = zf();
+        zstep();
+    }
+    __device__ __forceinline__ void zstep() {
+#pragma unroll
+        for (int c = 0; c < 4; c++) { zg[c] *= qz[c]; zi[c] *= qz[c]; }
+        t -= dz;
+    }
+    __device__ __forceinline__ void step() {
+#pragma unroll
+        for (int c = 0; c < 4; c++) { x[c] *= qx[c]; y[c] *= qy[c]; }
+    }
+    __device__ __forceinline__ void skip() { step(); zstep(); }
+    __device__ __forceinline__ void two() {
+#pragma unroll
+        for (int c = 0; c < 4; c++) { qx[c] *= qx[c]; qy[c] *= qy[c]; }
+    }
+    __device__ __forceinline__ double cxm() const { return x[0] + x[1]; }
+    __device__ __forceinline__ double cxp() const { return x[2] + x[3]; }
+    __device__ __forceinline__ double cym() const { return y[0] + y[1]; }
+    __device__ __forceinline__ double cyp() const { return y[2] + y[3]; }
+};
+
+// TFChain2's table: thread (i, j) of (nx + 1) × (ny + 1), chunk blockIdx.z
+__global__ void tf_table_kernel(double *__restrict__ tab, TFM<double> gm, int nx, int ny, int kc, double ix2, double iy2,
+                                double iz2) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
+    if (i > nx) return;
+    const uint32_t w = (uint32_t)nx + 1, n = w * ((uint32_t)ny + 1), c = (uint32_t)i + w * (uint32_t)j;
+    double *v = tab + (size_t)n * (TFC_Q + TFC_V * blockIdx.z);
+    const int I = 2 * i + gm.H, J = 2 * j + gm.H, K = 2 * kc * (int)blockIdx.z + gm.H;
+    const double sc = gm.sigc(K);
+    for (int o = 0; o < 2; o++) {
+        // (the last column and row have no faces beyond their first)
+        const int jo = j < ny ? J + o : J, io = i < nx ? I + o : I;
+        const double Jx = gm.Jx(I, jo), Jy = gm.Jy(io, J);
+        const double rx = exp(-(gm.dz * Jx) * gm.iHs), ry = exp(-(gm.dz * Jy) * gm.iHs);
+        v[o * n + c] = gm.rho(gm.hxf(I, jo) + sc * Jx) * Jx * (1.0 + rx) * (0.25 * ix2);
+        v[(2 + o) * n + c] = gm.rho(gm.hyf(io, J) + sc * Jy) * Jy * (1.0 + ry) * (0.25 * iy2);
+        tab[o * n + c] = rx * rx;
+        tab[(2 + o) * n + c] = ry * ry;
+    }
+    for (int o = 0; o < 4; o++) {
+        const int a = i < nx ? I + (o & 1) : I, b = j < ny ? J + (o >> 1) : J;
+        const double hc = gm.hp(a, b), Jc = gm.J(a, b), den = gm.Hl - hc;
+        const double ax = gm.hx[a + gm.sx * b] / den, ay = gm.hy[a + gm.sx * b] / den;
+        const double z = gm.rho(hc + gm.sigf(K) * Jc) * Jc * (0.25 * iz2);
+        v[(4 + o) * n + c] = z * (ax * ax + ay * ay);
+        v[(8 + o) * n + c] = z / (Jc * Jc);
+        tab[(4 + o) * n + c] = exp(-2.0 * (gm.dz * Jc) * gm.iHs);
+    }
+}
 
 // One colour of the red-black sweep on the terrain grid's finest level
 // (FP64), with the face coefficients evaluated from the Gal-Chen metrics
@@ -307,8 +422,9 @@ struct TFChain {
 constexpr int RBC_BY = 2;   // rows per block
 constexpr int RBC_KC = 32;  // most levels per chunk
 constexpr int RBC_FILL = 2048;  // blocks a round (chunk_levels); 96×96×48 step 22.1 ms with 32 levels, 18.8 to 19.2 with 1024 or 2048 blocks
-template <bool FROM0, bool SUM>
-__global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, TFM<double> gm, int colour, int kc,
+template <bool FROM0, bool SUM, class CH>
+__global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, TFM<double> gm,
+                                                              const double *__restrict__ tab, int colour, int kc,
                                                               int first, double *__restrict__ partials, int npb,
                                                               uint32_t half) {
     static_assert(!(FROM0 && SUM), "the from-zero pass is a sweep's first");
@@ -317,10 +433,9 @@ __global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, 
     if (!SUM && !ok) return;
     const int i = ok ? i0 : 0, j = ok ? j0 : 0;
     const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, L.nz);
-    const int I = i + gm.H, J = j + gm.H;
     double srz = 0.0, sz = 0.0, sr = 0.0;
-    TFChain<double> q;
-    q.init(gm, L, I, J, k0 + gm.H, k1 + gm.H);
+    CH q;
+    q.col(gm, L, tab, i, j, k0, k1);
     const double *f = L.phi;
     // a neighbour cn of cell cs (cn == cs: a mirror boundary)
     auto nb = [&](uint32_t cn, uint32_t cs) {
@@ -331,7 +446,7 @@ __global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, 
     const int jyp = wrapc(j + 1, L.ny, L.bcy), jym = wrapc(j - 1, L.ny, L.bcy);
     auto pi = [&](int ii, int jj, int kk) { return split_at(half, ii, jj, kk, lidx(L, ii, jj, kk)); };  // the index of φ and b
     int k = k0 + ((i + j + k0 + colour) & 1);
-    if (k > k0) q.step();
+    if (k > k0) q.skip();
     double zm = 0.0;
     if (ok && k < k1) {
         const uint32_t cb = pi(i, j, wrapc(k - 1, L.nz, L.bcz));
@@ -363,24 +478,22 @@ __global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, 
     const uint32_t oxp = lat(ixp, j), oxm = lat(ixm, j), oyp = lat(i, jyp), oym = lat(i, jym);
     const uint32_t ozp = spl ? dbase + (nxy >> 1) : nxy, sstep = spl ? nxy : 2 * nxy;
     uint32_t cs = pi(i, j, k);  // the cell's index
-    // from here the chain steps two levels at once
-    const double qz = q.qz;
-    q.qxm *= q.qxm; q.qxp *= q.qxp; q.qym *= q.qym; q.qyp *= q.qyp; q.qz *= q.qz;
-    q.dz += q.dz;
+    q.two();
     for (; ok && k < k1; k += 2, cs += sstep) {
         const double xp = nb(cs + oxp, cs), xm = nb(cs + oxm, cs);
         const double yp = nb(cs + oyp, cs), ym = nb(cs + oym, cs);
         const uint32_t cu = k + 1 < L.nz ? cs + ozp : pi(i, j, wrapc(k + 1, L.nz, L.bcz));
         const double zp = nb(cu, cs);
-        const double fzm = q.lower(), tu = q.t - gm.dz;
-        const double fzp = (k + 1 < k1 ? q.z * qz : q.z1) * __builtin_fma(tu * tu, q.g2, q.iJJ);
+        double fzm, fzp;
+        q.zfaces(k, k1, fzm, fzp);
+        const double fxm = q.cxm(), fxp = q.cxp(), fym = q.cym(), fyp = q.cyp();
         const double bv = L.b[cs];
-        const double diag = ((q.xp + q.xm) + (q.yp + q.ym)) + (fzp + fzm);  // −diag of A
+        const double diag = ((fxp + fxm) + (fyp + fym)) + (fzp + fzm);  // −diag of A
         double vnew;
         if (diag < Eps<double>::v) {
             vnew = FROM0 || first ? 0.0 : f[cs];
         } else {
-            const double ox = __builtin_fma(q.xp, xp, q.xm * xm), oy = __builtin_fma(q.yp, yp, q.ym * ym);
+            const double ox = __builtin_fma(fxp, xp, fxm * xm), oy = __builtin_fma(fyp, yp, fym * ym);
             const double oz = __builtin_fma(fzp, zp, __builtin_fma(fzm, zm, -bv));
             vnew = qdiv<double>((ox + oy) + oz, diag);
         }
@@ -434,7 +547,7 @@ constexpr int RRC_BW = 4;  // waves per block
 __global__ void __launch_bounds__(64 * RRC_BW) residual_restrict_tf_kernel(LevelD<double> L, LevelD<double> C,
                                                                            TFM<double> gm, int kc,
                                                                            double *__restrict__ partials,
-                                                                           uint32_t half) {
+                                                                           uint32_t half, uint32_t halfc) {
     __shared__ double sh[RRC_BW];
     const int lane = threadIdx.x, wv = threadIdx.y;
     const int ci = blockIdx.x * 32 + (lane & 31), cj = blockIdx.y * RRC_BW + wv;
@@ -504,7 +617,7 @@ __global__ void __launch_bounds__(64 * RRC_BW) residual_restrict_tf_kernel(Level
         r += __shfl_xor(r, 32, 64);
         const double bc = r * 0.125;
         if (ok && lane < 32) {
-            C.b[lidx(C, ci, cj, k >> 1)] = bc;
+            C.b[split_at(halfc, ci, cj, k >> 1, lidx(C, ci, cj, k >> 1))] = bc;
             total += bc;
         }
     }
@@ -535,7 +648,7 @@ constexpr int PRC_BY = 4;   // rows per block
 constexpr int PRC_KC = 16;  // most fine levels per chunk (even)
 constexpr int PRC_FILL = 1024;  // blocks a round (chunk_levels)
 __global__ void __launch_bounds__(64 * PRC_BY) prolong_tf_kernel(LevelD<double> F, LevelD<double> C, int kc,
-                                                                 uint32_t half) {
+                                                                 uint32_t half, uint32_t halfc) {
     const int pr = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * PRC_BY + __builtin_amdgcn_readfirstlane(threadIdx.y);
     if (pr >= C.nx || j >= F.ny) return;
     const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, F.nz);
@@ -544,9 +657,9 @@ __global__ void __launch_bounds__(64 * PRC_BY) prolong_tf_kernel(LevelD<double> 
     // the x-y sums of coarse level m for the pair's columns 2·pr (l) and 2·pr + 1 (r)
     auto plane = [&](int m, double &l, double &r) {
         const int mm = wrapc(m, C.nz, C.bcz);
-        const uint32_t a = lidx(C, 0, J, mm), b = lidx(C, 0, jy, mm);
-        const double near = 0.75 * C.phi[a + pr] + 0.25 * C.phi[b + pr];
-        const double nl = 0.75 * C.phi[a + xl] + 0.25 * C.phi[b + xl], nr = 0.75 * C.phi[a + xr] + 0.25 * C.phi[b + xr];
+        auto at = [&](int i, int jc) { return C.phi[split_at(halfc, i, jc, mm, lidx(C, i, jc, mm))]; };
+        const double near = 0.75 * at(pr, J) + 0.25 * at(pr, jy);
+        const double nl = 0.75 * at(xl, J) + 0.25 * at(xl, jy), nr = 0.75 * at(xr, J) + 0.25 * at(xr, jy);
         l = 0.75 * near + 0.25 * nl;
         r = 0.75 * near + 0.25 * nr;
     };
@@ -706,8 +819,9 @@ __global__ void restrict_kernel(LevelD<T> C, LevelD<T> F, const double *__restri
 // are formed, as in residual_restrict_tf_kernel; a cell on a mirror boundary
 // is formed whichever its colour), with the block sums of b when asked.
 // One coarse cell per work item; r is not stored.
-template <typename T>
-__global__ void residual_restrict_kernel(LevelD<T> C, LevelD<T> F, double *__restrict__ partials) {
+// SPL: the fine level is colour-split (with stored coefficients)
+template <typename T, bool SPL = false>
+__global__ void residual_restrict_kernel(LevelD<T> C, LevelD<T> F, double *__restrict__ partials, uint32_t half = 0) {
     __shared__ double sh[RB / 64];
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     double v = 0.0;
@@ -721,7 +835,23 @@ __global__ void residual_restrict_kernel(LevelD<T> C, LevelD<T> F, double *__res
             const bool even = (((q & 1) + ((q >> 1) & 1) + (q >> 2)) & 1) == 0;
             if (even || (mx && (i == 0 || i == F.nx - 1)) || (my && (j == 0 || j == F.ny - 1)) ||
                 (mz && (k == 0 || k == F.nz - 1)))
-                s += F.b[lidx(F, i, j, k)] - applyA(F, F.phi, i, j, k);
+            {
+                if constexpr (SPL) {
+                    auto at = [&](int a, int b, int c) { return split_at(half, a, b, c, lidx(F, a, b, c)); };
+                    const uint32_t nx1 = F.nx + 1, ny1 = F.ny + 1, row = (uint32_t)j + (uint32_t)F.ny * k;
+                    const T c = F.phi[at(i, j, k)];
+                    const T dxp = F.phi[at(wrapc(i + 1, F.nx, F.bcx), j, k)] - c, dxm = F.phi[at(wrapc(i - 1, F.nx, F.bcx), j, k)] - c;
+                    const T dyp = F.phi[at(i, wrapc(j + 1, F.ny, F.bcy), k)] - c, dym = F.phi[at(i, wrapc(j - 1, F.ny, F.bcy), k)] - c;
+                    const T dzp = F.phi[at(i, j, wrapc(k + 1, F.nz, F.bcz))] - c, dzm = F.phi[at(i, j, wrapc(k - 1, F.nz, F.bcz))] - c;
+                    const T *cx = F.cx + ((uint32_t)i + nx1 * row), *cy = F.cy + ((uint32_t)i + (uint32_t)F.nx * ((uint32_t)j + ny1 * k));
+                    const T *cz = F.cz + lidx(F, i, j, k);
+                    const T ax = (cx[1] * dxp + cx[0] * dxm) * F.ix2, ay = (cy[F.nx] * dyp + cy[0] * dym) * F.iy2;
+                    const T az = (cz[(uint32_t)F.nx * (uint32_t)F.ny] * dzp + cz[0] * dzm) * F.iz2;
+                    s += F.b[at(i, j, k)] - ((ax + ay) + az);
+                } else {
+                    s += F.b[lidx(F, i, j, k)] - applyA(F, F.phi, i, j, k);
+                }
+            }
         }
         const T bval = s * T(1.0 / 8);
         C.b[t] = bval;
@@ -1237,6 +1367,9 @@ struct MGPlan {
     int nlev = 0;
     bool gen0 = false;  // the finest level's coefficients from the terrain metrics (FP64 red-black)
     int kc0 = RBC_KC;   // levels per chunk of its kernels
+    bool gen1 = false;  // the level below likewise
+    int kc1 = RBC_KC;
+    double *tab1 = nullptr;  // TFChain2's
     TFM<double> gm{};
     bool gen0f = false;  // likewise in FP32 (FP32 Jacobi V-cycle)
     TFM<float> gmf{};
@@ -1244,9 +1377,9 @@ struct MGPlan {
     // the pending mean of a coarse level's b in a red-black cycle (set by the
     // level above for the cycle's visit, null otherwise)
     const double *bmL[24] = {};
-    // the colour split of the finest φ and b (SplitMap::half; 0: natural), on
-    // during an FP64 terrain PCG solve
-    uint32_t half0 = 0;
+    // the colour split of the finest φ and b and, with gen1, of the next level's
+    // (SplitMap::half; 0: natural), on during an FP64 terrain PCG solve
+    uint32_t half0 = 0, half1 = 0;
     // every cell of every level has a non-vanishing diagonal
     bool open = false;
     int bcx, bcy, bcz, nu1, nu2, smoother, prec;  // prec 0 double, 1 float
@@ -1381,25 +1514,30 @@ static void smooth(MGPlan *P, hipStream_t st, int l, int nsweeps, bool from_zero
     if (P->smoother == 0) {
         dim3 g(((h.nx + 1) / 2 + RB - 1) / RB, h.ny, h.nz);
         const bool gen = sizeof(T) == 8 && l == 0 && P->gen0;
+        const bool gen1 = sizeof(T) == 8 && l == 1 && P->half1;
         for (int s = 0; s < nsweeps; s++)
             for (int colour = 0; colour <= 1; colour++) {
                 ProfScope ps(tag);
-                if (gen) {
-                    const dim3 gr((h.nx + 63) / 64, (h.ny + RBC_BY - 1) / RBC_BY, (h.nz + P->kc0 - 1) / P->kc0);
+                if (gen || gen1) {
+                    const int kc = gen ? P->kc0 : P->kc1;
+                    const dim3 gr((h.nx + 63) / 64, (h.ny + RBC_BY - 1) / RBC_BY, (h.nz + kc - 1) / kc);
                     const int nb = (int)(gr.x * gr.y * gr.z);
                     const bool zero = from_zero && s == 0;
                     const bool sums = sum_nb && s == nsweeps - 1 && colour == 1;
                     auto launch = [&](auto kern) {
-                        hipLaunchKernelGGL(kern, gr, dim3(64, RBC_BY), 0, st, devlevel<double>(P, 0), P->gm, colour, P->kc0,
-                                           (int)(zero && colour == 1), P->part, nb, P->half0);
+                        hipLaunchKernelGGL(kern, gr, dim3(64, RBC_BY), 0, st, devlevel<double>(P, l), P->gm, (const double *)P->tab1, colour, kc,
+                                           (int)(zero && colour == 1), P->part, nb, gen ? P->half0 : P->half1);
                     };
-                    if (sums) {
+                    if (gen1) {
+                        if (zero && colour == 0) launch(rbgs_tf_kernel<true, false, TFChain2>);
+                        else launch(rbgs_tf_kernel<false, false, TFChain2>);
+                    } else if (sums) {
                         *sum_nb = nb;
-                        launch(rbgs_tf_kernel<false, true>);
+                        launch(rbgs_tf_kernel<false, true, TFChain<double>>);
                     } else if (zero && colour == 0) {
-                        launch(rbgs_tf_kernel<true, false>);
+                        launch(rbgs_tf_kernel<true, false, TFChain<double>>);
                     } else {
-                        launch(rbgs_tf_kernel<false, false>);
+                        launch(rbgs_tf_kernel<false, false, TFChain<double>>);
                     }
                 } else {
                     // the generic sweep: a pending b mean (bmL), the first pass
@@ -1448,8 +1586,7 @@ static bool coarse_fold(const MGPlan *P, int l) {
     return sizeof(T) == 8 && P->prec == 0 && !rb_cycle(P) && !P->wcycle && P->smoother == 0 && l >= 1 && 33 + 2 * l < MG_NSCAL;
 }
 
-static int prolong_chunk(const MGPlan *P) {
-    const MGLevelH &h = P->L[0];
+static int prolong_chunk(const MGLevelH &h) {
     return chunk_levels(((h.nx + 63) / 64) * ((h.ny + PRC_BY - 1) / PRC_BY), h.nz, PRC_KC, PRC_FILL, 2, 2);
 }
 
@@ -1461,7 +1598,7 @@ static int prolong(MGPlan *P, hipStream_t st, int l, const double *pre_m, const 
     const MGLevelH &h = P->L[l];
     const LevelD<T> L = devlevel<T>(P, l), C = devlevel<T>(P, l + 1);
     if (l == 0 && h.nx % 2 == 0 && h.ny % 2 == 0 && h.nz % 2 == 0) {
-        const int kc = prolong_chunk(P);
+        const int kc = prolong_chunk(h);
         const dim3 gp((h.nx + 63) / 64, (h.ny + PRC_BY - 1) / PRC_BY, (h.nz + kc - 1) / kc);
         hipLaunchKernelGGL(prolong_col_kernel<T>, gp, dim3(64, PRC_BY), 0, st, L, C, kc, P->part, pre_m, mc);
         return (int)(gp.x * gp.y * gp.z);
@@ -1522,10 +1659,13 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
             const dim3 gr((c.nx + 31) / 32, (c.ny + RRC_BW - 1) / RRC_BW, (h.nz + P->kc0 - 1) / P->kc0);
             nb = (int)(gr.x * gr.y * gr.z);
             hipLaunchKernelGGL(residual_restrict_tf_kernel, gr, dim3(64, RRC_BW), 0, st, devlevel<double>(P, 0),
-                               devlevel<double>(P, 1), P->gm, P->kc0, part, P->half0);
+                               devlevel<double>(P, 1), P->gm, P->kc0, part, P->half0, P->half1);
         } else {
             nb = stream_blocks(nc);
-            hipLaunchKernelGGL(residual_restrict_kernel<T>, dim3(nb), dim3(RB), 0, st, C, L, part);
+            if (l == 1 && P->half1)
+                hipLaunchKernelGGL((residual_restrict_kernel<T, true>), dim3(nb), dim3(RB), 0, st, C, L, part, P->half1);
+            else
+                hipLaunchKernelGGL((residual_restrict_kernel<T>), dim3(nb), dim3(RB), 0, st, C, L, part, 0u);
         }
         if (last) {
             P->bmL[l + 1] = P->scal + 32 + 2 * (l + 1);
@@ -1533,10 +1673,11 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
         }
         for (int rec = 0; rec < (P->wcycle ? 2 : 1); rec++) vcycle<T>(P, st, l + 1, rec == 0);
         P->bmL[l + 1] = nullptr;
-        if (gen) {
-            const int kc = prolong_chunk(P);
+        if (gen || (l == 1 && P->half1)) {
+            const int kc = prolong_chunk(h);
             hipLaunchKernelGGL(prolong_tf_kernel, dim3((c.nx + 63) / 64, (h.ny + PRC_BY - 1) / PRC_BY, (h.nz + kc - 1) / kc),
-                               dim3(64, PRC_BY), 0, st, devlevel<double>(P, 0), devlevel<double>(P, 1), kc, P->half0);
+                               dim3(64, PRC_BY), 0, st, devlevel<double>(P, l), devlevel<double>(P, l + 1), kc,
+                               l == 0 ? P->half0 : P->half1, l == 0 ? P->half1 : 0u);
         } else {
             prolong<T>(P, st, l, nullptr, nullptr);
         }
@@ -1744,7 +1885,7 @@ void mg_destroy(MGPlan *P) {
     }
     hipFree(P->cx64); hipFree(P->cy64); hipFree(P->cz64); hipFree(P->rhs_scale);
     hipFree(P->x); hipFree(P->r); hipFree(P->z); hipFree(P->p); hipFree(P->Ap);
-    hipFree(P->part); hipFree(P->part2); hipFree(P->scal);
+    hipFree(P->part); hipFree(P->part2); hipFree(P->scal); hipFree(P->tab1);
     delete P;
 }
 
@@ -2006,8 +2147,9 @@ int mg_pcg_solve_op(MGPlan *P, hipStream_t st, const FCGOp &op, double *xout, co
     // the FP64 terrain preconditioner keeps its finest φ and b colour-split for
     // the solve (a level with a coarser one has even extents)
     P->half0 = P->gen0 && P->nlev > 1 ? (uint32_t)(n / 2) : 0u;
+    P->half1 = P->half0 && P->gen1 ? (uint32_t)((size_t)P->L[1].nx * P->L[1].ny * P->L[1].nz / 2) : 0u;
     const int status = pcg_run(P, st, &op, tol, bnorm, maxit, &iters, &rnorm);
-    P->half0 = 0;
+    P->half0 = P->half1 = 0;
     mean_to<double>(P, st, P->x, n, 13);
     const double mx = read_scal(st, P->scal + 13);
     hipLaunchKernelGGL(shift_copy_kernel, dim3(stream_blocks(n)), dim3(RB), 0, st, xout, (const double *)P->x, n, mx);
@@ -2041,6 +2183,30 @@ void mg_set_terrain_coef(MGPlan *P, const TFWView &v) {
     P->open = P->open || dims;
     P->gen0 = dims && P->prec == 0 && P->smoother == 0 && (P->nlev == 1 || (P->nu1 >= 1 && P->nu2 >= 1));
     P->kc0 = chunk_levels(((v.Nx + 63) / 64) * ((v.Ny + RBC_BY - 1) / RBC_BY), v.Nz, RBC_KC, RBC_FILL, 3, 2);
+    // the next level's sweeps likewise, with its φ and b colour-split, where
+    // its coefficients, φ and b (40 B a cell) would stream from memory. A pass
+    // at 256×256×128 (336 MB, past the 256 MB of the Infinity Cache): 86 us with
+    // the stored coefficients, 36 from the metrics (and the transfers
+    // below it 133 → 87 us); at 160×128×80 (66 MB) 14.4 and 13.9; at 108×100×76
+    // (33 MB) 8.4 and 10.6, where the chunks' table costs more than it saves.
+    const int nx1 = v.Nx / 2, ny1 = v.Ny / 2, nz1 = v.Nz / 2;
+    P->gen1 = false;
+    hipFree(P->tab1);
+    P->tab1 = nullptr;
+    if (P->gen0 && P->nlev > 2 && (size_t)nx1 * ny1 * nz1 >= TFC_MIN) {
+        P->kc1 = chunk_levels(((nx1 + 63) / 64) * ((ny1 + RBC_BY - 1) / RBC_BY), nz1, RBC_KC, RBC_FILL, 3, 2);
+        const int nch = (nz1 + P->kc1 - 1) / P->kc1;
+        const size_t n = (size_t)(nx1 + 1) * (ny1 + 1) * (TFC_Q + TFC_V * (size_t)nch);
+        if (hipMalloc(&P->tab1, sizeof(double) * n) == hipSuccess) {
+            const LevelD<double> L = devlevel<double>(P, 1);
+            hipLaunchKernelGGL(tf_table_kernel, dim3((nx1 + 64) / 64, ny1 + 1, nch), dim3(64), 0, 0, P->tab1, P->gm, nx1,
+                               ny1, P->kc1, L.ix2, L.iy2, L.iz2);
+            P->gen1 = hipDeviceSynchronize() == hipSuccess;
+        } else {
+            P->tab1 = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     P->gen0f = dims && P->prec == 1 && P->smoother == 1;
 }
 
