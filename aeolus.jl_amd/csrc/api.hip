@@ -2046,12 +2046,6 @@ struct aeo_mw_stepper {
     double *Wc = nullptr, *Wf = nullptr, *thf = nullptr;  // device, Nz + 2H
 };
 
-template <typename T>
-__global__ void combine_kernel(T *__restrict__ f, const T *__restrict__ a, T ca, T cb, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        f[i] = ca * a[i] + cb * f[i];
-}
-
 extern "C" int aeo_mw_stepper_create(aeo_grid *g, const aeo_mw_params *sp, const double *Wc, const double *Wf,
                                      const double *thetabar_f, aeo_poisson *solver, aeo_mw_stepper **out) {
     NEED_CTX();
@@ -2107,7 +2101,7 @@ extern "C" int aeo_mw_stepper_destroy(aeo_mw_stepper *h) {
 }
 
 template <typename T>
-static int mw_step(aeo_mw_stepper *h, T *u, T *v, T *w, T *th, T *p, double dt) {
+static int mw_step(aeo_mw_stepper *h, T *u, T *v, T *w, T *th, T *p, double dt, double ca = 0.0, double cb = 1.0) {
     aeo_grid *g = h->g;
     const aeo_mw_params &sp = h->sp;
     hipStream_t st = g_ctx->stream;
@@ -2115,10 +2109,12 @@ static int mw_step(aeo_mw_stepper *h, T *u, T *v, T *w, T *th, T *p, double dt) 
     T *us = (T *)h->us, *vs = (T *)h->vs, *ws = (T *)h->ws, *tn = (T *)h->tn;
     {
         Timed t("halo");
-        launch_halo<T>(st, u, Nx, Ny, Nz, H, LOC_FX, sp.bc_x, sp.bc_y, sp.bc_z);
-        launch_halo<T>(st, v, Nx, Ny, Nz, H, LOC_FY, sp.bc_x, sp.bc_y, sp.bc_z);
-        launch_halo<T>(st, w, Nx, Ny, Nz, H, LOC_FZ, sp.bc_x, sp.bc_y, sp.bc_z);
-        launch_halo<T>(st, th, Nx, Ny, Nz, H, LOC_CC, sp.tbc_x, sp.tbc_y, sp.tbc_z);
+        HaloSet<T> hs{};
+        hs.add(u, LOC_FX, sp.bc_x, sp.bc_y, sp.bc_z);
+        hs.add(v, LOC_FY, sp.bc_x, sp.bc_y, sp.bc_z);
+        hs.add(w, LOC_FZ, sp.bc_x, sp.bc_y, sp.bc_z);
+        hs.add(th, LOC_CC, sp.tbc_x, sp.tbc_y, sp.tbc_z);
+        launch_halo_multi<T>(st, hs, Nx, Ny, Nz, H);
     }
     MWPhys ph{sp.nu, dt, sp.g_accel, sp.flux_bot * (1 / g->dz), sp.flux_top * (1 / g->dz), sp.buoyancy,
               h->fcor, h->spg};
@@ -2150,25 +2146,44 @@ static int mw_step(aeo_mw_stepper *h, T *u, T *v, T *w, T *th, T *p, double dt) 
         hs.add(ws, LOC_FZ, sp.bc_x, sp.bc_y, sp.bc_z);
         launch_halo_multi<T>(st, hs, Nx, Ny, Nz, H);
     }
-    {
-        Timed t("divergence");
-        launch_wdiv<T>(st, g->m64, h->solver->src, (T *)nullptr, us, vs, ws, h->Wc, h->Wf, 0);
+    bool fused = false;
+    if (h->solver->kind == 1) {
+        // the column solver forms the divergence inside its forward row
+        // transform (-1, nothing launched, where x is not periodic)
+        Timed t("poisson");
+        fused = spectral_column_solve_wdiv<T>(h->solver->sp, st, h->solver->phi, us, vs, ws, h->Wc, h->Wf, g->m64) == 0;
+        if (fused) {
+            HIPCHK(hipGetLastError());
+            h->solver->iters = 0;
+            h->solver->resid = NAN;
+            h->solver->status = AEO_DIRECT;
+        }
     }
-    int rc = poisson_run(h->solver, h->solver->phi);
-    if (rc) return rc;
+    if (!fused) {
+        {
+            Timed t("divergence");
+            launch_wdiv<T>(st, g->m64, h->solver->src, (T *)nullptr, us, vs, ws, h->Wc, h->Wf, 0);
+        }
+        int rc = poisson_run(h->solver, h->solver->phi);
+        if (rc) return rc;
+    }
     {
         Timed t("correct");
         int bx = sp.bc_x == AEO_PERIODIC ? BC_PERIODIC : BC_NOFLUX;
         int by = sp.bc_y == AEO_PERIODIC ? BC_PERIODIC : BC_NOFLUX;
         int bz = sp.bc_z == AEO_PERIODIC ? BC_PERIODIC : BC_NOFLUX;
-        launch_correct<T>(st, u, v, w, us, vs, ws, u, v, w, h->solver->phi, p, g->m64, bx, by, bz, 0.0, 1.0, 0, dt);
+        // the Runge-Kutta combination c(x, snap) = ca·snap + cb·x of the whole storage in the same passes
+        const bool combine = ca != 0.0;
+        const T *s0 = combine ? (const T *)h->snap[0] : u, *s1 = combine ? (const T *)h->snap[1] : v;
+        const T *s2 = combine ? (const T *)h->snap[2] : w, *s3 = combine ? (const T *)h->snap[3] : th;
+        launch_correct<T>(st, u, v, w, us, vs, ws, s0, s1, s2, h->solver->phi, p, g->m64, bx, by, bz, ca, cb, combine,
+                          dt, th, tn, s3);
         ShellSet<T> ss{};
-        ss.add(u, us, u);
-        ss.add(v, vs, v);
-        ss.add(w, ws, w);
-        launch_shell<T>(st, ss, Nx, Ny, Nz, H, 0.0, 1.0);
-        dim3 grid((Nx + 255) / 256, Ny, Nz);
-        hipLaunchKernelGGL(copy_interior_kernel<T>, grid, dim3(256), 0, st, th, tn, Nx, Ny, Nz, H);
+        ss.add(u, us, s0);
+        ss.add(v, vs, s1);
+        ss.add(w, ws, s2);
+        if (combine) ss.add(th, th, s3);
+        launch_shell<T>(st, ss, Nx, Ny, Nz, H, ca, cb);
     }
     HIPCHK(hipGetLastError());
     return AEO_OK;
@@ -2244,7 +2259,7 @@ extern "C" int aeo_mw_stepper_set_sgs(aeo_mw_stepper *h, double C_s, double Pr_t
 }
 
 // step_rk3! of the sound-proof core (src/Anelastic.jl:1905-1945): three
-// mass-weighted Euler steps with the whole storage combined in between
+// mass-weighted Euler steps, the second and third combining the whole storage with the start's
 template <typename T>
 static int mw_rk3(aeo_mw_stepper *h, T *u, T *v, T *w, T *th, T *p, double dt) {
     hipStream_t st = g_ctx->stream;
@@ -2253,16 +2268,10 @@ static int mw_rk3(aeo_mw_stepper *h, T *u, T *v, T *w, T *th, T *p, double dt) {
     T *f[4] = {u, v, w, th};
     for (int q = 0; q < 4; q++) HIPCHK(hipMemcpyAsync(h->snap[q], f[q], h->n * sizeof(T), hipMemcpyDeviceToDevice, st));
     int rc;
-    if ((rc = mw_step<T>(h, u, v, w, th, p, dt))) return rc;
-    if ((rc = mw_step<T>(h, u, v, w, th, p, dt))) return rc;
-    for (int q = 0; q < 4; q++)
-        hipLaunchKernelGGL(combine_kernel<T>, dim3(1024), dim3(256), 0, st, f[q], (const T *)h->snap[q], T(0.75),
-                           T(0.25), h->n);
-    if ((rc = mw_step<T>(h, u, v, w, th, p, dt))) return rc;
     const double third = 1.0 / 3;
-    for (int q = 0; q < 4; q++)
-        hipLaunchKernelGGL(combine_kernel<T>, dim3(1024), dim3(256), 0, st, f[q], (const T *)h->snap[q], T(third),
-                           T(2 * third), h->n);
+    if ((rc = mw_step<T>(h, u, v, w, th, p, dt))) return rc;
+    if ((rc = mw_step<T>(h, u, v, w, th, p, dt, 0.75, 0.25))) return rc;
+    if ((rc = mw_step<T>(h, u, v, w, th, p, dt, third, 2 * third))) return rc;
     HIPCHK(hipGetLastError());
     return AEO_OK;
 }

@@ -239,6 +239,26 @@ template <typename T> struct DivRows {
     }
 };
 
+// likewise the rows of the W-weighted divergence of a sound-proof core
+// (wdiv_kernel's expression)
+template <typename T> struct WDivRows {
+    const T *u, *v, *w;
+    const double *Wc, *Wf;
+    Metrics<double> md;
+    __device__ __forceinline__ double2 operator()(int row, int m, int) const {
+        const int j = row % md.Ny, k = row / md.Ny;
+        const int K = k + md.H;
+        const size_t sx = md.sx, sxy = (size_t)md.sx * md.sy;
+        const size_t c = (size_t)(2 * m + md.H) + sx * ((size_t)(j + md.H) + (size_t)md.sy * K);
+        const double wc = Wc[K], wfb = Wf[K], wft = Wf[K + 1];
+        auto at = [&](size_t q) {
+            return wc * (((double)u[q + 1] - (double)u[q]) * md.idx + ((double)v[q + sx] - (double)v[q]) * md.idy) +
+                   (wft * (double)w[q + sxy] - wfb * (double)w[q]) * md.idz;
+        };
+        return make_double2(at(c), at(c + 1));
+    }
+};
+
 template <class Rows>
 __global__ void r2c_rows_kernel(double2 *__restrict__ hat, Rows rows, FFTLen f, int rpb, int nrows, int LD,
                                 const double2 *__restrict__ twN) {
@@ -873,6 +893,19 @@ template int spectral_column_solve_div<double>(SpectralPlan *, hipStream_t, doub
                                                const double *, const Metrics<double> &);
 template int spectral_column_solve_div<float>(SpectralPlan *, hipStream_t, double *, const float *, const float *,
                                               const float *, const Metrics<double> &);
+
+template <typename T>
+int spectral_column_solve_wdiv(SpectralPlan *p, hipStream_t st, double *phi, const T *u, const T *v, const T *w,
+                               const double *Wc, const double *Wf, const Metrics<double> &md) {
+    if (p->mode != 1 || p->neu_x) return -1;
+    xfwd_rows(p, st, WDivRows<T>{u, v, w, Wc, Wf, md});
+    column_tail(p, st, phi);
+    return 0;
+}
+template int spectral_column_solve_wdiv<double>(SpectralPlan *, hipStream_t, double *, const double *, const double *,
+                                                const double *, const double *, const double *, const Metrics<double> &);
+template int spectral_column_solve_wdiv<float>(SpectralPlan *, hipStream_t, double *, const float *, const float *,
+                                               const float *, const double *, const double *, const Metrics<double> &);
 
 static void column_tail(SpectralPlan *p, hipStream_t st, double *phi) {
     ytrans(p, st, +1);

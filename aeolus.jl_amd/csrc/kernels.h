@@ -78,7 +78,8 @@ void launch_div_into(hipStream_t st, double *buf, const T *u, const T *v, const 
 template <typename T>
 void launch_correct(hipStream_t st, T *uo, T *vo, T *wo, const T *us, const T *vs, const T *ws, const T *u0,
                     const T *v0, const T *w0, const double *phi, T *p, const Metrics<double> &md, int bcx, int bcy,
-                    int bcz, double ca, double cb, int combine, double dt);
+                    int bcz, double ca, double cb, int combine, double dt, T *th = nullptr, const T *tn = nullptr,
+                    const T *th0 = nullptr);
 // up to four (out, x, snap) triples whose halo shells are combined in one launch
 template <typename T> struct ShellSet {
     T *out[4];
@@ -261,6 +262,10 @@ int spectral_column_solve(SpectralPlan *p, hipStream_t st, double *phi, const do
 template <typename T>
 int spectral_column_solve_div(SpectralPlan *p, hipStream_t st, double *phi, const T *u, const T *v, const T *w,
                               const Metrics<double> &md);
+// the same for the W-weighted divergence of a sound-proof core
+template <typename T>
+int spectral_column_solve_wdiv(SpectralPlan *p, hipStream_t st, double *phi, const T *u, const T *v, const T *w,
+                               const double *Wc, const double *Wf, const Metrics<double> &md);
 
 // A profile scope on the library stream (api.hip): with profiling on and a
 // name, events bracket the launches made inside the scope and their time is

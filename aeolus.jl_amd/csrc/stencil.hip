@@ -931,7 +931,7 @@ template void launch_div_into<float>(hipStream_t, double *, const float *, const
 // ---------------------------------------------------------------------------
 // _b_correct! (src/FiniteVolume.jl:1823-1833) with the stage combination
 // c(x, snap) = a·snap + b·x (src/Simulations.jl:1192-1194) and p = φ/Δt. φ
-// is the solver's interior-sized FP64 solution; its halo (the velocity BCs
+// is the solver's interior-sized FP64 solution; with th, θ = c(tn, th0) too. φ's halo (the velocity BCs
 // at a cell centre: periodic wrap or mirror) is read through the index map.
 // ---------------------------------------------------------------------------
 template <typename T>
@@ -939,7 +939,8 @@ __global__ void correct_kernel(T *uo, T *vo, T *wo,
                                const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
                                const T *u0, const T *v0, const T *w0,
                                const double *__restrict__ phi, T *__restrict__ p, Metrics<double> md, int bcx,
-                               int bcy, int bcz, double ca, double cb, int combine, double dt) {
+                               int bcy, int bcz, double ca, double cb, int combine, double dt, T *th, const T *tn,
+                               const T *th0) {
     const int H = md.H, sx = md.sx, sy = md.sy, Nx = md.Nx, Ny = md.Ny, Nz = md.Nz;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int j = blockIdx.y, k = blockIdx.z;
@@ -966,22 +967,25 @@ __global__ void correct_kernel(T *uo, T *vo, T *wo,
     vo[c] = (T)vn;
     wo[c] = (T)wn;
     if (p) p[c] = (T)(pc / dt);
+    if (th) th[c] = combine ? (T)(ca * (double)th0[c] + cb * (double)tn[c]) : tn[c];
 }
 
 template <typename T>
 void launch_correct(hipStream_t st, T *uo, T *vo, T *wo, const T *us, const T *vs, const T *ws, const T *u0,
                     const T *v0, const T *w0, const double *phi, T *p, const Metrics<double> &md, int bcx, int bcy,
-                    int bcz, double ca, double cb, int combine, double dt) {
+                    int bcz, double ca, double cb, int combine, double dt, T *th, const T *tn, const T *th0) {
     dim3 grid((md.Nx + 255) / 256, md.Ny, md.Nz);
     hipLaunchKernelGGL(correct_kernel<T>, grid, dim3(256), 0, st, uo, vo, wo, us, vs, ws, u0, v0, w0, phi, p, md, bcx,
-                       bcy, bcz, ca, cb, combine, dt);
+                       bcy, bcz, ca, cb, combine, dt, th, tn, th0);
 }
 template void launch_correct<double>(hipStream_t, double *, double *, double *, const double *, const double *,
                                      const double *, const double *, const double *, const double *, const double *,
-                                     double *, const Metrics<double> &, int, int, int, double, double, int, double);
+                                     double *, const Metrics<double> &, int, int, int, double, double, int, double,
+                                     double *, const double *, const double *);
 template void launch_correct<float>(hipStream_t, float *, float *, float *, const float *, const float *,
                                     const float *, const float *, const float *, const float *, const double *,
-                                    float *, const Metrics<double> &, int, int, int, double, double, int, double);
+                                    float *, const Metrics<double> &, int, int, int, double, double, int, double,
+                                    float *, const float *, const float *);
 
 // ---------------------------------------------------------------------------
 // The RK3 combination of the halo shell, out = a·snap + b·x at every storage
