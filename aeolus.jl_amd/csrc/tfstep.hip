@@ -712,30 +712,6 @@ __global__ void tfw_div_kernel(double *__restrict__ out, const double *__restric
     out[op.o(a, b, c)] = ((FE - FW) * m.idx + (FN - FS) * m.idy) + (Omv[1] - Omv[0]) * m.idz;
 }
 
-// u = c(u0, u* − Gxφ), v, w (interior σ-faces); θ = θ'; p = φ/Δt (p nullable)
-__global__ void tfw_correct_kernel(double *__restrict__ u, double *__restrict__ v, double *__restrict__ w,
-                                   double *__restrict__ th, double *__restrict__ p, const double *__restrict__ us,
-                                   const double *__restrict__ vs, const double *__restrict__ ws,
-                                   const double *__restrict__ tn, const double *__restrict__ u0,
-                                   const double *__restrict__ v0, const double *__restrict__ w0,
-                                   const double *__restrict__ phi, TFOp op, double dt, double ca, double cb,
-                                   int combine) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y, c = blockIdx.z;
-    if (a >= op.nx) return;
-    const TFM<double> &m = op.m;
-    const uint32_t s = lin(a + m.H, b + m.H, c + m.H, m.sx, m.sy);
-    const double un = us[s] - op.Gx(phi, a, b, c);
-    const double vn = vs[s] - op.Gy(phi, a, b, c);
-    u[s] = combine ? ca * u0[s] + cb * un : un;
-    v[s] = combine ? ca * v0[s] + cb * vn : vn;
-    if (c > 0) {
-        const double wn = ws[s] - op.Gw(phi, a, b, c);
-        w[s] = combine ? ca * w0[s] + cb * wn : wn;
-    }
-    if (th) th[s] = tn[s];
-    if (p) p[s] = phi[op.o(a, b, c)] / dt;
-}
-
 // block maxima of |b|/(ρ_c J) over an interior-sized vector (NaN propagates)
 __global__ void __launch_bounds__(256) tfw_absdiv_kernel(double *__restrict__ part, const double *__restrict__ b,
                                                          TFOp op) {
@@ -762,9 +738,10 @@ __global__ void __launch_bounds__(256) tfw_absdiv_kernel(double *__restrict__ pa
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// the correction by columns: thread (a, b) marches CH levels with rolling
-// windows of φ on its own, west and south columns and of their metric terms
-// S; the same G as tfw_correct_kernel without its recomputation
+// u = c(u0, u* − Gxφ), v, w (interior σ-faces); θ = θ'; p = φ/Δt (p nullable),
+// by columns: thread (a, b) marches CH levels with rolling windows of φ on its
+// own, west and south columns and of their metric terms S; the same G as
+// tfw_grad_kernel without its recomputation
 template <int CH>
 __global__ void __launch_bounds__(256) tfw_correct_march_kernel(
     double *__restrict__ u, double *__restrict__ v, double *__restrict__ w, double *__restrict__ th,

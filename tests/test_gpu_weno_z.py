@@ -1,5 +1,5 @@
-"""WENO-Z5 from differences, with the three weights' ratios from one reciprocal
-(FP64), at the ends of its range, against the oracle's form from the values.
+"""WENO-Z5 and Z7 from differences, with the weights' ratios from one reciprocal
+per three or two (FP64), at the ends of their range, against the oracle's form from the values.
 
 Each of the two forms rounds the smoothness indicators and candidates a few
 times (about 10 roundings of 1.1e-16 of the largest stencil value each, times
@@ -19,7 +19,7 @@ from helpers import rel_err
 pytestmark = pytest.mark.gpu
 
 
-def _case(orc, hip, phi, n=(70, 21, 13), H=3):
+def _case(orc, hip, phi, scheme, n=(70, 21, 13), H=4):
     g, og = hip.Grid(n, (3.0, 1.0, 2.0), halo=H), orc.Grid(n, (3.0, 1.0, 2.0), halo=H)
     rng = np.random.default_rng(3)
     up = hip.DeviceArray.from_numpy
@@ -30,15 +30,16 @@ def _case(orc, hip, phi, n=(70, 21, 13), H=3):
         vel.append(a)
     f = phi(rng, og.storage)
     orc.fill_halos(og, f, orc.CC, ("periodic",) * 3)
-    ref = orc.advect_scalar(og, og.zeros(), *vel, f, "weno_z5")
+    ref = orc.advect_scalar(og, og.zeros(), *vel, f, scheme)
     t = up(og.zeros())
-    hip.advection_scheme("weno_z5", g)(t, *[up(a) for a in vel], up(f))
+    hip.advection_scheme(scheme, g)(t, *[up(a) for a in vel], up(f))
     return t.download()[og.interior], ref[og.interior]
 
 
+@pytest.mark.parametrize("scheme", ["weno_z5", "weno_z7"])
 @pytest.mark.parametrize("scale", [2.0**-83, 2.0**-53, 1.0, 2.0**40, 2.0**133])
 @pytest.mark.parametrize("kind", ["noise", "steps", "offset"])
-def test_scales(hip, orc, scale, kind):
+def test_scales(hip, orc, scale, kind, scheme):
     def phi(rng, s):
         a = rng.standard_normal(s)
         if kind == "steps":  # flat stretches (every indicator 0) and jumps
@@ -46,17 +47,18 @@ def test_scales(hip, orc, scale, kind):
         if kind == "offset":  # a mean far above the variation
             a = 300.0 + 0.1 * a
         return np.asfortranarray(scale * a)
-    got, ref = _case(orc, hip, phi)
+    got, ref = _case(orc, hip, phi, scheme)
     assert np.abs(ref).max() > 0 and rel_err(got, ref) < 1e-12
 
 
+@pytest.mark.parametrize("scheme", ["weno_z5", "weno_z7"])
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
-def test_a_bad_cell_stays_in_its_stencils(hip, orc, bad):
+def test_a_bad_cell_stays_in_its_stencils(hip, orc, bad, scheme):
     def phi(rng, s):
         a = np.asfortranarray(rng.standard_normal(s))
         a[30, 10, 8] = bad
         return a
-    got, ref = _case(orc, hip, phi)
+    got, ref = _case(orc, hip, phi, scheme)
     assert np.array_equal(np.isfinite(got), np.isfinite(ref))
     ok = np.isfinite(ref)
     assert rel_err(got[ok], ref[ok]) < 1e-12
