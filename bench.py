@@ -707,13 +707,13 @@ def main():
     # the dominant kernel of the headline form: the finest level's red-black
     # colour pass of the FP64 V-cycle, which evaluates the face coefficients
     # from the terrain metrics. Algorithmic bytes per launch: the elements a
-    # colour pass cannot avoid, every φ (the colour's cells and their
-    # neighbours) read, the colour's half of b read and its half of φ written
-    # (2 × 8 B per cell; with φ and b stored colour-split the pass moves no
-    # more); beside it the VALU issue of its FP64 arithmetic
+    # colour pass cannot avoid, the other colour's half of φ and the colour's
+    # half of b read and its half of φ written (3 × 4 B per cell; φ and b are
+    # stored colour-split, a cell's own old value is not read); beside it the
+    # VALU issue of its FP64 arithmetic
     rb = head["by_phase"]["mg_rbgs_f64_l0"]
     avg_s = rb["ms_per_launch"] / 1e3
-    alg = 2 * 8 * cells
+    alg = 3 * 4 * cells
     achieved = alg / avg_s / 1e9
     valu = read_terrain_valu()
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
