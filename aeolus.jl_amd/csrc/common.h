@@ -187,34 +187,29 @@ template <typename T> __device__ __forceinline__ T b5_m4(T v1, T v2, T v3, T v4,
                     div24<T>((((v1 - T(4) * v2) + T(6) * v3) - T(4) * v4) + v5));
 }
 
-// The three ratios t_k = τ/b_k of the Z weights. FP64: one reciprocal, of the
-// product (b ≥ 4ε² = 2e-31, so the product is at least 8e-93, and finite for
-// fields below 1e50), and five products in place of two more refined
-// reciprocals; each ratio is within 5 roundings. FP32 has no such range:
-// three hardware reciprocals.
-template <typename T>
-__device__ __forceinline__ void z_ratios(T tau, T b0, T b1, T b2, T &t0, T &t1, T &t2) {
-    if constexpr (sizeof(T) == 8) {
-        const T b01 = b0 * b1, r = qdiv<T>(tau, b01 * b2);
-        t0 = (b1 * b2) * r;
-        t1 = (b0 * b2) * r;
-        t2 = b01 * r;
-    } else {
-        t0 = qdiv<T>(tau, b0);
-        t1 = qdiv<T>(tau, b1);
-        t2 = qdiv<T>(tau, b2);
-    }
+// 2^(K − e) from the high word of a double m·2^e, 1 ≤ m < 2 (positive, below 2^1022)
+template <int K> __device__ __forceinline__ double pow2_over(int hi) {
+    return __hiloint2double(0x7fe00000 + (K << 20) - (hi & 0x7ff00000), 0);
 }
 
 // _weno_z5_left, src/AdvectionSchemes.jl:240-255, from the differences
 // e_m = v_{m+1} − v_m: the smoothness indicators (times 4, with ε² times 4)
 // and the candidates less v3 (times 6) depend on nothing else, and the face is
-// v3 + Σ a_k (6 (q_k − v3)) / (6 Σ a_k). The reconstruction bounds the
-// advection kernels: of the tiled FP64 kernel's VALU instructions per
-// wave and level this form leaves 1143 where the indicators and candidates
-// from the values, each ratio by its own reciprocal, took 1439; it rounds
-// relative to the variation, not the value. 256×256×128 RK3 stage 606 → 506 us
-// (FP32 289 → 265), the limited tracer's two passes 316 → 278.
+// v3 + Σ a_k (6 (q_k − v3)) / (6 Σ a_k); it rounds relative to the variation,
+// not the value.
+// FP64: the weights a_k = g_k (1 + (τ/b_k)²) times (b0 b1 b2)², so that only
+// the face divides. Such a product of indicators would end at variations of
+// 1e51, so they are first scaled to 2^80 by the larger of b0 and b2 (b1 is at
+// most 5.4 times it), and no sum passes 1e151. Where one is so small that the
+// product vanishes, τ is either at least 2^-53 of the larger one, and the
+// weight of the small one, without the product, is what counts, or zero, and
+// the weights are the linear ones (w = 1). The range is that of one division
+// per ratio: ratios whose square is finite. FP32: three hardware reciprocals.
+// The reconstruction bounds the advection kernels. 256×256×128 RK3 stage with
+// the indicators and candidates from the values 606 us, from differences 506
+// (FP32 289 → 265); the limited tracer's two passes 316 → 278. A branch from
+// one reciprocal of the product to one per ratio where it overflows: 122
+// registers spilled, the step 2.49 → 4.59 ms.
 template <int P, typename T>
 __device__ __forceinline__ T weno_z5(T v1, T v2, T v3, T v4, T v5) {
     const T e1 = v2 - v1, e2 = v3 - v2, e3 = v4 - v3, e4 = v5 - v4;
@@ -223,21 +218,33 @@ __device__ __forceinline__ T weno_z5(T v1, T v2, T v3, T v4, T v5) {
     const T c = T(13.0 / 3.0), eps = T(4) * Eps<T>::v * Eps<T>::v;
     const T b0 = f0 * f0 + ((c * s0) * s0 + eps), b1 = f1 * f1 + ((c * s1) * s1 + eps),
             b2 = f2 * f2 + ((c * s2) * s2 + eps);
-    T t0, t1, t2;
-    z_ratios<T>(fabs(b0 - b2), b0, b1, b2, t0, t1, t2);
-    const T a0 = T(1.0 / 10.0) + T(1.0 / 10.0) * ipow<P>(t0);
-    const T a1 = T(6.0 / 10.0) + T(6.0 / 10.0) * ipow<P>(t1);
-    const T a2 = T(3.0 / 10.0) + T(3.0 / 10.0) * ipow<P>(t2);
     const T p0 = T(5) * e2 - T(2) * e1, p1 = T(2) * e3 + e2, p2 = T(4) * e3 - e4;
-    return v3 + qdiv<T>((a0 * p0 + a1 * p1) + a2 * p2, T(6) * ((a0 + a1) + a2));
+    if constexpr (sizeof(T) == 8) {
+        const T r = pow2_over<80>(max(__double2hiint(b0), __double2hiint(b2)));
+        const T c0 = b0 * r, c2 = b2 * r, tau = fabs(c0 - c2), c1 = b1 * r, c02 = c0 * c2;
+        T w = ipow<P>(c02 * c1);
+        w = __hiloint2double(tau == T(0) ? 0x3ff00000 : __double2hiint(w), __double2loint(w));
+        const T tc = tau * c1, z0 = w + ipow<P>(tc * c2), z1 = w + ipow<P>(tau * c02), z2 = w + ipow<P>(tc * c0);
+        const T a1 = T(6) * z1, a2 = T(3) * z2;
+        return v3 + qdiv<T>((z0 * p0 + a1 * p1) + a2 * p2, T(6) * ((z0 + a1) + a2));
+    } else {
+        const T tau = fabs(b0 - b2);
+        const T a0 = T(1.0 / 10.0) + T(1.0 / 10.0) * ipow<P>(qdiv<T>(tau, b0));
+        const T a1 = T(6.0 / 10.0) + T(6.0 / 10.0) * ipow<P>(qdiv<T>(tau, b1));
+        const T a2 = T(3.0 / 10.0) + T(3.0 / 10.0) * ipow<P>(qdiv<T>(tau, b2));
+        return v3 + qdiv<T>((a0 * p0 + a1 * p1) + a2 * p2, T(6) * ((a0 + a1) + a2));
+    }
 }
 // _weno_z7_left, src/AdvectionSchemes.jl:284-303, from the differences like
 // weno_z5: 36 b_k = D_k² + 39 B_k² + 39.05 C_k² with D_k six times the slope
 // plus a quarter, B_k the second and C_k the third differences of the
 // candidate's four cells (beta4's form with its square completed), and the
-// candidates less v4 times 12. FP64: a reciprocal per two indicators (fields
-// below 1e75), FP32 one each. At 187×141×75 32.6 → 25.5 us in FP32,
-// 62.6 → 48.3 in FP64.
+// candidates less v4 times 12. FP64: a reciprocal per two indicators, one of
+// each pair and τ scaled by the larger of b0 and b2 so that their product
+// stays in range; where it would vanish, 1e-307 in its place leaves the pair's
+// ratio to each other, and both far above the other pair's (or τ zero). FP32:
+// one reciprocal each. At 187×141×75 32.6 → 24.6 us in FP32, 62.6 → 49.7 in
+// FP64 (48.6 without the scaling, finite up to 1e75 only).
 template <int P, typename T>
 __device__ __forceinline__ T weno_z7(T v1, T v2, T v3, T v4, T v5, T v6, T v7) {
     const T e1 = v2 - v1, e2 = v3 - v2, e3 = v4 - v3, e4 = v5 - v4, e5 = v6 - v5, e6 = v7 - v6;
@@ -253,15 +260,18 @@ __device__ __forceinline__ T weno_z7(T v1, T v2, T v3, T v4, T v5, T v6, T v7) {
     const T tau = fabs(((b0 - b1) - b2) + b3);
     T t0, t1, t2, t3;
     if constexpr (sizeof(T) == 8) {
-        const T r = qdiv<T>(tau, b0 * b1), q = qdiv<T>(tau, b2 * b3);
+        const T n = pow2_over<0>(max(__double2hiint(b0), __double2hiint(b2))), taun = tau * n;
+        const T r = qdiv<T>(taun, fma(b0 * n, b1, T(1e-307))), q = qdiv<T>(taun, fma(b2 * n, b3, T(1e-307)));
         t0 = b1 * r; t1 = b0 * r;
         t2 = b3 * q; t3 = b2 * q;
     } else {
         t0 = qdiv<T>(tau, b0); t1 = qdiv<T>(tau, b1);
         t2 = qdiv<T>(tau, b2); t3 = qdiv<T>(tau, b3);
     }
-    const T a0 = T(1.0 / 35.0) + T(1.0 / 35.0) * ipow<P>(t0), a1 = T(12.0 / 35.0) + T(12.0 / 35.0) * ipow<P>(t1);
-    const T a2 = T(18.0 / 35.0) + T(18.0 / 35.0) * ipow<P>(t2), a3 = T(4.0 / 35.0) + T(4.0 / 35.0) * ipow<P>(t3);
+    // the weights over 16: twelve times their sum is then below what a ratio's square reaches
+    const T g0 = T(1.0 / 560.0), g1 = T(12.0 / 560.0), g2 = T(18.0 / 560.0), g3 = T(4.0 / 560.0);
+    const T a0 = g0 + g0 * ipow<P>(t0), a1 = g1 + g1 * ipow<P>(t1);
+    const T a2 = g2 + g2 * ipow<P>(t2), a3 = g3 + g3 * ipow<P>(t3);
     const T p0 = T(13) * e3 + (T(3) * e1 - T(10) * e2), p1 = T(3) * e4 + (T(4) * e3 - e2);
     const T p2 = T(6) * e4 + (e3 - e5), p3 = T(9) * e4 + (e6 - T(4) * e5);
     return v4 + qdiv<T>(((a0 * p0 + a1 * p1) + a2 * p2) + a3 * p3, T(12) * (((a0 + a1) + a2) + a3));
