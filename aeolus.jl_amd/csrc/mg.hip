@@ -642,13 +642,14 @@ __global__ void __launch_bounds__(64 * RRC_BW) residual_restrict_tf_kernel(Level
 // which column holds colour 1 on a level is uniform. The x-y part of the
 // weights is summed once per coarse level, for the pair's left and right
 // column, and kept for three coarse levels.
+// both: no smoothing follows, and every cell is corrected.
 // Bound: memory, half of φ read and written, 9 B per fine cell. At
 // 512×512×256: 258 us (both colours, one column per thread) → 142 us.
 constexpr int PRC_BY = 4;   // rows per block
 constexpr int PRC_KC = 16;  // most fine levels per chunk (even)
 constexpr int PRC_FILL = 1024;  // blocks a round (chunk_levels)
 __global__ void __launch_bounds__(64 * PRC_BY) prolong_tf_kernel(LevelD<double> F, LevelD<double> C, int kc,
-                                                                 uint32_t half, uint32_t halfc) {
+                                                                 uint32_t half, uint32_t halfc, int both) {
     const int pr = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * PRC_BY + __builtin_amdgcn_readfirstlane(threadIdx.y);
     if (pr >= C.nx || j >= F.ny) return;
     const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, F.nz);
@@ -676,9 +677,9 @@ __global__ void __launch_bounds__(64 * PRC_BY) prolong_tf_kernel(LevelD<double> 
         const double le = 0.75 * l1 + 0.25 * l0, re = 0.75 * r1 + 0.25 * r0;
         const double lo = 0.75 * l1 + 0.25 * l2, ro = 0.75 * r1 + 0.25 * r2;
         f1[s] += odd ? le : re;
-        if (mirror && k == 0) f0[s] += odd ? re : le;
+        if (both || (mirror && k == 0)) f0[s] += odd ? re : le;
         f1[s + pl] += odd ? ro : lo;
-        if (mirror && k + 2 == F.nz) f0[s + pl] += odd ? lo : ro;
+        if (both || (mirror && k + 2 == F.nz)) f0[s + pl] += odd ? lo : ro;
         s += 2 * pl;
         l0 = l1; r0 = r1; l1 = l2; r1 = r2;
     }
@@ -856,6 +857,30 @@ __global__ void residual_restrict_kernel(LevelD<T> C, LevelD<T> F, double *__res
         const T bval = s * T(1.0 / 8);
         C.b[t] = bval;
         v = (double)bval;
+    }
+    if (partials) {
+        const double sb = block_sum(v, sh);
+        if (threadIdx.x == 0) partials[blockIdx.x] = sb;
+    }
+}
+
+// coarse b = the mean of the 8 fine b, the residual of φ = 0, with its block
+// sums when asked (FP64 terrain cycle without pre-smoothing; half, halfc: the
+// levels' colour split, 0 natural)
+__global__ void restrict_rhs_kernel(LevelD<double> C, LevelD<double> F, double *__restrict__ partials, uint32_t half,
+                                    uint32_t halfc) {
+    __shared__ double sh[RB / 64];
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    double v = 0.0;
+    if (t < (uint32_t)C.nx * (uint32_t)C.ny * (uint32_t)C.nz) {
+        const uint32_t JK = t / (uint32_t)C.nx, I = t - JK * (uint32_t)C.nx, K = JK / (uint32_t)C.ny, J = JK - K * (uint32_t)C.ny;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const int i = 2 * I + (q & 1), j = 2 * J + ((q >> 1) & 1), k = 2 * K + (q >> 2);
+            v += F.b[split_at(half, i, j, k, lidx(F, i, j, k))];
+        }
+        v *= 0.125;
+        C.b[split_at(halfc, I, J, K, t)] = v;
     }
     if (partials) {
         const double sb = block_sum(v, sh);
@@ -1485,8 +1510,8 @@ static SplitMap split0(const MGPlan *P) {
     return SplitMap{sizeof(T) == 8 ? P->half0 : 0u, nx, ny, pow2 ? sx : -1, pow2 ? sy : -1};
 }
 // A red-black cycle on an open operator (no fully blocked cell) with
-// smoothing on both sides of the coarse correction leaves out what changes no
-// iterate of the CG beyond rounding:
+// smoothing on both sides of the coarse correction, or on the terrain grid
+// with any, leaves out what changes no iterate of the CG beyond rounding:
 //  - the mean removals inside the cycle: a constant is in the kernel of every
 //    level's operator, changes no residual and prolongs to a constant, and the
 //    residual and its restriction have the mean of b, which the CG keeps zero.
@@ -1497,7 +1522,13 @@ static SplitMap split0(const MGPlan *P) {
 //    the colour the next pass overwrites (residual_restrict_kernel,
 //    prolong_tf_kernel);
 //  - the clearing of φ: a cycle's first sweep starts from zero.
-static bool rb_cycle(const MGPlan *P) { return P->smoother == 0 && P->open && P->nu1 >= 1 && P->nu2 >= 1; }
+// Without post-smoothing every cell is corrected; without pre-smoothing φ is
+// zero (the terrain's cycles are V-cycles from zero) and b is restricted.
+// A CG iteration at 512×512×256 with sweeps (2, 0), (1, 0), (0, 2): 8.5, 6.7
+// and 8.5 ms through the full cycle and its stored coefficients → 3.7, 3.0, 3.4.
+static bool rb_cycle(const MGPlan *P) {
+    return P->smoother == 0 && P->open && ((P->nu1 >= 1 && P->nu2 >= 1) || (P->gen0 && !P->wcycle));
+}
 
 // m_first: a mean removal of φ still pending, folded into the first sweep
 // sums (FP64 terrain finest level): the last pass also writes the block sums
@@ -1617,7 +1648,7 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
     MGLevelH &h = P->L[l];
     const int n = h.nx * h.ny * h.nz;
     const bool cf = coarse_fold<T>(P, l);
-    const bool rb = rb_cycle(P) && P->nlev > 1;
+    const bool rb = rb_cycle(P) && P->nlev > 1 && (P->nu1 >= 1 || zero_start);
     if (l == P->nlev - 1) {
         const int own = coarsest_slots(h.nx, h.ny, h.nz, sizeof(T));
         if (own >= 0) {
@@ -1649,21 +1680,28 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
     MGLevelH &c = P->L[l + 1];
     const int nc = c.nx * c.ny * c.nz;
     if (rb) {
-        smooth<T>(P, st, l, P->nu1, zero_start);
+        if (P->nu1 >= 1) smooth<T>(P, st, l, P->nu1, zero_start);
+        else hipLaunchKernelGGL(zero_kernel<T>, dim3(stream_blocks(n)), dim3(RB), 0, st, (T *)h.phi, n);
         const bool last = l + 1 == P->nlev - 1;  // the coarsest right-hand side: its mean is left out
         const LevelD<T> L = devlevel<T>(P, l), C = devlevel<T>(P, l + 1);
         double *part = last ? P->part : nullptr;
-        const bool gen = sizeof(T) == 8 && l == 0 && P->gen0;
+        // the colour split of the levels (the finest one's transfers by the metrics take it)
+        const uint32_t half = l == 0 ? P->half0 : l == 1 ? P->half1 : 0u, halfc = l == 0 ? P->half1 : 0u;
+        const bool gen = sizeof(T) == 8 && l == 0 && half;
         int nb;
-        if (gen) {
+        if (P->nu1 == 0) {
+            nb = stream_blocks(nc);
+            hipLaunchKernelGGL(restrict_rhs_kernel, dim3(nb), dim3(RB), 0, st, devlevel<double>(P, l + 1),
+                               devlevel<double>(P, l), part, half, halfc);
+        } else if (gen) {
             const dim3 gr((c.nx + 31) / 32, (c.ny + RRC_BW - 1) / RRC_BW, (h.nz + P->kc0 - 1) / P->kc0);
             nb = (int)(gr.x * gr.y * gr.z);
             hipLaunchKernelGGL(residual_restrict_tf_kernel, gr, dim3(64, RRC_BW), 0, st, devlevel<double>(P, 0),
-                               devlevel<double>(P, 1), P->gm, P->kc0, part, P->half0, P->half1);
+                               devlevel<double>(P, 1), P->gm, P->kc0, part, half, halfc);
         } else {
             nb = stream_blocks(nc);
-            if (l == 1 && P->half1)
-                hipLaunchKernelGGL((residual_restrict_kernel<T, true>), dim3(nb), dim3(RB), 0, st, C, L, part, P->half1);
+            if (half)
+                hipLaunchKernelGGL((residual_restrict_kernel<T, true>), dim3(nb), dim3(RB), 0, st, C, L, part, half);
             else
                 hipLaunchKernelGGL((residual_restrict_kernel<T>), dim3(nb), dim3(RB), 0, st, C, L, part, 0u);
         }
@@ -1673,11 +1711,11 @@ static bool vcycle(MGPlan *P, hipStream_t st, int l, bool zero_start, bool defer
         }
         for (int rec = 0; rec < (P->wcycle ? 2 : 1); rec++) vcycle<T>(P, st, l + 1, rec == 0);
         P->bmL[l + 1] = nullptr;
-        if (gen || (l == 1 && P->half1)) {
+        if (half) {
             const int kc = prolong_chunk(h);
             hipLaunchKernelGGL(prolong_tf_kernel, dim3((c.nx + 63) / 64, (h.ny + PRC_BY - 1) / PRC_BY, (h.nz + kc - 1) / kc),
-                               dim3(64, PRC_BY), 0, st, devlevel<double>(P, l), devlevel<double>(P, l + 1), kc,
-                               l == 0 ? P->half0 : P->half1, l == 0 ? P->half1 : 0u);
+                               dim3(64, PRC_BY), 0, st, devlevel<double>(P, l), devlevel<double>(P, l + 1), kc, half, halfc,
+                               (int)(P->nu2 == 0));
         } else {
             prolong<T>(P, st, l, nullptr, nullptr);
         }
@@ -1931,10 +1969,17 @@ static void precond(MGPlan *P, hipStream_t st, const double *ap = nullptr, const
 }
 
 // the FP64 terrain cycle inside the CG: r in place as the finest right-hand
-// side (colour-split), the sums of (r·z, z, r), z = φ, from the last pass
+// side (colour-split), the sums of (r·z, z, r), z = φ, from the last pass, if there is one
 static void precond_split(MGPlan *P, hipStream_t st) {
     int nb = 0;
     vcycle<double>(P, st, 0, true, false, &nb);
+    if (nb == 0) {  // no post-smoothing
+        const MGLevelH &h = P->L[0];
+        const int n = h.nx * h.ny * h.nz;
+        nb = flat_blocks(n);
+        hipLaunchKernelGGL(store_rz_kernel<double>, dim3(nb), dim3(RB), 0, st, (double *)nullptr, (const double *)h.phi,
+                           (const double *)h.b, n, (const double *)nullptr, P->part, nb, (const double *)nullptr);
+    }
     finalize_multi_to(P, st, P->scal, P->part, nb, 3);
 }
 
@@ -2146,7 +2191,7 @@ int mg_pcg_solve_op(MGPlan *P, hipStream_t st, const FCGOp &op, double *xout, co
     int iters = 0;
     // the FP64 terrain preconditioner keeps its finest φ and b colour-split for
     // the solve (a level with a coarser one has even extents)
-    P->half0 = P->gen0 && P->nlev > 1 ? (uint32_t)(n / 2) : 0u;
+    P->half0 = P->gen0 && rb_cycle(P) && P->nlev > 1 ? (uint32_t)(n / 2) : 0u;
     P->half1 = P->half0 && P->gen1 ? (uint32_t)((size_t)P->L[1].nx * P->L[1].ny * P->L[1].nz / 2) : 0u;
     const int status = pcg_run(P, st, &op, tol, bnorm, maxit, &iters, &rnorm);
     P->half0 = P->half1 = 0;
@@ -2181,7 +2226,7 @@ void mg_set_terrain_coef(MGPlan *P, const TFWView &v) {
     P->gmf = make_tfm<float>(v);
     // ρ̄ > 0 and J > 0 on every face, so every diagonal is negative
     P->open = P->open || dims;
-    P->gen0 = dims && P->prec == 0 && P->smoother == 0 && (P->nlev == 1 || (P->nu1 >= 1 && P->nu2 >= 1));
+    P->gen0 = dims && P->prec == 0 && P->smoother == 0;
     P->kc0 = chunk_levels(((v.Nx + 63) / 64) * ((v.Ny + RBC_BY - 1) / RBC_BY), v.Nz, RBC_KC, RBC_FILL, 3, 2);
     // the next level's sweeps likewise, with its φ and b colour-split, where
     // its coefficients, φ and b (40 B a cell) would stream from memory. A pass
@@ -2193,7 +2238,7 @@ void mg_set_terrain_coef(MGPlan *P, const TFWView &v) {
     P->gen1 = false;
     hipFree(P->tab1);
     P->tab1 = nullptr;
-    if (P->gen0 && P->nlev > 2 && (size_t)nx1 * ny1 * nz1 >= TFC_MIN) {
+    if (P->gen0 && rb_cycle(P) && P->nlev > 2 && (size_t)nx1 * ny1 * nz1 >= TFC_MIN) {
         P->kc1 = chunk_levels(((nx1 + 63) / 64) * ((ny1 + RBC_BY - 1) / RBC_BY), nz1, RBC_KC, RBC_FILL, 3, 2);
         const int nch = (nz1 + P->kc1 - 1) / P->kc1;
         const size_t n = (size_t)(nx1 + 1) * (ny1 + 1) * (TFC_Q + TFC_V * (size_t)nch);
