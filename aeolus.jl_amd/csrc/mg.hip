@@ -1185,13 +1185,13 @@ __global__ void cg_apply_kernel(LevelD<double> L, const double *__restrict__ p, 
     if (threadIdx.x == 0) partials[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = s;
 }
 
-// r −= αAp, block sums of (r², r)  (α from the device; null: 0); sm: r is
-// colour-split, Ap natural
+// r −= αAp, block sums of (r², r)  (α from the device); sm: r is colour-split,
+// Ap natural
 __global__ void cg_update_kernel(double *__restrict__ r, const double *__restrict__ Ap,
                                  const double *__restrict__ aptr, int n, double *__restrict__ partials, int nblk,
                                  SplitMap sm) {
     __shared__ double sh[RB / 64];
-    const double alpha = aptr ? aptr[0] : 0.0;
+    const double alpha = aptr[0];
     double s2 = 0.0, s1 = 0.0;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
         const uint32_t q = split_t(sm, t);
@@ -2123,10 +2123,8 @@ int mg_pcg_solve(MGPlan *P, hipStream_t st, double *xout, const double *bin, dou
     double mb = read_scal(st, P->scal + 9);
     hipLaunchKernelGGL(shift_copy_kernel, dim3(stream_blocks(n)), dim3(RB), 0, st, P->r, (const double *)b, n, mb);
     hipLaunchKernelGGL(fill_kernel, dim3(stream_blocks(n)), dim3(RB), 0, st, P->x, n, 0.0);
-    // b2 = Σ r²: the update kernel with α = 0
-    hipLaunchKernelGGL(cg_update_kernel, dim3(fb), dim3(RB), 0, st, P->r, (const double *)P->r, (const double *)nullptr, n,
-                       P->part, fb, SplitMap{0, 0, 0, -1, -1});
-    finalize_multi_to(P, st, P->scal + 12, P->part, fb, 2);
+    hipLaunchKernelGGL(dot_kernel, dim3(fb), dim3(RB), 0, st, (const double *)P->r, (const double *)P->r, n, P->part);
+    finalize_to(P, st, P->scal + 12, P->part, fb, 1.0);
     double b2 = read_scal(st, P->scal + 12);
     double bnorm = sqrt(b2);
     *bnorm_out = bnorm;
