@@ -1095,7 +1095,7 @@ struct aeo_tf_stepper {
     double *us = nullptr, *vs = nullptr, *ws = nullptr, *tn = nullptr;  // predictor and θ' (storage)
     double *snap[4] = {};                                                 // the RK3 step-start state
     double *bx = nullptr, *by = nullptr, *rs = nullptr;                   // the operator's face arrays
-    double *gx = nullptr, *gy = nullptr, *gw = nullptr;                   // G φ work (interior-sized)
+    double *work = nullptr;                                               // of the residual checks (interior-sized)
     double *b = nullptr, *phi = nullptr;                                  // source and potential (interior-sized)
     MGPlan *mg = nullptr;
     bool have_phi = false;  // phi holds a previous solve's result (the warm start)
@@ -1166,7 +1166,7 @@ extern "C" int aeo_tf_stepper_create(aeo_terrain *t, const aeo_tf_params *p, aeo
         HIPCHK(hipMalloc(q, sizeof(double) * h->n));
         HIPCHK(zero_dev(*q, sizeof(double) * h->n));
     }
-    for (double **q : {&h->bx, &h->by, &h->gx, &h->gy, &h->gw, &h->b, &h->phi}) {
+    for (double **q : {&h->bx, &h->by, &h->work, &h->b, &h->phi}) {
         HIPCHK(hipMalloc(q, sizeof(double) * h->ni));
         HIPCHK(zero_dev(*q, sizeof(double) * h->ni));
     }
@@ -1201,7 +1201,7 @@ extern "C" int aeo_tf_stepper_create(aeo_terrain *t, const aeo_tf_params *p, aeo
 extern "C" int aeo_tf_stepper_destroy(aeo_tf_stepper *h) {
     if (!h) return AEO_OK;
     if (g_ctx) hipStreamSynchronize(g_ctx->stream);
-    for (double *q : {h->us, h->vs, h->ws, h->tn, h->bx, h->by, h->rs, h->gx, h->gy, h->gw, h->b, h->phi})
+    for (double *q : {h->us, h->vs, h->ws, h->tn, h->bx, h->by, h->rs, h->work, h->b, h->phi})
         if (q) hipFree(q);
     for (double *q : h->snap)
         if (q) hipFree(q);
@@ -1550,8 +1550,8 @@ static int tfw_true_residual(aeo_tf_stepper *h, double *out) {
     double mb = 0;
     for (int q = 0; q < NB; q++) mb += hp[q];
     mb /= (double)h->ni;
-    tfw_apply_cb(h, st, h->gw, h->phi);
-    hipLaunchKernelGGL(tfw_resid_kernel, dim3(NB), dim3(256), 0, st, d, h->last_b, (const double *)h->gw, mb, h->ni);
+    tfw_apply_cb(h, st, h->work, h->phi);
+    hipLaunchKernelGGL(tfw_resid_kernel, dim3(NB), dim3(256), 0, st, d, h->last_b, (const double *)h->work, mb, h->ni);
     HIPCHK(hipMemcpyAsync(hp.data(), d, sizeof(double) * 2 * NB, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     double bb = 0, rr = 0;
@@ -1597,8 +1597,8 @@ extern "C" int aeo_tf_constraint_residual(aeo_tf_stepper *h, double *u, double *
     constexpr int NB = 512;
     double *d = red_scratch(NB);
     if (!d) return fail(AEO_ERR_HIP, "reduction scratch: out of device memory");
-    launch_tfw_div(st, h->v, h->bx, h->by, h->rs, h->gx, u, v, w);
-    launch_tfw_absdiv(st, h->v, d, NB, h->gx);
+    launch_tfw_div(st, h->v, h->bx, h->by, h->rs, h->work, u, v, w);
+    launch_tfw_absdiv(st, h->v, d, NB, h->work);
     double hb[NB];
     HIPCHK(hipMemcpyAsync(hb, d, sizeof hb, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));

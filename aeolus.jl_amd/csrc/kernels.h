@@ -171,10 +171,8 @@ struct TFM {
     __device__ __forceinline__ TC J(int i, int j) const { return (Hl - hp(i, j)) * iHl; }
     __device__ __forceinline__ TC hxf(int i, int j) const { return (hp(i, j) + hp(i > 0 ? i - 1 : 0, j)) / TC(2); }
     __device__ __forceinline__ TC hyf(int i, int j) const { return (hp(i, j) + hp(i, j > 0 ? j - 1 : 0)) / TC(2); }
-    __device__ __forceinline__ TC hxy(int i, int j) const { return (hxf(i, j) + hxf(i, j > 0 ? j - 1 : 0)) / TC(2); }
     __device__ __forceinline__ TC Jx(int i, int j) const { return (Hl - hxf(i, j)) * iHl; }
     __device__ __forceinline__ TC Jy(int i, int j) const { return (Hl - hyf(i, j)) * iHl; }
-    __device__ __forceinline__ TC Jxy(int i, int j) const { return (Hl - hxy(i, j)) * iHl; }
     // J·σ_x and J·σ_y at the σ-face k: −(H − σ_f) h_x/H (the (H − h) of σ_x cancels J's)
     __device__ __forceinline__ TC jsx(int i, int j, int k) const { return (sigf(k) - Hl) * iHl * (TC)hx[i + sx * j]; }
     __device__ __forceinline__ TC jsy(int i, int j, int k) const { return (sigf(k) - Hl) * iHl * (TC)hy[i + sx * j]; }
@@ -192,9 +190,6 @@ struct TFM {
     __device__ __forceinline__ TC rho_xf(int i, int j, int k) const { return rho(hxf(i, j) + sigc(k) * Jx(i, j)); }
     __device__ __forceinline__ TC rho_yf(int i, int j, int k) const { return rho(hyf(i, j) + sigc(k) * Jy(i, j)); }
     __device__ __forceinline__ TC rho_sf(int i, int j, int k) const { return rho(hp(i, j) + sigf(k) * J(i, j)); }
-    __device__ __forceinline__ TC rho_xy(int i, int j, int k) const { return rho(hxy(i, j) + sigc(k) * Jxy(i, j)); }
-    __device__ __forceinline__ TC rho_xs(int i, int j, int k) const { return rho(hxf(i, j) + sigf(k) * Jx(i, j)); }
-    __device__ __forceinline__ TC rho_ys(int i, int j, int k) const { return rho(hyf(i, j) + sigf(k) * Jy(i, j)); }
 };
 
 template <typename TC>

@@ -1212,28 +1212,24 @@ __global__ void load_rhs_kernel(T *__restrict__ b, const double *__restrict__ r,
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) b[t] = (T)(r[t] - m);
 }
 
-// z = φ − mean φ (_store_solution!, :789-793), then the block sums of (r·z, z,
-// r) and, with ap (the last A p), of z·Ap for the flexible β
+// z = φ − mean φ (_store_solution!, :789-793), stored when z is given, and the
+// block sums of (r·z, z, r)
 template <typename T>
 __global__ void store_rz_kernel(double *__restrict__ z, const T *__restrict__ phi, const double *__restrict__ r, int n,
-                                const double *__restrict__ mptr, double *__restrict__ partials, int nblk,
-                                const double *__restrict__ ap) {
+                                const double *__restrict__ mptr, double *__restrict__ partials, int nblk) {
     __shared__ double sh[RB / 64];
     const double m = mptr ? mptr[0] : 0.0;
-    double srz = 0.0, sz = 0.0, sr = 0.0, szap = 0.0;
+    double srz = 0.0, sz = 0.0, sr = 0.0;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
         const double zv = (double)phi[t] - m;
         if (z) z[t] = zv;
         srz += r[t] * zv;
         sz += zv;
         sr += r[t];
-        if (ap) szap += zv * ap[t];
     }
     double a = block_sum(srz, sh), b = block_sum(sz, sh), c = block_sum(sr, sh);
-    double d = ap ? block_sum(szap, sh) : 0.0;
     if (threadIdx.x == 0) {
         partials[blockIdx.x] = a; partials[nblk + blockIdx.x] = b; partials[2 * nblk + blockIdx.x] = c;
-        partials[3 * nblk + blockIdx.x] = d;
     }
 }
 
@@ -1415,7 +1411,7 @@ struct MGPlan {
     double *cx64 = nullptr, *cy64 = nullptr, *cz64 = nullptr;
     double *rhs_scale = nullptr;
     // CG arrays and reduction scratch
-    double *x = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *Ap = nullptr;
+    double *x = nullptr, *r = nullptr, *p = nullptr, *Ap = nullptr;
     double *part = nullptr, *scal = nullptr;  // scal: device scalars
     double *part2 = nullptr;                  // the block sums of a long partial list (≤ 2048)
     int npart = 0;
@@ -1891,7 +1887,7 @@ MGPlan *mg_create(int nx, int ny, int nz, double dx, double dy, double dz, int b
         ddx *= 2; ddy *= 2; ddz *= 2;
     }
     size_t n0 = (size_t)nx * ny * nz;
-    double **cg[5] = {&P->x, &P->r, &P->z, &P->p, &P->Ap};
+    double **cg[4] = {&P->x, &P->r, &P->p, &P->Ap};
     for (auto a : cg) {
         if (hipMalloc(a, 8 * n0) != hipSuccess) return fail("mg: allocation failed");
         zero_dev(*a, 8 * n0);
@@ -1922,7 +1918,7 @@ void mg_destroy(MGPlan *P) {
         hipFree(h.phi); hipFree(h.b); hipFree(h.r); hipFree(h.tmp); hipFree(h.cx); hipFree(h.cy); hipFree(h.cz);
     }
     hipFree(P->cx64); hipFree(P->cy64); hipFree(P->cz64); hipFree(P->rhs_scale);
-    hipFree(P->x); hipFree(P->r); hipFree(P->z); hipFree(P->p); hipFree(P->Ap);
+    hipFree(P->x); hipFree(P->r); hipFree(P->p); hipFree(P->Ap);
     hipFree(P->part); hipFree(P->part2); hipFree(P->scal); hipFree(P->tab1);
     delete P;
 }
@@ -1930,24 +1926,19 @@ void mg_destroy(MGPlan *P) {
 int mg_levels(const MGPlan *P) { return P->nlev; }
 
 // z = M⁻¹ r: one V-cycle from zero, the reference's _mg_precond! (src/Multigrid.jl:922-932);
-// returns with the block sums of (r·z, z, r) finalised into scal[0..2] and,
-// with ap, z·Ap into scal[3]. r is P->r and z P->z unless given (not
-// aliased). The FP32 V-cycle neither removes r's mean (r is mean-free in a
+// returns with the block sums of (r·z, z, r) finalised into scal[0..2]. z is
+// stored when given (not aliased with r); the CG forms it again from φ with
+// cg_dir_phi_kernel. The FP32 V-cycle neither removes r's mean (r is mean-free in a
 // consistent CG to its rounding) nor z's: the CG subtracts Σz/n when it
 // forms the direction (the sums above carry what it needs). A red-black
 // cycle on an open operator leaves z's mean in likewise.
-// store_z false: z is not written (the caller forms it again from φ with
-// cg_dir_phi_kernel)
 // rsum_in_part: P->part[fb .. 2fb) holds the block sums of r in sum_kernel's
 // layout (cg_update_kernel's second component), so r's mean needs no pass
 template <typename T>
-static void precond(MGPlan *P, hipStream_t st, const double *ap = nullptr, const double *rin = nullptr,
-                    double *zout = nullptr, bool store_z = true, bool rsum_in_part = false) {
+static void precond(MGPlan *P, hipStream_t st, const double *r, double *z = nullptr, bool rsum_in_part = false) {
     MGLevelH &h = P->L[0];
     const int n = h.nx * h.ny * h.nz;
     const int fb = flat_blocks(n);
-    const double *r = rin ? rin : P->r;
-    double *z = zout ? zout : P->z;
     const bool lean = P->prec != 0;
     const bool rb = rb_cycle(P) && P->nlev > 1;
     // the mean of r, then b = r − m
@@ -1963,9 +1954,8 @@ static void precond(MGPlan *P, hipStream_t st, const double *ap = nullptr, const
         mean_to<T>(P, st, (const T *)h.phi, n, 8);
         m2 = P->scal + 8;
     }
-    hipLaunchKernelGGL(store_rz_kernel<T>, dim3(fb), dim3(RB), 0, st, store_z ? z : (double *)nullptr, (const T *)h.phi, r, n,
-                       m2, P->part, fb, ap);
-    finalize_multi_to(P, st, P->scal, P->part, fb, ap ? 4 : 3);
+    hipLaunchKernelGGL(store_rz_kernel<T>, dim3(fb), dim3(RB), 0, st, z, (const T *)h.phi, r, n, m2, P->part, fb);
+    finalize_multi_to(P, st, P->scal, P->part, fb, 3);
 }
 
 // the FP64 terrain cycle inside the CG: r in place as the finest right-hand
@@ -1978,7 +1968,7 @@ static void precond_split(MGPlan *P, hipStream_t st) {
         const int n = h.nx * h.ny * h.nz;
         nb = flat_blocks(n);
         hipLaunchKernelGGL(store_rz_kernel<double>, dim3(nb), dim3(RB), 0, st, (double *)nullptr, (const double *)h.phi,
-                           (const double *)h.b, n, (const double *)nullptr, P->part, nb, (const double *)nullptr);
+                           (const double *)h.b, n, (const double *)nullptr, P->part, nb);
     }
     finalize_multi_to(P, st, P->scal, P->part, nb, 3);
 }
@@ -2040,7 +2030,7 @@ static int pcg_run(MGPlan *P, hipStream_t st, const FCGOp *op, double tol, doubl
         } else if (split) {
             precond_split(P, st);
         } else {
-            precond<double>(P, st, nullptr, nullptr, nullptr, false);
+            precond<double>(P, st, P->r);
         }
         hipLaunchKernelGGL(cg_init_scalars_kernel, dim3(1), dim3(1), 0, st, P->scal, dn);
         if (fused)
@@ -2091,7 +2081,7 @@ static int pcg_run(MGPlan *P, hipStream_t st, const FCGOp *op, double tol, doubl
         }
         if (fused) precond_fused<float>(P, st, P->Ap);
         else if (split) precond_split(P, st);
-        else precond<double>(P, st, nullptr, nullptr, nullptr, false, true);
+        else precond<double>(P, st, P->r, nullptr, true);
         hipLaunchKernelGGL(cg_beta_kernel, dim3(1), dim3(1), 0, st, P->scal, dn, (int)fused);
         if (fused)
             hipLaunchKernelGGL(cg_dir_x_kernel<float>, dim3(sb), dim3(RB), 0, st, P->x, P->p, (const float *)h.phi, n,
@@ -2112,8 +2102,6 @@ int mg_pcg_solve(MGPlan *P, hipStream_t st, double *xout, const double *bin, dou
     MGLevelH &h = P->L[0];
     const int n = h.nx * h.ny * h.nz;
     const int fb = flat_blocks(n);
-    const double dn = (double)n;
-    LevelD<double> F = finelevel64(P);
     double *b = P->Ap;  // the scaled source lives in Ap until the first apply
     hipMemcpyAsync(b, bin, sizeof(double) * n, hipMemcpyDeviceToDevice, st);
     if (P->rhs_scale)
@@ -2158,7 +2146,6 @@ int mg_pcg_solve_op(MGPlan *P, hipStream_t st, const FCGOp &op, double *xout, co
     MGLevelH &h = P->L[0];
     const int n = h.nx * h.ny * h.nz;
     const int fb = flat_blocks(n);
-    const double dn = (double)n;
     double *b = P->Ap;  // the source's copy lives in Ap until the first apply
     hipMemcpyAsync(b, bin, sizeof(double) * n, hipMemcpyDeviceToDevice, st);
     mean_to<double>(P, st, b, n, 9);
@@ -2344,7 +2331,7 @@ void mg_precond_apply(MGPlan *P, hipStream_t st, double *z, const double *r) {
         hipMemcpyAsync(P->r, r, sizeof(double) * n, hipMemcpyDeviceToDevice, st);
         r = P->r;
     }
-    if (P->prec == 0) precond<double>(P, st, nullptr, r, z); else precond<float>(P, st, nullptr, r, z);
+    if (P->prec == 0) precond<double>(P, st, r, z); else precond<float>(P, st, r, z);
     if (P->prec != 0 || (rb_cycle(P) && P->nlev > 1)) {  // the cycle leaves z's mean in: remove it here
         mean_to<double>(P, st, z, n, 8);
         hipLaunchKernelGGL(shift_kernel<double>, dim3(stream_blocks(n)), dim3(RB), 0, st, z, n, P->scal + 8);
