@@ -168,6 +168,7 @@ SIGNATURES = {
     "aeo_profile_enable": [_i],
     "aeo_profile_reset": [],
     "aeo_profile_get": [ctypes.c_char_p, _pi, _pd],
+    "aeo_launch_levels": [ctypes.c_char_p, _i, _i, _i, _pi],
 }
 
 _lib = None

@@ -2565,6 +2565,21 @@ extern "C" int aeo_kinetic_energy(aeo_grid *g, int precision, const void *u, con
     return rc;
 }
 
+extern "C" int aeo_launch_levels(const char *kernel, int Nx, int Ny, int Nz, int *levels) {
+    if (!kernel || !levels) return fail(AEO_ERR_ARG, "null argument");
+    if (Nx < 1 || Ny < 1 || Nz < 1) return fail(AEO_ERR_ARG, "bad extents %d x %d x %d", Nx, Ny, Nz);
+    static const struct { const char *name; int (*rule)(int, int, int); } rules[] = {
+        {"tendency", chunk_tile}, {"scalar", chunk_brick}, {"limited", chunk_limited},
+        {"terrain_tendency", chunk_tfw_tendency}, {"terrain_apply", chunk_tfw_apply},
+        {"terrain_smooth", chunk_tf_smooth}, {"terrain_prolong", chunk_tf_prolong}};
+    for (const auto &r : rules)
+        if (!strcmp(kernel, r.name)) {
+            *levels = r.rule(Nx, Ny, Nz);
+            return AEO_OK;
+        }
+    return fail(AEO_ERR_ARG, "no marching kernel named %s", kernel);
+}
+
 extern "C" int aeo_profile_enable(int on) {
     NEED_CTX();
     g_ctx->profile = on != 0;

@@ -262,6 +262,15 @@ template <typename T>
 int spectral_column_solve_wdiv(SpectralPlan *p, hipStream_t st, double *phi, const T *u, const T *v, const T *w,
                                const double *Wc, const double *Wf, const Metrics<double> &md);
 
+// the levels per block of the marching kernels on a grid of nx × ny × nz cells (chunk_levels; aeo_launch_levels)
+int chunk_tile(int nx, int ny, int nz);
+int chunk_brick(int nx, int ny, int nz);
+int chunk_limited(int nx, int ny, int nz);
+int chunk_tfw_tendency(int nx, int ny, int nz);
+int chunk_tfw_apply(int nx, int ny, int nz);
+int chunk_tf_smooth(int nx, int ny, int nz);
+int chunk_tf_prolong(int nx, int ny, int nz);
+
 // A profile scope on the library stream (api.hip): with profiling on and a
 // name, events bracket the launches made inside the scope and their time is
 // booked under the name (aeo_profile_get)

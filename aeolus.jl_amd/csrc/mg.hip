@@ -1613,9 +1613,13 @@ static bool coarse_fold(const MGPlan *P, int l) {
     return sizeof(T) == 8 && P->prec == 0 && !rb_cycle(P) && !P->wcycle && P->smoother == 0 && l >= 1 && 33 + 2 * l < MG_NSCAL;
 }
 
-static int prolong_chunk(const MGLevelH &h) {
-    return chunk_levels(((h.nx + 63) / 64) * ((h.ny + PRC_BY - 1) / PRC_BY), h.nz, PRC_KC, PRC_FILL, 2, 2);
+int chunk_tf_prolong(int nx, int ny, int nz) {
+    return chunk_levels(((nx + 63) / 64) * ((ny + PRC_BY - 1) / PRC_BY), nz, PRC_KC, PRC_FILL, 2, 2);
 }
+int chunk_tf_smooth(int nx, int ny, int nz) {
+    return chunk_levels(((nx + 63) / 64) * ((ny + RBC_BY - 1) / RBC_BY), nz, RBC_KC, RBC_FILL, 3, 2);
+}
+static int prolong_chunk(const MGLevelH &h) { return chunk_tf_prolong(h.nx, h.ny, h.nz); }
 
 // φ of level l += the prolongation of the coarse φ, with the block sums of
 // the result in P->part; returns their count. pre_m, mc: pending means of the
@@ -2212,7 +2216,7 @@ void mg_set_terrain_coef(MGPlan *P, const TFWView &v) {
     // ρ̄ > 0 and J > 0 on every face, so every diagonal is negative
     P->open = P->open || dims;
     P->gen0 = dims && P->prec == 0 && P->smoother == 0;
-    P->kc0 = chunk_levels(((v.Nx + 63) / 64) * ((v.Ny + RBC_BY - 1) / RBC_BY), v.Nz, RBC_KC, RBC_FILL, 3, 2);
+    P->kc0 = chunk_tf_smooth(v.Nx, v.Ny, v.Nz);
     // the next level's sweeps likewise, with its φ and b colour-split, where
     // its coefficients, φ and b (40 B a cell) would stream from memory. A pass
     // at 256×256×128 (336 MB, past the 256 MB of the Infinity Cache): 86 us with
@@ -2224,7 +2228,7 @@ void mg_set_terrain_coef(MGPlan *P, const TFWView &v) {
     hipFree(P->tab1);
     P->tab1 = nullptr;
     if (P->gen0 && rb_cycle(P) && P->nlev > 2 && (size_t)nx1 * ny1 * nz1 >= TFC_MIN) {
-        P->kc1 = chunk_levels(((nx1 + 63) / 64) * ((ny1 + RBC_BY - 1) / RBC_BY), nz1, RBC_KC, RBC_FILL, 3, 2);
+        P->kc1 = chunk_tf_smooth(nx1, ny1, nz1);
         const int nch = (nz1 + P->kc1 - 1) / P->kc1;
         const size_t n = (size_t)(nx1 + 1) * (ny1 + 1) * (TFC_Q + TFC_V * (size_t)nch);
         if (hipMalloc(&P->tab1, sizeof(double) * n) == hipSuccess) {

@@ -243,12 +243,16 @@ __global__ void __launch_bounds__(PW *PBY) pos_tile_kernel(T *__restrict__ out, 
     }
 }
 
+// two blocks per CU a round: 33×29×25 FP64 86 → 14 us, 100×80×60 FP32
+// WENO-Z7 83 → 34 us, 256×256×128 as before (16 levels)
+int chunk_limited(int nx, int ny, int nz) {
+    return chunk_levels(((nx + PW - 1) / PW) * ((ny + PBY - 1) / PBY), nz, PKC, 512, 1);
+}
+
 template <int S, int P, typename T>
 static void launch_pos_tile(hipStream_t st, T *tend, T *Rd, const T *u, const T *v, const T *w, const T *phi, T dt,
                             const Metrics<T> &m, const int *bcs, int accumulate) {
-    // two blocks per CU a round: 33×29×25 FP64 86 → 14 us, 100×80×60 FP32
-    // WENO-Z7 83 → 34 us, 256×256×128 as before (16 levels)
-    const int kc = chunk_levels(((m.Nx + PW - 1) / PW) * ((m.Ny + PBY - 1) / PBY), m.Nz, PKC, 512, 1);
+    const int kc = chunk_limited(m.Nx, m.Ny, m.Nz);
     const dim3 blk(PW, PBY), grd((m.Nx + PW - 1) / PW, (m.Ny + PBY - 1) / PBY, (m.Nz + kc - 1) / kc);
     hipLaunchKernelGGL((pos_tile_kernel<POS_RATIO, S, P, T>), grd, blk, 0, st, Rd, u, v, w, phi, (const T *)nullptr,
                        dt, m, 0, kc);

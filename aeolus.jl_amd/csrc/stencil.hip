@@ -773,13 +773,25 @@ __global__ void __launch_bounds__(MW *BY, TILE_MINW) adv_tile_kernel(MarchArgs<T
     }
 }
 
+constexpr int MBY = 8;  // rows per block of the tile and brick kernels
+int chunk_tile(int nx, int ny, int nz) {
+    return chunk_levels(((nx + MW - 1) / MW) * ((ny + MBY - 1) / MBY), nz, TILE_KC, TILE_FILL, 1);
+}
+// the brick kernel holds several blocks per CU: shorter chunks pay only
+// where KCM leaves CUs without a block (33×29×25 FP64 20.6 → 5.5 us,
+// 130×70×60 WENO-Z7 35.6 → 31.9; 187×141×75 FP32 31.9, 33.3 if shortened)
+int chunk_brick(int nx, int ny, int nz) {
+    const int tiles = ((nx + MW - 1) / MW) * ((ny + MBY - 1) / MBY), kmax = nz < KCM ? nz : KCM;
+    return tiles * ((nz + kmax - 1) / kmax) >= 256 ? kmax : chunk_levels(tiles, nz, kmax, 256, 3);
+}
+
 template <int MODE, int S, int P, typename T>
 static void launch_march_sp(hipStream_t st, const MarchArgs<T> &a) {
-    constexpr int BY = 8;
+    constexpr int BY = MBY;
     const Metrics<T> &m = a.m;
     if constexpr (MODE != MODE_SCALAR) {
         MarchArgs<T> t = a;
-        t.kc = chunk_levels(((m.Nx + MW - 1) / MW) * ((m.Ny + BY - 1) / BY), m.Nz, TILE_KC, TILE_FILL, 1);
+        t.kc = chunk_tile(m.Nx, m.Ny, m.Nz);
         dim3 grid((m.Nx + MW - 1) / MW, (m.Ny + BY - 1) / BY, (m.Nz + t.kc - 1) / t.kc);
         if (m.stretched)
             hipLaunchKernelGGL((adv_tile_kernel<MODE, S, P, T, BY, 1>), grid, dim3(MW, BY), 0, st, t);
@@ -858,11 +870,7 @@ int launch_advect(hipStream_t st, const Metrics<T> &m, int mode, int scheme, int
     a.m = m;
     a.in = Fields<T>{u, v, w, s};
     a.tu = tu; a.tv = tv; a.tw = tw; a.ts = ts;
-    // the brick kernel holds several blocks per CU: shorter chunks pay only
-    // where KCM leaves CUs without a block (33×29×25 FP64 20.6 → 5.5 us,
-    // 130×70×60 WENO-Z7 35.6 → 31.9; 187×141×75 FP32 31.9, 33.3 if shortened)
-    const int tiles = ((m.Nx + MW - 1) / MW) * ((m.Ny + 7) / 8), kmax = m.Nz < KCM ? m.Nz : KCM;
-    a.kc = tiles * ((m.Nz + kmax - 1) / kmax) >= 256 ? kmax : chunk_levels(tiles, m.Nz, kmax, 256, 3);
+    a.kc = chunk_brick(m.Nx, m.Ny, m.Nz);
     if (mode == MODE_SCALAR) return launch_march_mode<MODE_SCALAR, T>(st, a, scheme, p);
     return launch_march_mode<MODE_MOMENTUM, T>(st, a, scheme, p);
 }

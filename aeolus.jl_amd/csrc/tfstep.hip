@@ -857,13 +857,20 @@ static TFOp make_op(const TFWView &v, const double *bx, const double *by, const 
     return op;
 }
 
+int chunk_tfw_tendency(int nx, int ny, int nz) {
+    return chunk_levels(((nx + 63) / 64) * ((ny + TFT_BY - 1) / TFT_BY), nz, TFT_KC, TFT_FILL, 2);
+}
+int chunk_tfw_apply(int nx, int ny, int nz) {
+    return chunk_levels(((nx + 63) / 64) * ((ny + TFA_BY - 1) / TFA_BY), nz, TFA_KC, TFA_FILL, 4);
+}
+
 template <int S, typename TC>
 static void launch_tendency_tile(hipStream_t st, const TFWView &v, double *us, double *vs, double *ws, double *tn,
                                  const double *u, const double *vv, const double *w, const double *th,
                                  const double *th0, double dt, double ca, double cb, int combine, int raw) {
     constexpr int BY = TFT_BY;
     const int tx = (v.Nx + 63) / 64, ty = (v.Ny + BY - 1) / BY;
-    const int kc = chunk_levels(tx * ty, v.Nz, TFT_KC, TFT_FILL, 2);
+    const int kc = chunk_tfw_tendency(v.Nx, v.Ny, v.Nz);
     hipLaunchKernelGGL((tfw_tendency_tile_kernel<S, TC, BY>), dim3(tx, ty, (v.Nz + kc - 1) / kc), dim3(64, BY), 0, st,
                        us, vs, ws, tn, u, vv, w, th, th0, make_tfm<TC>(v), dt, ca, cb, combine, raw, kc);
 }
@@ -904,7 +911,7 @@ void launch_tfw_div(hipStream_t st, const TFWView &v, const double *bx, const do
 // blocks (cap); returns the block count, or −1 when no sums were written
 int launch_tfw_apply_march(hipStream_t st, const TFWView &v, double *out, const double *x, double *part, int cap) {
     const int tx = (v.Nx + 63) / 64, ty = (v.Ny + TFA_BY - 1) / TFA_BY;
-    const int kc = chunk_levels(tx * ty, v.Nz, TFA_KC, TFA_FILL, 4);
+    const int kc = chunk_tfw_apply(v.Nx, v.Ny, v.Nz);
     const dim3 grid(tx, ty, (v.Nz + kc - 1) / kc);
     const int nb = (int)(grid.x * grid.y * grid.z);
     if (part && nb > cap) part = nullptr;

@@ -524,6 +524,12 @@ int aeo_profile_reset(void);
  * "poisson", "shell" */
 int aeo_profile_get(const char *kernel, int *count, double *total_ms);
 
+/* The levels of a column that one block of a marching kernel works through on
+ * a grid of this size (no reference counterpart; computed on the host, no GPU
+ * needed): "tendency" (also momentum advection), "scalar", "limited",
+ * "terrain_tendency", "terrain_apply", "terrain_smooth", "terrain_prolong" */
+int aeo_launch_levels(const char *kernel, int Nx, int Ny, int Nz, int *levels);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,6 +1,7 @@
-"""The marching kernels at the chunk lengths their rule picks: one level per
-block on the smallest grids, then 2 to 15 as the grid grows, with a shorter
-last chunk, against the CPU oracle. The values of a face do not depend on the
+"""The marching kernels at the short chunks their rule picks on small grids: one
+level per block on the smallest, up to 6 in the tile and brick kernels and 3 in
+the limited one, with a shorter last chunk, against the CPU oracle (the longest
+chunks: test_gpu_long_chunks.py). The values of a face do not depend on the
 chunk it is computed in, so the tolerance is the parity tests' (FP64 roundings
 of a fused multiply-add, 1e-12 relative)."""
 import numpy as np

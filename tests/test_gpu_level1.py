@@ -6,8 +6,9 @@ One iteration of the CG, x = α z with z one V-cycle: its sums have up to n
 terms and the carried coefficients are within about 64 ulp of the stored ones,
 so 1e-10 of the largest value holds; a coefficient of the wrong face, or a
 value read from the wrong colour's half, shows at 1e-3. The levels below the
-second are the generic ones; 32 and 36 levels give one chunk and a chunk with
-a remainder, the widths whole and partial blocks.
+second are the generic ones; the second level's 16 and 18 levels are two chunks
+of 8, and 10 and 8 (32 in test_gpu_long_chunks.py), the widths whole and
+partial blocks.
 """
 import numpy as np
 import pytest

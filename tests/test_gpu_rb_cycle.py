@@ -6,8 +6,8 @@ The two are the same in exact arithmetic, so the CG's iterates after a fixed
 number of iterations agree to rounding: three iterations of a cycle whose
 sums have up to n terms, within 1e-10 of the largest value (a residual
 formed on the wrong cells, or a missing correction, shows at 1e-3). Sizes:
-pairs and rows past and short of the blocks, one and several chunks of
-levels, mirror boundaries on every axis.
+pairs and rows past and short of the blocks, chunks of 2 and 4 levels (32 in
+test_gpu_long_chunks.py), mirror boundaries on every axis.
 """
 import ctypes
 

@@ -2,11 +2,12 @@
 
 The kernel carries ρ, ρJ and 1/ρJ up a chunk by their ratio between levels:
 over at most 64 levels each is within 64 x 2 roundings (1.4e-14) of the value
-the oracle evaluates, and the terms of L φ are at most about ten times its
+the oracle evaluates (on these small grids the chunks have 1 to 7 levels; 43 and
+64 in test_gpu_long_chunks.py), and the terms of L φ are at most about ten times its
 largest value (steep hills, dz << dx), so 1e-12 holds; a coefficient of the
 wrong level or column is off by dz/Hs = 1e-3 or more. Sizes: columns and rows
-one past, one short of and well below the block's 64 x 4; levels in one chunk,
-in several with a remainder, and past the longest chunk.
+one past, one short of and well below the block's 64 x 4; chunks of one level
+and of several with a remainder.
 """
 import numpy as np
 import pytest

@@ -5,8 +5,8 @@ levels by their ratio (2 roundings a half level), against the largest
 tendency: 1e-12, as for the other sizes. FP32 fluxes: the bound stated for
 them elsewhere, 1e-4. A flux taken from the wrong cell shows at 0.1. Sizes:
 columns and rows one past, one short of and below the block's 64 x 4, a last
-block of one cell, and chunks with remainders and of every length down to one
-level.
+block of one cell, and chunks of 1, 2 and 17 levels with remainders (32 in
+test_gpu_long_chunks.py).
 """
 import numpy as np
 import pytest
