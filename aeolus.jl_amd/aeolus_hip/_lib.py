@@ -164,6 +164,7 @@ SIGNATURES = {
     "aeo_unet_forward": [_vp, _vp, _vp, _vp],
     "aeo_unet_gradients": [_vp, _vp, _vp, _vp, _vp, ctypes.POINTER(ctypes.c_float)],
     "aeo_unet_train_step": [_vp, _vp, _vp, _vp, ctypes.c_float, ctypes.POINTER(ctypes.c_float)],
+    "aeo_conv3_weight_gradient": [_i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _pi],
     "aeo_poisson_fcg_create": [_vp, _vp, _vp, _i, _i, _d, _i, _pvp],
     "aeo_profile_enable": [_i],
     "aeo_profile_reset": [],

@@ -1674,6 +1674,18 @@ extern "C" int aeo_unet_train_step(aeo_unet *h, const double *src, const double 
     if (unet_train_step(h->N, g_ctx->stream, src, mask, target, lr, loss)) return fail(AEO_ERR_HIP, "training step failed");
     return AEO_OK;
 }
+extern "C" int aeo_conv3_weight_gradient(int cin, int cout, int nx, int ny, int nz, const void *in, const void *dy,
+                                         float *dw, float *db, int *plan) {
+    NEED_CTX();
+    if (!in || !dy || !dw || !db) return fail(AEO_ERR_ARG, "null argument");
+    if (nx < 1 || ny < 1 || nz < 1 || cin < 1 || cout < 1 ||
+        (double)nx * ny * nz * (cin > cout ? cin : cout) >= 2147483648.0)
+        return fail(AEO_ERR_ARG, "bad extents %d x %d x %d", nx, ny, nz);
+    const int rc = conv3_wgrad(g_ctx->stream, cin, cout, nx, ny, nz, in, dy, dw, db, plan);
+    if (rc == -1) return fail(AEO_ERR_ARG, "no layer of %d input and %d output channels", cin, cout);
+    if (rc) return fail(AEO_ERR_HIP, "weight gradient failed");
+    return AEO_OK;
+}
 extern "C" int aeo_poisson_fcg_create(aeo_poisson *base, aeo_unet *net, const double *mask, int mode, int use_guess,
                                       double tol, int maxit, aeo_poisson **out) {
     NEED_CTX();

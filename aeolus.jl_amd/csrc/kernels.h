@@ -322,6 +322,10 @@ int unet_gradients(UNet *N, hipStream_t st, const double *src, const double *mas
                    float *grad_host, float *loss);
 int unet_train_step(UNet *N, hipStream_t st, const double *src, const double *mask, const double *target, float lr,
                     float *loss);
+// dW[tap][c][n] and db[n] of a 3³ convolution from BF16 channels-last in and dy (aeo_conv3_weight_gradient);
+// −1: no such layer shape
+int conv3_wgrad(hipStream_t st, int cin, int cout, int nx, int ny, int nz, const void *in, const void *dy, float *dw,
+                float *db, int *plan);
 struct FCGState;
 // an operator on interior-sized FP64 vectors: apply(ctx, stream, out, x)
 struct FCGOp {

@@ -767,8 +767,7 @@ struct UNet {
     float *y;           // head output (scaled space)
     double *scal;       // [0] 1/rms, [1] rms, [2] loss
     double *dpart;      // reduction partials (FP64)
-    float *fpart;       // weight-gradient partials (FP32)
-    size_t fpart_n;
+    float *fpart;       // weight-gradient partials (FP32, WGRAD_PART)
 };
 
 #define UCHK(x)                                  \
@@ -817,9 +816,11 @@ static int conv_run(hipStream_t st, int cin, int cout, const bf16 *in, const bf1
 
 // CS: the input channels of a block (with 16 or 32 the accumulators of a
 // wave's taps stay within 144 registers; 48 needs 84 with 16 outputs)
+// part: the partials' room; plan: takes the rows, tasks and blocks when given
+constexpr size_t WGRAD_PART = (size_t)768 * (27 * 1024 + 64);  // blocks × (taps × (channels · outputs) + outputs)
 template <int CIN, int COUT, int CS>
-static int wgrad_launch(hipStream_t st, UNet *N, const bf16 *in, const bf16 *dy, Vol g, float *grad, float *bias,
-                        int cin) {
+static int wgrad_launch(hipStream_t st, float *part, const bf16 *in, const bf16 *dy, Vol g, float *grad, float *bias,
+                        int cin, int *plan) {
     constexpr int NS = CIN / CS;
     const int ntx = (g.nx + 31) / 32;
     // rows per block: few (a row's start costs three rows of loads) until the
@@ -829,22 +830,37 @@ static int wgrad_launch(hipStream_t st, UNet *N, const bf16 *in, const bf16 *dy,
     const int nyc = (g.ny + yc - 1) / yc;
     long long nb = (long long)ntx * nyc * g.nz;
     if (nb > 768 / NS) nb = 768 / NS;
+    if (plan) {
+        plan[0] = yc;
+        plan[1] = ntx * nyc * g.nz;
+        plan[2] = (int)nb;
+    }
     const size_t wpart = (size_t)NS * nb * 27 * CS * COUT;
-    if (wpart + nb * COUT > N->fpart_n) return -1;
-    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, CS>), dim3((unsigned)nb, NS), dim3(256), 0, st, in, dy, N->fpart,
-                       N->fpart + wpart, g, ntx, nyc, yc);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblk((size_t)27 * cin * COUT + COUT, 16)), dim3(256), 0, st, N->fpart,
-                       N->fpart + wpart, grad, bias, (int)nb, CS, cin, COUT);
+    if (wpart + nb * COUT > WGRAD_PART) return -1;
+    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT, CS>), dim3((unsigned)nb, NS), dim3(256), 0, st, in, dy, part,
+                       part + wpart, g, ntx, nyc, yc);
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblk((size_t)27 * cin * COUT + COUT, 16)), dim3(256), 0, st, part,
+                       part + wpart, grad, bias, (int)nb, CS, cin, COUT);
     return 0;
 }
-static int wgrad_run(hipStream_t st, UNet *N, int cinp, int cin, int cout, const bf16 *in, const bf16 *dy, Vol g,
-                     float *grad, float *bias) {
+static int wgrad_run(hipStream_t st, float *part, int cinp, int cin, int cout, const bf16 *in, const bf16 *dy, Vol g,
+                     float *grad, float *bias, int *plan = nullptr) {
 #define CASE(a, b, cs) \
-    if (cinp == a && cout == b) return wgrad_launch<a, b, cs>(st, N, in, dy, g, grad, bias, cin);
+    if (cinp == a && cout == b) return wgrad_launch<a, b, cs>(st, part, in, dy, g, grad, bias, cin, plan);
     CASE(8, 16, 8) CASE(16, 16, 16) CASE(16, 32, 16) CASE(32, 32, 32) CASE(32, 64, 16) CASE(64, 64, 16)
     CASE(96, 32, 32) CASE(48, 16, 48)
 #undef CASE
     return -1;
+}
+
+int conv3_wgrad(hipStream_t st, int cin, int cout, int nx, int ny, int nz, const void *in, const void *dy, float *dw,
+                float *db, int *plan) {
+    float *part = nullptr;
+    if (hipMalloc(&part, WGRAD_PART * 4) != hipSuccess) return -2;
+    int rc = wgrad_run(st, part, cin, cin, cout, (const bf16 *)in, (const bf16 *)dy, Vol{nx, ny, nz}, dw, db, plan);
+    if (rc == 0 && (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess)) rc = -2;
+    hipFree(part);
+    return rc;
 }
 
 static int refresh_layouts(UNet *N, hipStream_t st) {
@@ -949,8 +965,7 @@ UNet *unet_create(int nx, int ny, int nz, int inc, uint64_t seed, char *err, siz
     A((void **)&N->scal, 8 * 8);
     const int nbh = nblk(n0);
     A((void **)&N->dpart, (size_t)(nbh > 4096 ? nbh : 4096) * 18 * 8);
-    N->fpart_n = (size_t)768 * (27 * 1024 + 64);  // blocks × (taps × (channels · outputs) + outputs), wgrad_launch's bounds
-    A((void **)&N->fpart, N->fpart_n * 4);
+    A((void **)&N->fpart, WGRAD_PART * 4);
     if (!ok) {
         snprintf(err, errlen, "hipMalloc failed for the U-Net buffers");
         unet_destroy(N);
@@ -1025,7 +1040,7 @@ int unet_backward(UNet *N, hipStream_t st, const double *target) {
     hipLaunchKernelGGL(head_reduce_kernel, dim3(18), dim3(256), 0, st, N->dpart, nbh, n0, N->scal, G + N->headoff);
     // layer 9 (16 → 16 at full resolution): g9 in g0b16
     auto layer_grads = [&](int l, const bf16 *in, const bf16 *g, Vol gv) {
-        rc |= wgrad_run(st, N, L[l].cinp, L[l].cin, L[l].cout, in, g, gv, G + L[l].woff, G + L[l].boff);
+        rc |= wgrad_run(st, N->fpart, L[l].cinp, L[l].cin, L[l].cout, in, g, gv, G + L[l].woff, G + L[l].boff);
     };
     layer_grads(9, N->a8, N->g0b16, N->g0);
     rc |= conv_run(st, 16, 16, N->g0b16, L[9].wt, nullptr, N->g1b16, 16, 0, N->g0, 0);

@@ -506,6 +506,15 @@ int aeo_unet_gradients(aeo_unet *h, const double *src, const double *mask, const
 /* one Adam step (β = 0.9, 0.999) on one sample; loss may be NULL */
 int aeo_unet_train_step(aeo_unet *h, const double *src, const double *mask, const double *target, float lr,
                         float *loss);
+/* The weight and bias gradients of one 3x3x3 convolution of that network, the
+ * kernels its training runs: in (nx*ny*nz x cin) and dy (x cout) are BF16,
+ * channels last, x fastest among the voxels, dw[tap][c][n] (tap = dx + 1 +
+ * 3 (dy + 1) + 9 (dz + 1)) and db[n] FP32, all on the device. (cin, cout) is one
+ * of the layers': (8, 16), (16, 16), (16, 32), (32, 32), (32, 64), (64, 64),
+ * (96, 32), (48, 16). plan, if given: the rows of a task, the tasks and the
+ * blocks that shared them out. */
+int aeo_conv3_weight_gradient(int cin, int cout, int nx, int ny, int nz, const void *in, const void *dy, float *dw,
+                              float *db, int *plan);
 /* Flexible CG (Notay 2000, one previous direction kept) on the operator of
  * an MG-preconditioned CG solver `base` (same grid as the network), with
  * the network as initial guess (use_guess) and preconditioner. mode 0: the

@@ -3,7 +3,9 @@ segments and row chunks can go wrong: axes of one voxel at the coarsest level,
 one past and one short of a segment, several segments, rows past one chunk,
 and one and two input channels. Against the CPU network oracle with BF16
 rounding at the same points, per layer, at the tolerance stated for the
-network's gradients (BF16 ties carried through ten layers: 5e-2 relative L2)."""
+network's gradients (BF16 ties carried through ten layers: 5e-2 relative L2).
+Blocks of several tasks, longer row chunks and the sums to FP32 rounding:
+test_gpu_weight_gradient.py."""
 import numpy as np
 import pytest
 
