@@ -544,7 +544,7 @@ __global__ void __launch_bounds__(64 * RBC_BY) rbgs_tf_kernel(LevelD<double> L, 
 // sums meet in a lane exchange.
 // With partials, the block sums of the coarse values (for their mean).
 // Bound: memory, φ and half of b read, 13 B per fine cell. At 512×512×256:
-// residual 470 us + restriction 111 us → 202 us.
+// residual 470 us + restriction 111 us → 210 us.
 constexpr int RRC_BW = 4;  // waves per block
 __global__ void __launch_bounds__(64 * RRC_BW) residual_restrict_tf_kernel(LevelD<double> L, LevelD<double> C,
                                                                            TFM<double> gm, int kc,
@@ -646,7 +646,8 @@ __global__ void __launch_bounds__(64 * RRC_BW) residual_restrict_tf_kernel(Level
 // column, and kept for three coarse levels.
 // both: no smoothing follows, and every cell is corrected.
 // Bound: memory, half of φ read and written, 9 B per fine cell. At
-// 512×512×256: 258 us (both colours, one column per thread) → 142 us.
+// 512×512×256: 258 us (both colours, one column per thread) → 155 us (142
+// before the coarse φ was colour-split).
 constexpr int PRC_BY = 4;   // rows per block
 constexpr int PRC_KC = 16;  // most fine levels per chunk (even)
 constexpr int PRC_FILL = 1024;  // blocks a round (chunk_levels)

@@ -72,9 +72,9 @@ __device__ __forceinline__ TC tf_face6(TC a0, TC a1, TC a2, TC a3, TC a4, TC a5,
 // What bounds it is the FP64 VALU: about 13 WENO faces a cell, where a thread
 // per column that evaluates both faces of each direction has 20 and 15
 // density families, and at one wave per SIMD (over 256 registers) issued
-// half the time. At 512×512×256 7.95 → 3.70 ms, 320×256×160 with FP32
+// half the time. At 512×512×256 7.95 → 3.58 ms, 320×256×160 with FP32
 // fluxes 1.37 → 0.70, 96×96×48 250 → 49 us (chunks of 32 levels on every grid
-// before). Two waves per SIMD (225 registers): three for the FP32 form spill
+// before). Two waves per SIMD (227 registers): three for the FP32 form spill
 // (0.80 ms); blocks of 8 rows, one per CU: 3.79, 0.67 ms, 46 us.
 #pragma clang fp contract(fast)
 constexpr int TFT_BY = 4;
