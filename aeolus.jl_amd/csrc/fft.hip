@@ -539,8 +539,9 @@ __global__ void __launch_bounds__(64) thomas_kernel(double2 *__restrict__ hat, d
 // x_{2n+1} and V = DFT_N(v), X_k = 2 Re(e^{-iπk/(2N)} V_k) (Makhoul, IEEE
 // TASSP 28 (1980) 27). REDFT01: x_n = X_0 + 2 Σ_{k≥1} X_k cos(πk(2n+1)/(2N));
 // with W_k = (X_k − i X_{N−k}) e^{iπk/(2N)} (X_N = 0), v = N·IDFT_N(W) and
-// x_{2n} = v_n, x_{2n+1} = v_{N-1-n}. REDFT01 ∘ REDFT10 = 2N.
-__device__ __forceinline__ int dct_pos(int m, int N) { return m < N / 2 ? 2 * m : 2 * (N - 1 - m) + 1; }
+// x_{2n} = v_n, x_{2n+1} = v_{N-1-n}. REDFT01 ∘ REDFT10 = 2N. The even places
+// are ⌈N/2⌉ (an odd N has its last one in the middle of v).
+__device__ __forceinline__ int dct_pos(int m, int N) { return m < (N + 1) / 2 ? 2 * m : 2 * (N - 1 - m) + 1; }
 
 // rows along x of N reals: forward src → hat (X_k, 0), k < N; inverse Re(hat) → dst · scale
 __global__ void dct_rows_kernel(double2 *__restrict__ hat, const double *__restrict__ src, double *__restrict__ dst,
