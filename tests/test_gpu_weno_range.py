@@ -84,3 +84,25 @@ def test_limited(hip, orc, e, scheme):
     hip.advect_positive(g, t, *[up(a) for a in vel], up(f), 0.01, scheme=scheme, accumulate=False)
     I = og.interior
     assert np.isfinite(ref[I]).all() and rel_err(t.download()[I], ref[I]) < 1e-12
+
+
+@pytest.mark.parametrize("scheme", ["weno_z5", "weno_z7"])
+@pytest.mark.parametrize("e,half", [(0, False), (166, False), (330, False), (480, False), (120, True), (240, True),
+                                    (440, True)])
+def test_exponent_one(hip, orc, e, half, scheme):
+    """p = 1, whose weights take the ratios themselves: small beside large up to 2^440."""
+    n, H = (70, 21, 13), 4
+    g, og = hip.Grid(n, (3.0, 1.0, 2.0), halo=H), orc.Grid(n, (3.0, 1.0, 2.0), halo=H)
+    rng = np.random.default_rng(5)
+    f = [np.asfortranarray(rng.standard_normal(og.storage)) for _ in range(4)]
+    f[3][og.storage[0] // 2 if half else 0:] *= 2.0**e
+    for a, loc in zip(f, (orc.FX, orc.FY, orc.FZ, orc.CC)):
+        orc.fill_halos(og, a, loc, ("periodic",) * 3)
+    ref = orc.advect_scalar(og, og.zeros(), *f, scheme, p=1)[og.interior]
+    t = g.field()
+    hip.advection_scheme(scheme, g, p=1)(t, *[hip.DeviceArray.from_numpy(a) for a in f])
+    got = t.download()[og.interior]
+    assert np.isfinite(ref).all() and rel_err(got, ref) < 1e-12
+    if half:
+        m = n[0] // 2
+        assert rel_err(got[5:m - 5], ref[5:m - 5]) < 1e-12
